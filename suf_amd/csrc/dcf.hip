@@ -13,7 +13,7 @@
 // only on bit 0 of the terms, and bit 0 of -v equals bit 0 of v, so this
 // holds for both output groups.
 //
-// One element per lane; each lane streams its own key front to back
+// Batches of more than 256 keys per CU: one element per lane; each lane streams its own key front to back
 // (33 bytes per level), so successive levels hit the same cache lines.
 //
 // The evaluation kernels run 1024 lanes per CU (four waves per SIMD): their
@@ -26,6 +26,7 @@
 #include <cstring>
 
 #include "dcf_device.hpp"
+#include "dcf_quad_device.hpp"
 
 namespace sufhip {
 namespace {
@@ -46,13 +47,26 @@ struct DcfEvalArgs {
 
 constexpr int kDcfBitBlock = 1024;
 
+// First element of this wave in the pass that starts at `pass`.  A full pass
+// gives each workgroup 1024 neighbouring keys; the last one deals its
+// elements out 64 at a time, so that what does not fill the chip spreads over
+// every CU (50021 keys of 32 levels: 182 -> 90 us) instead of filling the
+// first ones.  Dealing the full passes out too made 2^20 keys 4% slower (the
+// keys in flight on a CU then span the whole 2 GB).
+__device__ __forceinline__ size_t wave_base(size_t pass, size_t n) {
+  const size_t wave = threadIdx.x >> 6;
+  return n - pass >= size_t(gridDim.x) * kDcfBitBlock
+             ? pass + size_t(blockIdx.x) * kDcfBitBlock + wave * 64
+             : pass + (size_t(blockIdx.x) + size_t(gridDim.x) * wave) * 64;
+}
+
 template <int kMode>
 __global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_bit_kernel(DcfEvalArgs a) {
   SUFHIP_DCF_TABLE_SETUP();
   const KeySelPtr keys = kernarg_key_sel(offsetof(DcfEvalArgs, key_sel));
   const size_t stride = size_t(gridDim.x) * kDcfBitBlock;
-  for (size_t base = size_t(blockIdx.x) * kDcfBitBlock; base < a.n; base += stride) {
-    const size_t e = base + threadIdx.x;
+  for (size_t pass = 0; pass < a.n; pass += stride) {
+    const size_t e = wave_base(pass, a.n) + (threadIdx.x & 63);
     uint32_t bit = 0;
     if (e < a.n) {
       const uint8_t* key = a.broadcast ? a.keys : a.keys + e * a.key_bytes;
@@ -77,7 +91,9 @@ __global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_bytes_kernel(DcfEvalArg
   const KeySelPtr keys = kernarg_key_sel(offsetof(DcfEvalArgs, key_sel));
   const size_t stride = size_t(gridDim.x) * kDcfBitBlock;
   const size_t chunk_bytes = 32 + 33 * size_t(a.in_bits);
-  for (size_t e = size_t(blockIdx.x) * kDcfBitBlock + threadIdx.x; e < a.n; e += stride) {
+  for (size_t pass = 0; pass < a.n; pass += stride) {
+    const size_t e = wave_base(pass, a.n) + (threadIdx.x & 63);
+    if (e >= a.n) continue;
     const uint8_t* key = a.broadcast ? a.keys : a.keys + e * a.key_bytes;
     const uint32_t party = key[2] & 1u;
     uint64_t x = a.xs[e];
@@ -93,6 +109,72 @@ __global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_bytes_kernel(DcfEvalArg
         out[base + b] = uint8_t(word >> (8 * (b & 7)));
       }
     }
+  }
+}
+
+// Small batches: 8 lanes per walk (dcf_quad_device.hpp), a walk being one
+// chunk of one element.  A wave takes 8 consecutive elements' walks; passes
+// deal waves to the workgroups in turn.
+template <int kMode>
+__global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_quad_bit_kernel(DcfEvalArgs a) {
+  SUFHIP_DCF_TABLE_SETUP();
+  const QuadKeys K = load_quad_keys(kernarg_key_sel(offsetof(DcfEvalArgs, key_sel)));
+  // Packed outputs are whole words: the last word's missing elements are 0.
+  const size_t octets = kMode == SUFHIP_DCF_OUT_BIT ? (a.n + 7) / 8 : (a.n + 63) / 64 * 8;
+  const size_t stride = size_t(gridDim.x) * (kDcfBitBlock / 64);
+  const uint32_t lane = threadIdx.x & 63u;
+  for (size_t o = size_t(blockIdx.x) + size_t(gridDim.x) * (threadIdx.x >> 6); o < octets;
+       o += stride) {
+    const size_t e = 8 * o + (lane >> 3);
+    const size_t ec = e < a.n ? e : a.n - 1;  // whole groups of 8 lanes keep walking
+    const uint8_t* key = a.broadcast ? a.keys : a.keys + ec * a.key_bytes;
+    const uint32_t party = key[2] & 1u;
+    const uint64_t x = a.xs[ec];
+    QuadState st = quad_root(key + 8, party);
+    quad_walk<kQuadBit, SUFHIP_GROUP_XOR>(aes, K, key + 8, a.in_bits, 0, a.in_bits, x, party, st);
+    const uint32_t bit = uint32_t(
+        quad_finish<kQuadBit, SUFHIP_GROUP_XOR>(key + 8, a.in_bits, party, false, st).lo);
+    const bool mine = (lane & 7u) == 4u && e < a.n;
+    if constexpr (kMode == SUFHIP_DCF_OUT_BIT) {
+      if (mine) static_cast<uint8_t*>(a.out)[e] = uint8_t(bit);
+    } else {
+      // Bit 8 g + 4 of the ballot is element g of the octet; the product
+      // gathers the eight bits in its top byte.
+      const uint64_t b = __ballot(mine && bit != 0) >> 4;
+      if (lane == 0)
+        static_cast<uint8_t*>(a.out)[o] = uint8_t((b * 0x0102040810204080ull) >> 56);
+    }
+  }
+}
+
+template <int kGroup>
+__global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_quad_bytes_kernel(DcfEvalArgs a) {
+  SUFHIP_DCF_TABLE_SETUP();
+  const QuadKeys K = load_quad_keys(kernarg_key_sel(offsetof(DcfEvalArgs, key_sel)));
+  const size_t chunk_bytes = 32 + 33 * size_t(a.in_bits);
+  const size_t walks = a.n * size_t(a.chunks);
+  const size_t stride = size_t(gridDim.x) * (kDcfBitBlock / 8);
+  for (size_t w = (size_t(blockIdx.x) + size_t(gridDim.x) * (threadIdx.x >> 6)) * 8 +
+                  ((threadIdx.x & 63u) >> 3);
+       w < walks; w += stride) {
+    const size_t e = w / size_t(a.chunks);
+    const int c = int(w - e * size_t(a.chunks));
+    const uint8_t* key = a.broadcast ? a.keys : a.keys + e * a.key_bytes;
+    const uint8_t* chunk = key + 8 + size_t(c) * chunk_bytes;
+    const uint32_t party = key[2] & 1u;
+    const uint64_t x = a.xs[e];
+    const bool more = size_t(c + 1) * chunk_bytes + 8 < a.key_bytes;
+    QuadState st = quad_root(chunk, party);
+    quad_walk<kQuadFull, kGroup>(aes, K, chunk, a.in_bits, 0, a.in_bits, x, party, st);
+    const U128 r = quad_finish<kQuadFull, kGroup>(chunk, a.in_bits, party, more, st);
+    // Lane q of the value half writes word q of the chunk.
+    const uint32_t l = threadIdx.x & 7u, q = l & 3u;
+    const uint64_t half = q < 2 ? r.lo : r.hi;
+    const uint32_t word = uint32_t(half >> (32 * (q & 1u)));
+    uint8_t* out = static_cast<uint8_t*>(a.out) + e * size_t(a.out_bytes) + 16 * c + 4 * q;
+    const int left = a.out_bytes - 16 * c - 4 * int(q);
+    if (l >= 4)
+      for (int b = 0; b < 4 && b < left; ++b) out[b] = uint8_t(word >> (8 * b));
   }
 }
 
@@ -213,23 +295,38 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
   a.out_bytes = out_mode == SUFHIP_DCF_OUT_BYTES ? out_bytes : 1;
   hipStream_t s = as_stream(stream);
   fill_key_sel(a.prg, &a.key_sel);
+  if (out_mode == SUFHIP_DCF_OUT_BYTES) a.chunks = (out_bytes + 15) / 16;
+  const size_t walks = n * size_t(a.chunks);
+  int cus = 0;
+  if (int rc = cu_count(&cus)) return rc;
+  // 8 lanes per walk up to two full passes of them (256 walks per CU), one
+  // lane above: at 300, 32768 and 65536 keys of 64 levels 42, 77 and 140 us
+  // against 134, 138 and 155; at 131072, 276 against 205.  The quad walks are
+  // bound by their serial chain up to one pass and by VALU issue beyond.
+  const bool quad = walks <= 256 * size_t(cus);
+  // Waves of 64 elements, or of 8 quad walks, one workgroup per CU at most.
+  const size_t waves = quad ? (walks + 7) / 8 : (n + 63) / 64;
+  const dim3 grid(unsigned(waves < size_t(cus) ? waves : size_t(cus))), block(kDcfBitBlock);
   if (out_mode != SUFHIP_DCF_OUT_BYTES) {
-    unsigned int g = 0;
-    if (int rc = dcf_grid(n, &g, kDcfBitBlock)) return rc;
-    const dim3 grid(g), block(kDcfBitBlock);
     if (out_mode == SUFHIP_DCF_OUT_BIT) {
-      hipLaunchKernelGGL((dcf_eval_bit_kernel<SUFHIP_DCF_OUT_BIT>), grid, block, 0, s, a);
+      if (quad)
+        hipLaunchKernelGGL((dcf_eval_quad_bit_kernel<SUFHIP_DCF_OUT_BIT>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((dcf_eval_bit_kernel<SUFHIP_DCF_OUT_BIT>), grid, block, 0, s, a);
     } else {
       SUFHIP_REQUIRE((reinterpret_cast<uintptr_t>(d_out) & 7) == 0,
                      "sufhip_dcf_eval: packed output must be 8-byte aligned");
-      hipLaunchKernelGGL((dcf_eval_bit_kernel<SUFHIP_DCF_OUT_PACKED>), grid, block, 0, s, a);
+      if (quad)
+        hipLaunchKernelGGL((dcf_eval_quad_bit_kernel<SUFHIP_DCF_OUT_PACKED>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((dcf_eval_bit_kernel<SUFHIP_DCF_OUT_PACKED>), grid, block, 0, s, a);
     }
   } else {
-    unsigned int g = 0;
-    if (int rc = dcf_grid(n, &g, kDcfBitBlock)) return rc;
-    const dim3 grid(g), block(kDcfBitBlock);
-    a.chunks = (out_bytes + 15) / 16;
-    if (group == SUFHIP_GROUP_XOR)
+    if (quad && group == SUFHIP_GROUP_XOR)
+      hipLaunchKernelGGL((dcf_eval_quad_bytes_kernel<SUFHIP_GROUP_XOR>), grid, block, 0, s, a);
+    else if (quad)
+      hipLaunchKernelGGL((dcf_eval_quad_bytes_kernel<SUFHIP_GROUP_ADD>), grid, block, 0, s, a);
+    else if (group == SUFHIP_GROUP_XOR)
       hipLaunchKernelGGL((dcf_eval_bytes_kernel<SUFHIP_GROUP_XOR>), grid, block, 0, s, a);
     else
       hipLaunchKernelGGL((dcf_eval_bytes_kernel<SUFHIP_GROUP_ADD>), grid, block, 0, s, a);

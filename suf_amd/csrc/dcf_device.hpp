@@ -679,13 +679,19 @@ void fill_prg4(const uint8_t* state, Prg4* p) {
   }
 }
 
+int cu_count(int* cus) {
+  int dev = 0;
+  SUFHIP_CHECK(hipGetDevice(&dev), "hipGetDevice");
+  SUFHIP_CHECK(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev),
+               "hipDeviceGetAttribute(CU count)");
+  return SUFHIP_OK;
+}
+
 // Grid for the grid-stride DCF kernels: one workgroup per CU (LDS-limited),
 // never more workgroups than the batch needs.
 int dcf_grid(size_t n, unsigned int* grid, int block = kDcfBlock) {
-  int dev = 0, cus = 0;
-  SUFHIP_CHECK(hipGetDevice(&dev), "hipGetDevice");
-  SUFHIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev),
-               "hipDeviceGetAttribute(CU count)");
+  int cus = 0;
+  if (int rc = cu_count(&cus)) return rc;
   const size_t need = (n + size_t(block) - 1) / size_t(block);
   *grid = static_cast<unsigned int>(need < size_t(cus) ? need : size_t(cus));
   return SUFHIP_OK;

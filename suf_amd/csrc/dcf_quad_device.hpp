@@ -1,0 +1,207 @@
+// The myl7 DCF walk (third_party/myl7_fss/src/dcf.c:146-193) on 8 lanes, for
+// batches too small to fill the chip with one walk per lane.
+//
+// Lanes 0-3 of a group compute the next-seed block AES_{K_{2b}}(s) and lanes
+// 4-7 the value block AES_{K_{2b+1}}(s), one state column per lane
+// (AesLds4::encrypt_quad_n's scheme).  A level is bounded by its serial
+// chain -- ten rounds of table address, LDS read, three quad exchanges -- and
+// a lane here issues 4 table reads a round where the one-lane walk issues 32,
+// so the chain is 0.65 us a level against 2.1 us (measured at 300 to 8192
+// keys, one or two waves per SIMD).  The exchanges make it 36 VALU operations
+// per block and round instead of 28, so the one-lane walk keeps the batches
+// that fill the chip.
+//
+// A lane only ever needs one column of two keys, K_h and K_{2+h} (h its
+// half), so the round keys live in 22 registers: nothing but table reads goes
+// through the LDS, and the choice of key by the input bit is off the chain.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "dcf_device.hpp"
+
+namespace sufhip {
+namespace {
+
+// Value of lane - 4 in this lane's row of 16 (lanes 4-7 and 12-15 of a row;
+// the others hold nothing of use).
+__device__ __forceinline__ uint32_t row_shr4(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x114, 0xf, 0xf, false));
+}
+
+// Little-endian word at byte address p + 4 idx (any alignment; reads the
+// aligned words idx and idx + 1 around it).
+__device__ __forceinline__ uint32_t word_at(const uint8_t* p, int idx) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
+  return __builtin_amdgcn_alignbyte(w[idx + 1], w[idx], uint32_t(a & 3));
+}
+
+// Round key column q of this lane's half: K_h and K_h ^ K_{2+h}.
+struct QuadKeys {
+  uint32_t k[11], d[11];
+};
+
+__device__ __forceinline__ QuadKeys load_quad_keys(KeySelPtr sel) {
+  QuadKeys K;
+  const uint32_t l = threadIdx.x & 7u;
+  const uint32_t at = (l >> 2) * 8u + (l & 3u);
+#pragma unroll
+  for (int r = 0; r < 11; ++r) {
+    K.k[r] = sel[16 * r + at];
+    K.d[r] = sel[16 * r + at + 4];
+  }
+  return K;
+}
+
+// AES_{K_{2b + h}} of the group's seed (column q in s), b chosen by m = -b.
+__device__ __forceinline__ uint32_t quad_encrypt(const AesLds4& aes, const QuadKeys& K,
+                                                 uint32_t m, uint32_t s) {
+  s ^= xor_and(K.k[0], m, K.d[0]);
+#pragma unroll
+  for (int r = 1; r < 10; ++r) {
+    const uint32_t a0 = aes.t<0, 0>(s);
+    const uint32_t a1 = aes.t<1, 1>(s);
+    const uint32_t a2 = aes.t<2, 2>(s);
+    const uint32_t a3 = aes.t<3, 3>(s);
+    const uint32_t kr = xor_and(K.k[r], m, K.d[r]);
+    s = a0 ^ kr ^ quad_rot<1>(a1) ^ quad_rot<2>(a2) ^ quad_rot<3>(a3);
+  }
+  // Final round: S(x) is byte 0 of T3[x], bytes 1 and 2 of T0[x] and byte 3
+  // of T1[x].
+  const uint32_t u0 = aes.t<3, 0>(s) & 0xffu, u1 = aes.t<0, 1>(s) & 0xff00u;
+  const uint32_t u2 = aes.t<0, 2>(s) & 0xff0000u, u3 = aes.t<1, 3>(s) & 0xff000000u;
+  return u0 ^ xor_and(K.k[10], m, K.d[10]) ^ quad_rot<1>(u1) ^ quad_rot<2>(u2) ^ quad_rot<3>(u3);
+}
+
+// What a walk accumulates: bit 0 of the share, its low 64 bits (additive
+// group: + and - carry only upwards), or all 16 bytes.
+enum QuadVal { kQuadBit, kQuadLow64, kQuadFull };
+
+// A correction word record: the aligned words a lane needs of it, read a
+// level ahead of their use.
+template <int kVal>
+struct QuadCw {
+  static constexpr int kV = kVal == kQuadBit ? 1 : (kVal == kQuadLow64 ? 3 : 5);
+  uint32_t s0, s1;  // words q and q + 1: s_cw column q
+  uint32_t v[kV];   // words 4..: v_cw
+  uint32_t tb;      // word 8: the t byte (bit mode and low 64)
+  uint32_t sh;
+};
+
+template <int kVal>
+__device__ __forceinline__ QuadCw<kVal> load_quad_cw(const uint8_t* p, uint32_t q) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+  GlobalWords w = (GlobalWords)(a & ~uintptr_t(3));
+  QuadCw<kVal> c;
+  c.s0 = w[q];
+  c.s1 = w[q + 1];
+#pragma unroll
+  for (int j = 0; j < QuadCw<kVal>::kV; ++j) c.v[j] = w[4 + j];
+  if constexpr (kVal == kQuadFull)
+    c.tb = 0;
+  else
+    c.tb = w[8];
+  c.sh = uint32_t(a & 3);
+  return c;
+}
+
+// Seed word q (both halves), control bit (both halves), accumulated value
+// (meaningful in the value half; kQuadBit: bit 0 of lane 4's lo).
+struct QuadState {
+  uint32_t s, t;
+  U128 v;
+};
+
+template <int kVal, int kGroup>
+__device__ __forceinline__ void quad_level(const AesLds4& aes, const QuadKeys& K,
+                                           const QuadCw<kVal>& c, uint32_t xi, uint32_t party,
+                                           QuadState& st) {
+  const uint32_t l = threadIdx.x & 7u, q = l & 3u;
+  uint32_t on = quad_encrypt(aes, K, 0u - xi, st.s) ^ st.s;
+  const uint32_t tmask = 0u - st.t;
+  if constexpr (kVal == kQuadBit) {
+    st.v.lo ^= (on ^ ((c.v[0] >> (8 * c.sh)) & tmask)) & 1u;
+  } else if constexpr (kVal == kQuadLow64) {
+    const uint64_t vd0 = uint64_t(quad_bcast<0>(on)) | uint64_t(quad_bcast<1>(on)) << 32;
+    const uint64_t cv = uint64_t(__builtin_amdgcn_alignbyte(c.v[1], c.v[0], c.sh)) |
+                        uint64_t(__builtin_amdgcn_alignbyte(c.v[2], c.v[1], c.sh)) << 32;
+    const uint64_t vd = vd0 + (st.t ? cv : 0);
+    st.v.lo += party ? 0 - vd : vd;
+  } else {
+    U128 vd = mk(quad_bcast<0>(on), quad_bcast<1>(on), quad_bcast<2>(on),
+                 quad_bcast<3>(on) & 0x7fffffffu);
+    const U128 cv = mk(__builtin_amdgcn_alignbyte(c.v[1], c.v[0], c.sh),
+                       __builtin_amdgcn_alignbyte(c.v[2], c.v[1], c.sh),
+                       __builtin_amdgcn_alignbyte(c.v[3], c.v[2], c.sh),
+                       __builtin_amdgcn_alignbyte(c.v[4], c.v[3], c.sh));
+    if (st.t) vd = gadd<kGroup>(vd, cv);
+    if (party) vd = gneg<kGroup>(vd);
+    st.v = gadd<kGroup>(st.v, vd);
+  }
+  const uint32_t tb = (kVal == kQuadFull ? c.v[QuadCw<kVal>::kV - 1] : c.tb) >> (8 * c.sh);
+  uint32_t tn = quad_bcast<3>(on) >> 31;
+  if (q == 3) on &= 0x7fffffffu;
+  on ^= __builtin_amdgcn_alignbyte(c.s1, c.s0, c.sh) & tmask;
+  tn ^= (xi ? tb : (tb >> 1)) & st.t & 1u;
+  // The seed half's next seed and t move to the value half (lane - 4).
+  const uint32_t os = row_shr4(on), ts = row_shr4(tn);
+  st.s = l >= 4 ? os : on;
+  st.t = l >= 4 ? ts : tn;
+}
+
+__device__ __forceinline__ QuadState quad_root(const uint8_t* chunk, uint32_t party) {
+  const uint32_t q = threadIdx.x & 3u;
+  uint32_t s = word_at(chunk, int(q));
+  if (q == 3) s &= 0x7fffffffu;
+  return QuadState{s, party, U128{0, 0}};
+}
+
+// Levels [from, to) of an in_bits-level walk at x, each record read a level
+// ahead of its use.
+template <int kVal, int kGroup>
+__device__ __forceinline__ void quad_walk(const AesLds4& aes, const QuadKeys& K,
+                                          const uint8_t* chunk, int in_bits, int from, int to,
+                                          uint64_t x, uint32_t party, QuadState& st) {
+  const uint32_t q = threadIdx.x & 3u;
+  const uint8_t* cw = chunk + 16 + 33 * from;
+  if (from >= to) return;
+  QuadCw<kVal> c = load_quad_cw<kVal>(cw, q);
+#pragma unroll 1
+  for (int i = from; i < to; ++i) {
+    // The last level's look-ahead reads its own record again.
+    if (i + 1 < to) cw += 33;
+    const QuadCw<kVal> next = load_quad_cw<kVal>(cw, q);
+    quad_level<kVal, kGroup>(aes, K, c, uint32_t(x >> (in_bits - 1 - i)) & 1u, party, st);
+    c = next;
+  }
+}
+
+// Share after the last level: v + (-1)^party (s + t cw_np1), in the value
+// half (kQuadBit: bit 0, in lane 4).
+template <int kVal, int kGroup>
+__device__ __forceinline__ U128 quad_finish(const uint8_t* chunk, int in_bits, uint32_t party,
+                                            bool more_after, const QuadState& st) {
+  const uint8_t* np1 = chunk + 16 + 33 * in_bits;
+  if constexpr (kVal == kQuadBit) {
+    return U128{(st.v.lo ^ st.s ^ (word_at(np1, 0) & st.t)) & 1u, 0};
+  } else {
+    uint32_t n[4];
+    load16_bytes(np1, more_after, n);
+    U128 sv = mk(quad_bcast<0>(st.s), quad_bcast<1>(st.s), quad_bcast<2>(st.s),
+                 quad_bcast<3>(st.s));
+    if constexpr (kVal == kQuadLow64) {
+      const uint64_t s = sv.lo + (st.t ? mk(n[0], n[1], 0, 0).lo : 0);
+      return U128{st.v.lo + (party ? 0 - s : s), 0};
+    } else {
+      if (st.t) sv = gadd<kGroup>(sv, mk(n[0], n[1], n[2], n[3]));
+      if (party) sv = gneg<kGroup>(sv);
+      return gadd<kGroup>(st.v, sv);
+    }
+  }
+}
+
+}  // namespace
+}  // namespace sufhip

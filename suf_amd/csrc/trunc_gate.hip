@@ -374,14 +374,6 @@ __global__ void __launch_bounds__(kDcfBlock) trunc_batch_expand_kernel(BatchLeve
   }
 }
 
-int cu_count(int* cus) {
-  int dev = 0;
-  SUFHIP_CHECK(hipGetDevice(&dev), "hipGetDevice");
-  SUFHIP_CHECK(hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev),
-               "hipDeviceGetAttribute(CU count)");
-  return SUFHIP_OK;
-}
-
 // Launch shape for the frontier kernels: spread `count` lanes over all CUs
 // (one workgroup per CU, the AES tables fill its LDS), 256..512 lanes each.
 int spread_grid(size_t count, unsigned int* grid, unsigned int* block) {

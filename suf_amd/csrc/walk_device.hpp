@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "dcf_device.hpp"
+#include "dcf_quad_device.hpp"
 #include "suf_hip.h"
 #include "trunc_device.hpp"
 
@@ -94,18 +95,6 @@ struct Walk8 {
   uint32_t t;  // control bit (both halves)
   uint64_t v;  // accumulated value, low 64 bits (value half)
 };
-
-// Little-endian word at byte address p + 4 idx (any alignment; reads the
-// aligned words idx and idx + 1 around it).
-__device__ __forceinline__ uint32_t word_at(const uint8_t* p, int idx) {
-  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(a & ~uintptr_t(3));
-  return __builtin_amdgcn_alignbyte(w[idx + 1], w[idx], uint32_t(a & 3));
-}
-
-__device__ __forceinline__ uint32_t row_shr4(uint32_t v) {
-  return uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x114, 0xf, 0xf, false));
-}
 
 template <class Aes>
 struct Walk8Ctx {

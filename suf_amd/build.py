@@ -42,10 +42,6 @@ HIPCC_FLAGS = [
 # Kernels allowed a private segment, with the reason.  Every other kernel
 # must report ScratchSize 0, or the build fails.
 SCRATCH_ALLOWED = {
-    # Dealer-side keygen (not on the online path): the four PRG blocks of a
-    # level, indexed by the block loop, spill 144 bytes per lane.
-    "dcf_gen_kernel": "dealer keygen",
-    "trunc_gen_kernel": "dealer keygen",
     # SGPR spill slots only: the block's ~100 uniform pointers exceed the
     # SGPR file, and the compiler keeps the overflow in VGPR lanes
     # (v_writelane / v_readlane).  The frame size is reported, but the kernel

@@ -26,6 +26,7 @@
 #include <cstring>
 
 #include "dcf_device.hpp"
+#include "dcf_gen_device.hpp"
 #include "dcf_quad_device.hpp"
 
 namespace sufhip {
@@ -195,17 +196,22 @@ struct DcfGenArgs {
   int chunks;
 };
 
-// myl7 dcf_gen (third_party/myl7_fss/src/dcf.c:42-142) for kLtAlpha, one key
-// pair per lane, written in the adapter layout (myl7_fss_backend.hpp:156-210).
+// Key generation: 8 lanes per chunk of a key pair (dcf_gen_device.hpp).  A
+// wave takes 8 consecutive walks; passes deal waves to the workgroups in turn.
 template <int kGroup>
-__global__ void __launch_bounds__(kDcfBlock) dcf_gen_kernel(DcfGenArgs a) {
-  SUFHIP_DCF_LDS_SETUP(a.prg);
-  const size_t stride = size_t(gridDim.x) * kDcfBlock;
-  for (size_t e = size_t(blockIdx.x) * kDcfBlock + threadIdx.x; e < a.n; e += stride) {
+__global__ void __launch_bounds__(kDcfBitBlock) dcf_gen_kernel(DcfGenArgs a) {
+  SUFHIP_DCF_TABLE_SETUP();
+  const GenKeys K = load_gen_keys(kernarg_key_sel(offsetof(DcfGenArgs, prg)));
+  const size_t walks = a.n * size_t(a.chunks);
+  const size_t stride = size_t(gridDim.x) * (kDcfBitBlock / 8);
+  for (size_t w = (size_t(blockIdx.x) + size_t(gridDim.x) * (threadIdx.x >> 6)) * 8 +
+                  ((threadIdx.x & 63u) >> 3);
+       w < walks; w += stride) {
+    const size_t e = w / size_t(a.chunks);
+    const int c = int(w - e * size_t(a.chunks));
     const uint8_t* pay = a.payload_bcast ? a.payload : a.payload + e * size_t(a.payload_len);
-    gen_key<kGroup>(aes, rkl, a.in_bits, a.chunks, a.payload_len, a.alpha[e], pay,
-                    a.seeds + e * size_t(a.chunks) * 32, a.keys0 + e * a.key_bytes,
-                    a.keys1 + e * a.key_bytes);
+    gen_chunk<kGroup>(aes, K, a.in_bits, a.chunks, a.payload_len, c, a.alpha[e], pay,
+                      a.seeds + w * 32, a.keys0 + e * a.key_bytes, a.keys1 + e * a.key_bytes);
   }
 }
 
@@ -251,14 +257,14 @@ int sufhip_dcf_gen(int group, int in_bits, const uint8_t* prg_state, const uint6
   a.payload_len = payload_len;
   a.in_bits = in_bits;
   a.chunks = (payload_len + 15) / 16;
-  unsigned int g = 0;
-  if (int rc = dcf_grid(n, &g)) return rc;
+  int cus = 0;
+  if (int rc = cu_count(&cus)) return rc;
+  const size_t waves = (n * size_t(a.chunks) + 7) / 8;
+  const dim3 grid(unsigned(waves < size_t(cus) ? waves : size_t(cus))), block(kDcfBitBlock);
   if (group == SUFHIP_GROUP_XOR)
-    hipLaunchKernelGGL((dcf_gen_kernel<SUFHIP_GROUP_XOR>), dim3(g), dim3(kDcfBlock), 0,
-                       as_stream(stream), a);
+    hipLaunchKernelGGL((dcf_gen_kernel<SUFHIP_GROUP_XOR>), grid, block, 0, as_stream(stream), a);
   else
-    hipLaunchKernelGGL((dcf_gen_kernel<SUFHIP_GROUP_ADD>), dim3(g), dim3(kDcfBlock), 0,
-                       as_stream(stream), a);
+    hipLaunchKernelGGL((dcf_gen_kernel<SUFHIP_GROUP_ADD>), grid, block, 0, as_stream(stream), a);
   return check_launch("dcf_gen_kernel");
 }
 

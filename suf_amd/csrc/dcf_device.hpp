@@ -520,158 +520,6 @@ __device__ __forceinline__ uint64_t add64_finish(const uint8_t* chunk, int in_bi
   __syncthreads();                                                 \
   const DcfAes aes = DcfAes::make(tabs)
 
-// Sequential little-endian byte writer: stores aligned dwords where it can
-// and single bytes at unaligned edges, so lanes writing neighbouring keys
-// never touch each other's bytes.
-struct ByteWriter {
-  uint8_t* p;
-  uint64_t acc;
-  int n;
-  __device__ __forceinline__ void drain() {
-    while (n > 0) {
-      if ((reinterpret_cast<uintptr_t>(p) & 3) == 0) {
-        if (n < 4) break;
-        *reinterpret_cast<uint32_t*>(p) = uint32_t(acc);
-        p += 4;
-        acc >>= 32;
-        n -= 4;
-      } else {
-        *p = uint8_t(acc);
-        ++p;
-        acc >>= 8;
-        --n;
-      }
-    }
-  }
-  __device__ __forceinline__ void put8(uint32_t b) {
-    acc |= uint64_t(b & 0xffu) << (8 * n);
-    ++n;
-    drain();
-  }
-  __device__ __forceinline__ void put32(uint32_t w) {
-    acc |= uint64_t(w) << (8 * n);
-    n += 4;
-    drain();
-  }
-  __device__ __forceinline__ void flush() {
-    while (n > 0) {
-      *p = uint8_t(acc);
-      ++p;
-      acc >>= 8;
-      --n;
-    }
-  }
-};
-
-__device__ __forceinline__ void prg4(const DcfAes& aes, const uint4* rkl, const U128& s,
-                                     U128 (&o)[4]) {
-  const uint32_t w0 = uint32_t(s.lo), w1 = uint32_t(s.lo >> 32), w2 = uint32_t(s.hi),
-                 w3 = uint32_t(s.hi >> 32);
-  // One block at a time keeps the dealer kernel inside the register budget.
-#pragma unroll 1
-  for (int j = 0; j < 4; ++j) {
-    uint32_t a0 = w0, a1 = w1, a2 = w2, a3 = w3;
-    aes.encrypt(a0, a1, a2, a3, rkl + 11 * j);
-    o[j] = mk(a0 ^ w0, a1 ^ w1, a2 ^ w2, a3 ^ w3);
-  }
-}
-
-__device__ __forceinline__ void put128(ByteWriter& w, U128 v) {
-  w.put32(uint32_t(v.lo));
-  w.put32(uint32_t(v.lo >> 32));
-  w.put32(uint32_t(v.hi));
-  w.put32(uint32_t(v.hi >> 32));
-}
-
-// One DCF key pair for f(x) = beta * 1[x < alpha] (myl7 dcf_gen,
-// third_party/myl7_fss/src/dcf.c:42-142), written in the adapter layout
-// (include/proto/myl7_fss_backend.hpp:156-210).  seeds: [chunks][32]
-// (party-0 seed, party-1 seed).
-template <int kGroup>
-__device__ __forceinline__ void gen_key(const DcfAes& aes, const uint4* rkl, int nb, int chunks,
-                                        int payload_len, uint64_t alpha, const uint8_t* pay,
-                                        const uint8_t* seeds, uint8_t* out0, uint8_t* out1) {
-  if (nb < 64) alpha &= (uint64_t(1) << nb) - 1;
-  ByteWriter w0{out0, 0, 0};
-  ByteWriter w1{out1, 0, 0};
-  const uint32_t plen = uint32_t(payload_len);
-  w0.put32(uint32_t(nb) | uint32_t(chunks) << 8 | 0u << 16);
-  w1.put32(uint32_t(nb) | uint32_t(chunks) << 8 | 1u << 16);
-  w0.put32(plen);
-  w1.put32(plen);
-  for (int c = 0; c < chunks; ++c) {
-    uint8_t beta_b[16];
-    for (int b = 0; b < 16; ++b) {
-      const int idx = 16 * c + b;
-      beta_b[b] = idx < payload_len ? pay[idx] : 0;
-    }
-    U128 beta{0, 0};
-    for (int b = 0; b < 8; ++b) beta.lo |= uint64_t(beta_b[b]) << (8 * b);
-    for (int b = 0; b < 8; ++b) beta.hi |= uint64_t(beta_b[8 + b]) << (8 * b);
-    beta.hi &= kMsbClear;
-    const uint8_t* sp = seeds + size_t(c) * 32;
-    uint32_t sw[8];
-    for (int j = 0; j < 8; ++j) {
-      sw[j] = uint32_t(sp[4 * j]) | uint32_t(sp[4 * j + 1]) << 8 | uint32_t(sp[4 * j + 2]) << 16 |
-              uint32_t(sp[4 * j + 3]) << 24;
-    }
-    for (int j = 0; j < 4; ++j) w0.put32(sw[j]);
-    for (int j = 0; j < 4; ++j) w1.put32(sw[4 + j]);
-    U128 s0 = mk(sw[0], sw[1], sw[2], sw[3]);
-    U128 s1 = mk(sw[4], sw[5], sw[6], sw[7]);
-    s0.hi &= kMsbClear;
-    s1.hi &= kMsbClear;
-    uint32_t t0 = 0, t1 = 1;
-    U128 v{0, 0};
-    for (int i = 0; i < nb; ++i) {
-      U128 e0[4], e1[4];
-      prg4(aes, rkl, s0, e0);
-      prg4(aes, rkl, s1, e1);
-      const uint32_t t0l = uint32_t(e0[0].hi >> 63), t0r = uint32_t(e0[2].hi >> 63);
-      const uint32_t t1l = uint32_t(e1[0].hi >> 63), t1r = uint32_t(e1[2].hi >> 63);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        e0[j].hi &= kMsbClear;
-        e1[j].hi &= kMsbClear;
-      }
-      const uint32_t ai = uint32_t(alpha >> (nb - 1 - i)) & 1u;
-      // lose = side alpha does not take, keep = side it takes
-      const U128 s0_lose = ai ? e0[0] : e0[2], s1_lose = ai ? e1[0] : e1[2];
-      const U128 v0_lose = ai ? e0[1] : e0[3], v1_lose = ai ? e1[1] : e1[3];
-      const U128 s0_keep = ai ? e0[2] : e0[0], s1_keep = ai ? e1[2] : e1[0];
-      const U128 v0_keep = ai ? e0[3] : e0[1], v1_keep = ai ? e1[3] : e1[1];
-      const U128 s_cw{s0_lose.lo ^ s1_lose.lo, s0_lose.hi ^ s1_lose.hi};
-      U128 v_cw = gadd<kGroup>(v1_lose, gneg<kGroup>(v0_lose));
-      v_cw = gadd<kGroup>(v_cw, gneg<kGroup>(v));
-      if (t1) v_cw = gneg<kGroup>(v_cw);
-      if (ai) v_cw = gadd<kGroup>(v_cw, t1 ? gneg<kGroup>(beta) : beta);
-      v = gadd<kGroup>(v, gneg<kGroup>(v1_keep));
-      v = gadd<kGroup>(v, v0_keep);
-      v = gadd<kGroup>(v, t1 ? gneg<kGroup>(v_cw) : v_cw);
-      const uint32_t tl_cw = t0l ^ t1l ^ ai ^ 1u;
-      const uint32_t tr_cw = t0r ^ t1r ^ ai;
-      put128(w0, s_cw);
-      put128(w1, s_cw);
-      put128(w0, v_cw);
-      put128(w1, v_cw);
-      w0.put8(tl_cw << 1 | tr_cw);
-      w1.put8(tl_cw << 1 | tr_cw);
-      const uint32_t t0k = ai ? t0r : t0l, t1k = ai ? t1r : t1l, tcwk = ai ? tr_cw : tl_cw;
-      s0 = t0 ? U128{s0_keep.lo ^ s_cw.lo, s0_keep.hi ^ s_cw.hi} : s0_keep;
-      s1 = t1 ? U128{s1_keep.lo ^ s_cw.lo, s1_keep.hi ^ s_cw.hi} : s1_keep;
-      t0 = t0 ? (t0k ^ tcwk) : t0k;
-      t1 = t1 ? (t1k ^ tcwk) : t1k;
-    }
-    U128 last = gadd<kGroup>(s1, gneg<kGroup>(s0));
-    last = gadd<kGroup>(last, gneg<kGroup>(v));
-    if (t1) last = gneg<kGroup>(last);
-    put128(w0, last);
-    put128(w1, last);
-  }
-  w0.flush();
-  w1.flush();
-}
-
 // K_0..K_3 expanded (FIPS-197 word order).
 void fill_prg4(const uint8_t* state, Prg4* p) {
   for (int j = 0; j < 4; ++j) {

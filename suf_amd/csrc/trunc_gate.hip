@@ -30,10 +30,12 @@
 // one launch.
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <mutex>
 #include <string>
 
 #include "dcf_device.hpp"
+#include "dcf_gen_device.hpp"
 #include "suf_hip.h"
 #include "trunc_device.hpp"
 #include "walk_device.hpp"
@@ -87,10 +89,11 @@ struct TruncGenArgs {
   uint32_t total;
 };
 
-// One workgroup: zero both blobs, write the headers, then lanes 0..2 each
-// generate one DCF key pair.
+// One workgroup: zero both blobs, write the headers, then three groups of 8
+// lanes generate one DCF key pair each, in waves of their own.
 __global__ void __launch_bounds__(kDcfBlock) trunc_gen_kernel(TruncGenArgs a) {
-  SUFHIP_DCF_LDS_SETUP(a.prg);
+  SUFHIP_DCF_TABLE_SETUP();
+  const GenKeys K = load_gen_keys(kernarg_key_sel(offsetof(TruncGenArgs, prg)));
   __shared__ uint8_t one8[8];
   __shared__ uint8_t seeds[3][32];
   if (threadIdx.x < 8) one8[threadIdx.x] = threadIdx.x == 0 ? 1 : 0;
@@ -105,10 +108,10 @@ __global__ void __launch_bounds__(kDcfBlock) trunc_gen_kernel(TruncGenArgs a) {
     reinterpret_cast<uint64_t*>(a.key1)[i] = v1;
   }
   __syncthreads();
-  const int j = threadIdx.x;
-  if (j < 3 && (a.flags >> j) & 1)
-    gen_key<SUFHIP_GROUP_ADD>(aes, rkl, a.bits[j], 1, 8, a.alpha[j], one8, seeds[j],
-                              a.key0 + a.off[j], a.key1 + a.off[j]);
+  const int j = threadIdx.x >> 6;
+  if (j < 3 && (threadIdx.x & 63) < 8 && (a.flags >> j) & 1)
+    gen_chunk<SUFHIP_GROUP_ADD>(aes, K, a.bits[j], 1, 8, 0, a.alpha[j], one8, seeds[j],
+                                a.key0 + a.off[j], a.key1 + a.off[j]);
 }
 
 // Frontier node v: {s0, s1, s2, s3} and {v_lo, v_hi, t, 0}.  With d == f the

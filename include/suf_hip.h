@@ -155,6 +155,21 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
                     const uint64_t* d_xs, size_t n, int out_mode, int out_bytes, void* d_out,
                     void* stream);
 
+/* One party's comparison bits of several broadcast keys (1-byte payload) at
+ * the same N points, in one launch per 64 keys: what sufhip_dcf_eval gives in
+ * mode SUFHIP_DCF_OUT_BIT for each key (composite_eval_batch_backend's
+ * predicate and cut queries, composite_fss.hpp:2132-2250).  jobs is a host
+ * array; job j writes d_out [N] bytes. */
+typedef struct sufhip_dcf_key_job {
+  const uint8_t* d_key;
+  size_t key_bytes;
+  uint8_t* d_out;
+  int in_bits;
+} sufhip_dcf_key_job;
+int sufhip_dcf_eval_keys(const uint8_t* prg_state, const sufhip_dcf_key_job* jobs, int count,
+                         const uint64_t* d_xs, size_t n, void* stream);
+
+
 /* ---------------------------------------------------------------------- */
 /* Truncation gate (one instance, scalar input mask r), both halves of SUF's */
 /* trunc pipeline: keygen composite_gen_trunc_gate                           */

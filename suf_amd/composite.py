@@ -25,8 +25,8 @@ Dealer (compile_suf_to_pfss_two_programs, src/compiler/suf_to_pfss.cpp:
     boolean outputs of the piece it comes from;
   * one broadcast myl7 DCF key pair (payload 1, XOR group) per query and per
     cut; bit triples for AND / OR; Beaver triples for the network.
-Online: the DCF bits of every query and cut at the public x^ (one launch per
-key and party), the whole selector / boolean network for both parties in one
+Online: the DCF bits of every query and cut, both parties, at the public x^
+(one launch, sufhip_dcf_eval_keys), the whole selector / boolean network for both parties in one
 launch (sufhip_composite_bool2), and the arithmetic words through the
 interval LUT of the rotated pieces (sufhip_interval_lut_eval2).
 
@@ -362,14 +362,17 @@ class CompositeGate:
     def pred_bits(self, xhat):
         """Both parties' XOR-shared bits of every query and cut at x^ (int64[n])."""
         n = self.n
-        for q, (bits, k0, k1) in enumerate(self.query_keys):
-            for p, k in ((0, k0), (1, k1)):
-                pfss.dcf_eval(native.GROUP_XOR, bits, 1, self.prg_state, k, xhat, broadcast=True,
-                              out=self.pred[p][q * n:(q + 1) * n])
-        for c, (bits, k0, k1) in enumerate(self.cut_keys):
-            for p, k in ((0, k0), (1, k1)):
-                pfss.dcf_eval(native.GROUP_XOR, bits, 1, self.prg_state, k, xhat, broadcast=True,
-                              out=self.cutb[p][c * n:(c + 1) * n])
+        jobs = (native.DcfKeyJob * (2 * (len(self.query_keys) + len(self.cut_keys))))()
+        j = 0
+        for keys, outs in ((self.query_keys, self.pred), (self.cut_keys, self.cutb)):
+            base = [ptr(outs[0]), ptr(outs[1])]
+            for q, key in enumerate(keys):
+                for p in (0, 1):
+                    k = key[1 + p]
+                    jobs[j] = (ptr(k), k.shape[-1], base[p] + q * n, key[0])
+                    j += 1
+        native.call("sufhip_dcf_eval_keys", pfss._state_buf(self.prg_state), jobs, j, ptr(xhat),
+                    xhat.numel(), stream_ptr())
 
     def args(self, out_bool):
         a = native.CompositeBoolArgs()

@@ -224,16 +224,14 @@ __device__ __forceinline__ CwBit decode_cw(const CwRaw& w) {
 // Bit-mode walk of one chunk: returns share byte 0 & 1.  The seed block is
 // AES_{K_{2 x_i}}(s) ^ s in full; of the value block only byte 0 is formed
 // (round 9 column 0, then one final S-box byte).
-__device__ __forceinline__ uint32_t walk_bit(const AesLds4& aes, KeySelPtr keys,
-                                             const uint8_t* chunk, int in_bits, uint64_t x,
-                                             uint32_t party) {
-  uint32_t seed[4];
-  load16_bytes(chunk, true, seed);
-  uint32_t s[4] = {seed[0], seed[1], seed[2], seed[3] & 0x7fffffffu};
-  uint32_t t = party;
-  uint32_t v = 0;
-  const uint8_t* cw = chunk + 16;
-  for (int i = 0; i < in_bits; ++i, cw += 33) {
+// walk_bit_from continues at level `from` with seed s, control bit t and
+// accumulated bit v.
+__device__ __forceinline__ uint32_t walk_bit_from(const AesLds4& aes, KeySelPtr keys,
+                                                  const uint8_t* chunk, int in_bits, int from,
+                                                  uint64_t x, uint32_t (&s)[4], uint32_t t,
+                                                  uint32_t v) {
+  const uint8_t* cw = chunk + 16 + 33 * from;
+  for (int i = from; i < in_bits; ++i, cw += 33) {
     const uint32_t xi = uint32_t(x >> (in_bits - 1 - i)) & 1u;
     const uint32_t m = 0u - xi;
     const CwRaw cr = load_cw_raw(cw);
@@ -297,6 +295,15 @@ __device__ __forceinline__ uint32_t walk_bit(const AesLds4& aes, KeySelPtr keys,
   return (v ^ s[0] ^ (np1[0] & t)) & 1u;
 }
 
+__device__ __forceinline__ uint32_t walk_bit(const AesLds4& aes, KeySelPtr keys,
+                                             const uint8_t* chunk, int in_bits, uint64_t x,
+                                             uint32_t party) {
+  uint32_t seed[4];
+  load16_bytes(chunk, true, seed);
+  uint32_t s[4] = {seed[0], seed[1], seed[2], seed[3] & 0x7fffffffu};
+  return walk_bit_from(aes, keys, chunk, in_bits, 0, x, s, party, 0);
+}
+
 // The aligned words 0..8 around a 33-byte correction-word record (s_cw,
 // v_cw, the t byte), read with global loads at the start of a level and
 // decoded after its AES (as CwRaw for the bit walk).
@@ -326,9 +333,64 @@ __device__ __forceinline__ CwFull decode_cw_full(const CwRawFull& w) {
   return c;
 }
 
-// Full-block walk of one chunk (any group): returns the 16-byte share.  The
-// same scheme as walk_bit -- round keys chosen per lane from scalar
-// registers, grouped rounds -- with both blocks computed in full.
+// Both blocks of a level, as walk_bit forms them (round keys chosen per lane
+// from scalar registers, grouped rounds): o = AES_{K_{2b}}(s) ^ s and the
+// first kW words (2 or 4) of AES_{K_{2b+1}}(s) ^ s in ob, m = -b.
+template <int kW>
+__device__ __forceinline__ void sel_blocks(const AesLds4& aes, KeySelPtr keys, uint32_t m,
+                                           const uint32_t (&s)[4], uint32_t (&o)[4],
+                                           uint32_t (&ob)[kW]) {
+  KeySelPtr k = keys;
+  asm volatile("" : "+s"(k));
+  uint32_t A[4], B[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    A[j] = xor_and(s[j], m, k[4 + j]) ^ k[j];
+    B[j] = xor_and(s[j], m, k[12 + j]) ^ k[8 + j];
+  }
+#pragma unroll
+  for (int r = 1; r < 10; ++r) key_sel_round<4>(aes, k + 16 * r, m, A, B);
+  // Final round of both blocks: S(x) is byte 0 of T3[x], bytes 1 and 2 of
+  // T0[x] and byte 3 of T1[x].
+  constexpr int kN = 16 + 4 * kW;
+  uint32_t ad[kN];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    ad[4 * c + 0] = __builtin_amdgcn_perm(A[c], aes.base[3], AesLds4::sel(0));
+    ad[4 * c + 1] = __builtin_amdgcn_perm(A[(c + 1) & 3], aes.base[0], AesLds4::sel(1));
+    ad[4 * c + 2] = __builtin_amdgcn_perm(A[(c + 2) & 3], aes.base[0], AesLds4::sel(2));
+    ad[4 * c + 3] = __builtin_amdgcn_perm(A[(c + 3) & 3], aes.base[1], AesLds4::sel(3));
+    if (c < kW) {
+      ad[16 + 4 * c + 0] = __builtin_amdgcn_perm(B[c], aes.base[3], AesLds4::sel(0));
+      ad[16 + 4 * c + 1] = __builtin_amdgcn_perm(B[(c + 1) & 3], aes.base[0], AesLds4::sel(1));
+      ad[16 + 4 * c + 2] = __builtin_amdgcn_perm(B[(c + 2) & 3], aes.base[0], AesLds4::sel(2));
+      ad[16 + 4 * c + 3] = __builtin_amdgcn_perm(B[(c + 3) & 3], aes.base[1], AesLds4::sel(3));
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  uint32_t tv[kN];
+#pragma unroll
+  for (int n = 0; n < kN; ++n) tv[n] = lds_word(aes.lds, ad[n]);
+  const KeySelPtr q = k + 160;
+  uint32_t kq[16];
+#pragma unroll
+  for (int n = 0; n < 16; ++n) kq[n] = q[n];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t lo = __builtin_amdgcn_perm(tv[4 * c + 1], tv[4 * c], 0x0c0c0500u);
+    const uint32_t hi = __builtin_amdgcn_perm(tv[4 * c + 3], tv[4 * c + 2], 0x07020c0cu);
+    o[c] = xor_and(SUFHIP_BITOP3(lo, hi, s[c], 0x56) ^ kq[c], m, kq[4 + c]);
+    if (c < kW) {
+      const uint32_t lb = __builtin_amdgcn_perm(tv[16 + 4 * c + 1], tv[16 + 4 * c], 0x0c0c0500u);
+      const uint32_t hb =
+          __builtin_amdgcn_perm(tv[16 + 4 * c + 3], tv[16 + 4 * c + 2], 0x07020c0cu);
+      ob[c < kW ? c : 0] = xor_and(SUFHIP_BITOP3(lb, hb, s[c], 0x56) ^ kq[8 + c], m, kq[12 + c]);
+    }
+  }
+}
+
+// Full-block walk of one chunk (any group): returns the 16-byte share.
 template <int kGroup>
 __device__ __forceinline__ U128 walk_full(const AesLds4& aes, KeySelPtr keys, const uint8_t* chunk,
                                           int in_bits, uint64_t x, uint32_t party,
@@ -341,51 +403,9 @@ __device__ __forceinline__ U128 walk_full(const AesLds4& aes, KeySelPtr keys, co
   const uint8_t* cw = chunk + 16;
   for (int i = 0; i < in_bits; ++i, cw += 33) {
     const uint32_t xi = uint32_t(x >> (in_bits - 1 - i)) & 1u;
-    const uint32_t m = 0u - xi;
     const CwRawFull cr = load_cw_raw_full(cw);
-    KeySelPtr k = keys;
-    asm volatile("" : "+s"(k));
-    uint32_t A[4], B[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      A[j] = xor_and(s[j], m, k[4 + j]) ^ k[j];
-      B[j] = xor_and(s[j], m, k[12 + j]) ^ k[8 + j];
-    }
-#pragma unroll
-    for (int r = 1; r < 10; ++r) key_sel_round<4>(aes, k + 16 * r, m, A, B);
-    // Final round of both blocks: S(x) is byte 0 of T3[x], bytes 1 and 2 of
-    // T0[x] and byte 3 of T1[x].
-    uint32_t ad[32];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      ad[4 * c + 0] = __builtin_amdgcn_perm(A[c], aes.base[3], AesLds4::sel(0));
-      ad[4 * c + 1] = __builtin_amdgcn_perm(A[(c + 1) & 3], aes.base[0], AesLds4::sel(1));
-      ad[4 * c + 2] = __builtin_amdgcn_perm(A[(c + 2) & 3], aes.base[0], AesLds4::sel(2));
-      ad[4 * c + 3] = __builtin_amdgcn_perm(A[(c + 3) & 3], aes.base[1], AesLds4::sel(3));
-      ad[16 + 4 * c + 0] = __builtin_amdgcn_perm(B[c], aes.base[3], AesLds4::sel(0));
-      ad[16 + 4 * c + 1] = __builtin_amdgcn_perm(B[(c + 1) & 3], aes.base[0], AesLds4::sel(1));
-      ad[16 + 4 * c + 2] = __builtin_amdgcn_perm(B[(c + 2) & 3], aes.base[0], AesLds4::sel(2));
-      ad[16 + 4 * c + 3] = __builtin_amdgcn_perm(B[(c + 3) & 3], aes.base[1], AesLds4::sel(3));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    uint32_t tv[32];
-#pragma unroll
-    for (int n = 0; n < 32; ++n) tv[n] = lds_word(aes.lds, ad[n]);
-    const KeySelPtr q = k + 160;
-    uint32_t kq[16];
-#pragma unroll
-    for (int n = 0; n < 16; ++n) kq[n] = q[n];
-    __builtin_amdgcn_sched_barrier(0);
     uint32_t o[4], ob[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const uint32_t lo = __builtin_amdgcn_perm(tv[4 * c + 1], tv[4 * c], 0x0c0c0500u);
-      const uint32_t hi = __builtin_amdgcn_perm(tv[4 * c + 3], tv[4 * c + 2], 0x07020c0cu);
-      o[c] = xor_and(SUFHIP_BITOP3(lo, hi, s[c], 0x56) ^ kq[c], m, kq[4 + c]);
-      const uint32_t lb = __builtin_amdgcn_perm(tv[16 + 4 * c + 1], tv[16 + 4 * c], 0x0c0c0500u);
-      const uint32_t hb = __builtin_amdgcn_perm(tv[16 + 4 * c + 3], tv[16 + 4 * c + 2], 0x07020c0cu);
-      ob[c] = xor_and(SUFHIP_BITOP3(lb, hb, s[c], 0x56) ^ kq[8 + c], m, kq[12 + c]);
-    }
+    sel_blocks<4>(aes, keys, 0u - xi, s, o, ob);
     const CwFull c = decode_cw_full(cr);
     U128 vd = mk(ob[0], ob[1], ob[2], ob[3] & 0x7fffffffu);
     uint32_t tn = o[3] >> 31;
@@ -488,6 +508,37 @@ __device__ __forceinline__ void add64_walk(const DcfAes& aes, const uint4* rkl,
     st.s1 = a1;
     st.s2 = a2;
     st.s3 = a3;
+    st.t = tn;
+  }
+}
+
+// add64_walk with the round keys in scalar registers (sel_blocks), for 1024
+// lanes per CU.
+__device__ __forceinline__ void walk_low64(const DcfAes& aes, KeySelPtr keys,
+                                           const uint8_t* chunk, int in_bits, int from, int to,
+                                           uint64_t x, uint32_t party, Add64State& st) {
+  const uint8_t* cw = chunk + 16 + 33 * from;
+  for (int i = from; i < to; ++i, cw += 33) {
+    const uint32_t xi = uint32_t(x >> (in_bits - 1 - i)) & 1u;
+    const CwRawFull cr = load_cw_raw_full(cw);
+    const uint32_t s[4] = {st.s0, st.s1, st.s2, st.s3};
+    uint32_t o[4], ob[2];
+    sel_blocks<2>(aes, keys, 0u - xi, s, o, ob);
+    const CwFull c = decode_cw_full(cr);
+    uint64_t vd = uint64_t(ob[0]) | uint64_t(ob[1]) << 32;
+    uint32_t tn = o[3] >> 31;
+    o[3] &= 0x7fffffffu;
+    if (st.t) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] ^= c.s[j];
+      tn ^= (xi ? c.tb : (c.tb >> 1)) & 1u;
+      vd += uint64_t(c.v[0]) | uint64_t(c.v[1]) << 32;
+    }
+    st.v += party ? 0 - vd : vd;
+    st.s0 = o[0];
+    st.s1 = o[1];
+    st.s2 = o[2];
+    st.s3 = o[3];
     st.t = tn;
   }
 }

@@ -74,6 +74,7 @@ _SIGS = {
     "sufhip_trunc_noalloc_max_work_bytes": (c_sz, []),
     "sufhip_trunc_eval_noalloc": (c_int, [c_int, c_int, c_vp, c_vp, c_sz, c_vp, c_sz, c_vp, c_vp]),
     "sufhip_trunc_prepare": (c_int, [c_int, c_int, c_vp, c_vp, c_sz, c_sz, c_vp, c_sz, c_vp]),
+    "sufhip_dcf_eval_keys": (c_int, [c_vp, c_vp, c_int, c_vp, c_sz, c_vp]),
     "sufhip_stage_hatx": (c_int, [c_vp, c_int, c_vp, c_sz, c_vp]),
     "sufhip_open_flush2_work_bytes": (c_sz, [c_sz, c_int]),
     "sufhip_open_flush2": (c_int, [c_vp, c_int, c_int, c_int, c_int, c_vp, c_vp, c_sz, c_vp]),
@@ -302,6 +303,11 @@ COMPOSITE_MAX_CUTS = 31
 COMPOSITE_MAX_WRAP = 32
 COMPOSITE_MAX_PROG = 384
 STAGE_MAX_SEGS = 64
+
+
+class DcfKeyJob(ctypes.Structure):
+    """sufhip_dcf_key_job (include/suf_hip.h)."""
+    _fields_ = [("d_key", c_vp), ("key_bytes", c_sz), ("d_out", c_vp), ("in_bits", c_int)]
 
 
 class StageSeg(ctypes.Structure):

@@ -122,11 +122,11 @@ __device__ __forceinline__ void forest_build(const AesLds4& aes, const QuadKeys&
   }
 }
 
-// Expansion depth for a tile of `points` points: none while the points walk
-// on 8 lanes each (a level of the expansion then costs what it saves), else
-// about one node per point.
+// Expansion depth for a tile of `points` points: none while their walks take
+// one pass of the workgroup on 8 lanes each (a level of the expansion then
+// costs what it saves), else about one node per point.
 inline int forest_depth(size_t points, int trees) {
-  if (points * size_t(trees) <= 256) return 0;
+  if (points * size_t(trees) <= 128) return 0;
   int d = 0;
   while ((size_t(2) << d) <= points && (trees << (d + 1)) <= kForestNodes) ++d;
   return d;

@@ -35,6 +35,7 @@
 #include <string>
 
 #include "dcf_device.hpp"
+#include "dcf_forest_device.hpp"
 #include "dcf_gen_device.hpp"
 #include "suf_hip.h"
 #include "trunc_device.hpp"
@@ -116,69 +117,8 @@ __global__ void __launch_bounds__(kDcfBlock) trunc_gen_kernel(TruncGenArgs a) {
 
 // Frontier node v: {s0, s1, s2, s3} and {v_lo, v_hi, t, 0}.  With d == f the
 // node's value word holds the final share at point v.
-struct FrontierArgs {
-  Prg4 prg;
-  const uint8_t* key;
-  uint4* nodes;
-  int f;
-  int d;
-};
-
-__global__ void __launch_bounds__(kDcfBlock) trunc_frontier_kernel(FrontierArgs a) {
-  SUFHIP_DCF_LDS_SETUP(a.prg);
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= (1u << a.d) || !(a.key[7] & 1)) return;
-  const uint32_t party = a.key[6] & 1u;
-  const uint8_t* chunk = a.key + kHdrBytes + 8;
-  const uint64_t x = uint64_t(v) << (a.f - a.d);
-  Add64State st = add64_root(chunk, party);
-  add64_walk(aes, rkl, chunk, a.f, 0, a.d, x, party, st);
-  if (a.d == a.f) {
-    const uint64_t out = add64_finish(chunk, a.f, party, st);
-    a.nodes[2 * v + 1] = make_uint4(uint32_t(out), uint32_t(out >> 32), 0, 0);
-  } else {
-    a.nodes[2 * v] = make_uint4(st.s0, st.s1, st.s2, st.s3);
-    a.nodes[2 * v + 1] = make_uint4(uint32_t(st.v), uint32_t(st.v >> 32), st.t, 0);
-  }
-}
-
-// One breadth-first level: nodes at depth `level` (in) -> depth level + 1
-// (out), one child per lane.  When level + 1 == f the children are final
-// shares.
-struct ExpandArgs {
-  Prg4 prg;
-  const uint8_t* key;
-  const uint4* in;
-  uint4* out;
-  int f;
-  int level;
-};
-
-__global__ void __launch_bounds__(kDcfBlock) trunc_expand_kernel(ExpandArgs a) {
-  SUFHIP_DCF_LDS_SETUP(a.prg);
-  if (!(a.key[7] & 1)) return;
-  const uint32_t party = a.key[6] & 1u;
-  const uint8_t* chunk = a.key + kHdrBytes + 8;
-  const uint32_t count = 2u << a.level;
-  for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < count;
-       c += gridDim.x * blockDim.x) {
-    const uint4 s = a.in[2 * (c >> 1)], q = a.in[2 * (c >> 1) + 1];
-    Add64State st{s.x, s.y, s.z, s.w, q.z, uint64_t(q.x) | uint64_t(q.y) << 32};
-    const uint64_t x = uint64_t(c & 1u) << (a.f - 1 - a.level);
-    add64_walk(aes, rkl, chunk, a.f, a.level, a.level + 1, x, party, st);
-    if (a.level + 1 == a.f) {
-      const uint64_t out = add64_finish(chunk, a.f, party, st);
-      a.out[2 * c + 1] = make_uint4(uint32_t(out), uint32_t(out >> 32), 0, 0);
-    } else {
-      a.out[2 * c] = make_uint4(st.s0, st.s1, st.s2, st.s3);
-      a.out[2 * c + 1] = make_uint4(uint32_t(st.v), uint32_t(st.v >> 32), st.t, 0);
-    }
-  }
-}
-
 // One launch evaluates one or both parties: grid.y selects the party slot.
 struct TruncEvalArgs {
-  Prg4 prg;
   const uint8_t* keys[2];
   const uint64_t* xhat;
   uint64_t* ys[2];
@@ -186,6 +126,12 @@ struct TruncEvalArgs {
   size_t n;
   int f;
   int d;
+  // trunc_eval_aes_kernel's launch (launch_finish).
+  DcfKeySel key_sel;
+  size_t tile;  // points per workgroup
+  int depth;    // expansion depth of a tile's trees
+  int span;     // item slots per key and pass
+  int quad;     // items walk on 8 lanes each
 };
 
 using Hdr = TruncHdr;
@@ -202,54 +148,132 @@ __device__ __forceinline__ uint64_t carry_from(const Hdr& h, uint64_t a) {
   return trunc_carry_from(h, a);
 }
 
-// Every DCF walk the element needs runs here (frontier continuation, 64-bit
-// wrap / sign keys).
+// Gates with DCF walks per element: the 64-bit wrap key (TR, ARS) and sign
+// key (ARS), and the carry key where the frontier stops above its leaves.  A
+// workgroup takes a tile of points: the levels that they share under the
+// 64-bit keys are walked once and a subtree is expanded in LDS
+// (dcf_forest_device.hpp); the items, (key, point) pairs, then continue one to
+// a lane, or one to 8 lanes where a tile has few, and meet in LDS for the
+// postproc.  ARS over 98304 points of 30 bits, one party: 175 us (445 with
+// one lane walking both 64-level keys in turn).
+constexpr int kEvalItems = 1024;
+
 template <int kKind>
-__global__ void __launch_bounds__(kDcfBlock) trunc_eval_aes_kernel(TruncEvalArgs a) {
-  SUFHIP_DCF_LDS_SETUP(a.prg);
+__global__ void __launch_bounds__(kForestBlock) trunc_eval_aes_kernel(TruncEvalArgs a) {
+  constexpr int kTrees = kKind == SUFHIP_TRUNC_ARS ? 2 : 1;
+  __shared__ ForestLds lds;
+  __shared__ uint64_t share[kEvalItems];
+  const size_t first = size_t(blockIdx.x) * a.tile;
+  const size_t count = a.n - first < a.tile ? a.n - first : a.tile;
+  const uint64_t* xs = a.xhat + first;
+  const uint64_t x0 = xs[0];
+  const uint64_t diff = kKind == SUFHIP_TRUNC_GAPARS ? 0 : xor_points(xs, count, x0);
+  if (threadIdx.x < 2) lds.diff[threadIdx.x] = 0;
+  SUFHIP_DCF_TABLE_SETUP();
+  const KeySelPtr keys = kernarg_key_sel(offsetof(TruncEvalArgs, key_sel));
+  const QuadKeys K = load_quad_keys(keys);
   const uint8_t* key = a.keys[blockIdx.y];
   const uint4* nodes = a.tables[blockIdx.y];
-  uint64_t* y = a.ys[blockIdx.y];
+  uint64_t* y = a.ys[blockIdx.y] + first;
   const Hdr h = read_hdr(key);
   const uint8_t* carry_chunk = key + kHdrBytes + 8;
   const uint8_t* wrap_chunk = key + kHdrBytes + pad8(h.ckb) + 8;
   const uint8_t* sign_chunk = wrap_chunk + pad8(h.ukb);
   const uint64_t low = (uint64_t(1) << a.f) - 1;
-  const size_t stride = size_t(gridDim.x) * kDcfBlock;
-  for (size_t e = size_t(blockIdx.x) * kDcfBlock + threadIdx.x; e < a.n; e += stride) {
-    const uint64_t x = a.xhat[e];
-    uint64_t carry = 0, wrap = 0, sign = 0;
-    if (h.flags & 1) {
-      const uint64_t xl = x & low;
-      uint64_t share;
-      if (a.d == a.f) {
-        const uint4 q = nodes[2 * xl + 1];
-        share = uint64_t(q.x) | uint64_t(q.y) << 32;
-      } else {
-        Add64State st;
-        if (a.d > 0) {
-          const size_t v = size_t(xl >> (a.f - a.d));
-          const uint4 s = nodes[2 * v], q = nodes[2 * v + 1];
-          st = Add64State{s.x, s.y, s.z, s.w, q.z, uint64_t(q.x) | uint64_t(q.y) << 32};
+  int from = 0, D = 0;
+  if constexpr (kKind != SUFHIP_TRUNC_GAPARS) {
+    const int L = shared_levels(lds, diff, 64);
+    D = a.depth < 64 - L ? a.depth : 64 - L;
+    from = L + D;
+    ForestTree tree[kTrees];
+    tree[0] = ForestTree{wrap_chunk, h.party};
+    if constexpr (kTrees == 2) tree[1] = ForestTree{sign_chunk, h.party};
+    forest_build<kQuadLow64, kTrees>(aes, K, tree, 64, x0, L, D, lds);
+  }
+  // Items of a pass: wrap, then sign, then the carry's walks, `span` slots
+  // each (a multiple of 64, so a wave has one key).
+  constexpr int kDcf = kKind == SUFHIP_TRUNC_GAPARS ? 0 : kTrees;
+  const bool carry_walk = (h.flags & 1) && a.d < a.f;
+  const int span = a.span;
+  const int kinds = kDcf + (carry_walk ? 1 : 0);
+  for (size_t pass = 0; pass < count; pass += size_t(span)) {
+    const int m = int(count - pass < size_t(span) ? count - pass : size_t(span));
+    if (a.quad) {
+      for (int it = int(threadIdx.x >> 3); it < kinds * m; it += kForestBlock / 8) {
+        const int p = it / m, i = it - p * m;
+        uint64_t x = xs[pass + size_t(i)];
+        const uint8_t* chunk = p == 0 ? wrap_chunk : sign_chunk;
+        int bits = 64, at = from;
+        QuadState st;
+        if (p == kDcf) {
+          x &= low;
+          chunk = carry_chunk;
+          bits = a.f;
+          at = a.d;
+          st = quad_root(chunk, h.party);
+          if (a.d > 0) {
+            const size_t v = size_t(x >> (a.f - a.d));
+            const uint4 qn = nodes[2 * v + 1];
+            st.s = reinterpret_cast<const uint32_t*>(nodes + 2 * v)[threadIdx.x & 3u];
+            st.t = qn.z;
+            st.v.lo = uint64_t(qn.x) | uint64_t(qn.y) << 32;
+          }
         } else {
-          st = add64_root(carry_chunk, h.party);
+          st = forest_get(lds, D & 1, forest_node(x, 64 - from, D) * kTrees + p);
         }
-        add64_walk(aes, rkl, carry_chunk, a.f, a.d, a.f, xl, h.party, st);
-        share = add64_finish(carry_chunk, a.f, h.party, st);
+        quad_walk<kQuadLow64, SUFHIP_GROUP_ADD>(aes, K, chunk, bits, at, bits, x, h.party, st);
+        const U128 r =
+            quad_finish<kQuadLow64, SUFHIP_GROUP_ADD>(chunk, bits, h.party, false, st);
+        if ((threadIdx.x & 7u) == 4u) share[p * span + i] = r.lo;
       }
-      carry = carry_from(h, share);
+    } else {
+      const int p = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / span);
+      const int i = int(threadIdx.x) - p * span;
+      if (p < kinds && i < m) {
+        uint64_t x = xs[pass + size_t(i)];
+        const uint8_t* chunk = p == 0 ? wrap_chunk : sign_chunk;
+        int bits = 64, at = from;
+        Add64State st;
+        if (p == kDcf) {
+          x &= low;
+          chunk = carry_chunk;
+          bits = a.f;
+          at = a.d;
+          if (a.d > 0) {
+            const size_t v = size_t(x >> (a.f - a.d));
+            const uint4 s = nodes[2 * v], q = nodes[2 * v + 1];
+            st = Add64State{s.x, s.y, s.z, s.w, q.z, uint64_t(q.x) | uint64_t(q.y) << 32};
+          } else {
+            st = add64_root(chunk, h.party);
+          }
+        } else {
+          const int node = forest_node(x, 64 - from, D) * kTrees + p;
+          const uint4 s = lds.s[D & 1][node];
+          st = Add64State{s.x, s.y, s.z, s.w, lds.t[D & 1][node], lds.v[D & 1][node]};
+        }
+        walk_low64(aes, keys, chunk, bits, at, bits, x, h.party, st);
+        share[p * span + i] = add64_finish(chunk, bits, h.party, st);
+      }
     }
-    if constexpr (kKind != SUFHIP_TRUNC_GAPARS) {
-      Add64State st = add64_root(wrap_chunk, h.party);
-      add64_walk(aes, rkl, wrap_chunk, 64, 0, 64, x, h.party, st);
-      wrap = add64_finish(wrap_chunk, 64, h.party, st);
+    __syncthreads();
+    for (int i = int(threadIdx.x); i < m; i += kForestBlock) {
+      const uint64_t x = xs[pass + size_t(i)];
+      uint64_t carry = 0, wrap = 0, sign = 0;
+      if (h.flags & 1) {
+        uint64_t c;
+        if (carry_walk) {
+          c = share[kDcf * span + i];
+        } else {
+          const uint4 q = nodes[2 * (x & low) + 1];
+          c = uint64_t(q.x) | uint64_t(q.y) << 32;
+        }
+        carry = carry_from(h, c);
+      }
+      if constexpr (kKind != SUFHIP_TRUNC_GAPARS) wrap = share[i];
+      if constexpr (kKind == SUFHIP_TRUNC_ARS) sign = (wrap - share[span + i]) + h.sw;
+      y[pass + size_t(i)] = postproc<kKind>(h, a.f, x, carry, wrap, sign);
     }
-    if constexpr (kKind == SUFHIP_TRUNC_ARS) {
-      Add64State st = add64_root(sign_chunk, h.party);
-      add64_walk(aes, rkl, sign_chunk, 64, 0, 64, x, h.party, st);
-      sign = (wrap - add64_finish(sign_chunk, 64, h.party, st)) + h.sw;
-    }
-    y[e] = postproc<kKind>(h, a.f, x, carry, wrap, sign);
+    __syncthreads();
   }
 }
 
@@ -414,7 +438,8 @@ constexpr size_t kMaxElems = size_t(1) << 38;
 
 // Finish for `parties` (1 or 2) key slots: the table kernel for GapARS with
 // a full-domain table, else the DCF-walk kernel.
-int launch_finish(int kind, const TruncEvalArgs& a, int parties, hipStream_t s) {
+int launch_finish(int kind, const uint8_t* prg_state, TruncEvalArgs& a, int parties,
+                  hipStream_t s) {
   if (kind == SUFHIP_TRUNC_GAPARS && a.d == a.f) {
     size_t blocks = (a.n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
@@ -422,16 +447,30 @@ int launch_finish(int kind, const TruncEvalArgs& a, int parties, hipStream_t s) 
                        a);
     return check_launch("trunc_eval_table_kernel");
   }
-  unsigned int g = 0;
-  if (int rc = dcf_grid(a.n, &g)) return rc;
-  const dim3 grid(g, parties);
+  Prg4 prg;
+  fill_prg4(prg_state, &prg);
+  fill_key_sel(prg, &a.key_sel);
+  int cus = 0;
+  if (int rc = cu_count(&cus)) return rc;
+  // One workgroup per CU for all parties (the AES tables fill its LDS), at
+  // least 8 points each.
+  size_t tiles = size_t(cus / parties > 0 ? cus / parties : 1);
+  a.tile = (a.n + tiles - 1) / tiles;
+  if (a.tile < 8) a.tile = 8;
+  tiles = (a.n + a.tile - 1) / a.tile;
+  const int trees = kind == SUFHIP_TRUNC_GAPARS ? 0 : (kind == SUFHIP_TRUNC_ARS ? 2 : 1);
+  const int kinds = trees + (a.d < a.f ? 1 : 0);
+  a.quad = a.tile * size_t(kinds) <= 256;
+  a.depth = trees > 0 ? forest_depth(a.tile, trees) : 0;
+  a.span = kEvalItems / kinds / 64 * 64;
+  const dim3 grid{unsigned(tiles), unsigned(parties)};
   if (kind == SUFHIP_TRUNC_GAPARS)
-    hipLaunchKernelGGL(trunc_eval_aes_kernel<SUFHIP_TRUNC_GAPARS>, grid, dim3(kDcfBlock), 0, s,
+    hipLaunchKernelGGL(trunc_eval_aes_kernel<SUFHIP_TRUNC_GAPARS>, grid, dim3(kForestBlock), 0, s,
                        a);
   else if (kind == SUFHIP_TRUNC_TR)
-    hipLaunchKernelGGL(trunc_eval_aes_kernel<SUFHIP_TRUNC_TR>, grid, dim3(kDcfBlock), 0, s, a);
+    hipLaunchKernelGGL(trunc_eval_aes_kernel<SUFHIP_TRUNC_TR>, grid, dim3(kForestBlock), 0, s, a);
   else
-    hipLaunchKernelGGL(trunc_eval_aes_kernel<SUFHIP_TRUNC_ARS>, grid, dim3(kDcfBlock), 0, s, a);
+    hipLaunchKernelGGL(trunc_eval_aes_kernel<SUFHIP_TRUNC_ARS>, grid, dim3(kForestBlock), 0, s, a);
   return check_launch("trunc_eval_aes_kernel");
 }
 
@@ -693,32 +732,9 @@ int sufhip_trunc_prepare(int kind, int frac_bits, const uint8_t* prg_state, cons
   if (int rc = trunc_check("sufhip_trunc_prepare", kind, frac_bits, prg_state, d_key, key_bytes,
                            n, d_work, work_bytes))
     return rc;
-  const int d = frontier_bits(frac_bits, n);
-  if (n == 0 || d == 0) return SUFHIP_OK;
-  hipStream_t s = as_stream(stream);
-  Prg4 prg;
-  fill_prg4(prg_state, &prg);
-  // Walk to depth k0, then expand level by level, alternating between the
-  // two workspace regions so that depth d ends in the first one.
-  uint4* lvl[2] = {static_cast<uint4*>(d_work), static_cast<uint4*>(d_work) + 2 * (size_t(1) << d)};
-  const int k0 = walk_bits(d);
-  int cur = (d - k0) & 1;
-  FrontierArgs fa{prg, d_key, lvl[cur], frac_bits, k0};
-  unsigned int g = 0, b = 0;
-  if (int rc = spread_grid(size_t(1) << k0, &g, &b)) return rc;
-  // The walk kernel is one lane per node (no stride loop): cover all nodes.
-  g = unsigned(((size_t(1) << k0) + b - 1) / b);
-  hipLaunchKernelGGL(trunc_frontier_kernel, dim3(g), dim3(b), 0, s, fa);
-  if (int rc = check_launch("trunc_frontier_kernel")) return rc;
-  for (int level = k0; level < d; ++level) {
-    ExpandArgs ea{prg, d_key, lvl[cur], lvl[cur ^ 1], frac_bits, level};
-    unsigned int eg = 0, eb = 0;
-    if (int rc = spread_grid(size_t(2) << level, &eg, &eb)) return rc;
-    hipLaunchKernelGGL(trunc_expand_kernel, dim3(eg), dim3(eb), 0, s, ea);
-    if (int rc = check_launch("trunc_expand_kernel")) return rc;
-    cur ^= 1;
-  }
-  return SUFHIP_OK;
+  if (n == 0) return SUFHIP_OK;
+  const sufhip_trunc_job job{kind, frac_bits, d_key, key_bytes, n, d_work, work_bytes};
+  return sufhip_trunc_prepare_batch(prg_state, &job, 1, stream);
 }
 
 int sufhip_trunc_finish(int kind, int frac_bits, const uint8_t* prg_state, const uint8_t* d_key,
@@ -731,11 +747,9 @@ int sufhip_trunc_finish(int kind, int frac_bits, const uint8_t* prg_state, const
   SUFHIP_REQUIRE(d_xhat && d_y, "sufhip_trunc_finish: null pointer");
   const int d = frontier_bits(frac_bits, n);
   hipStream_t s = as_stream(stream);
-  Prg4 prg;
-  fill_prg4(prg_state, &prg);
   const uint4* tab = static_cast<const uint4*>(d_work);
-  TruncEvalArgs a{prg, {d_key, d_key}, d_xhat, {d_y, d_y}, {tab, tab}, n, frac_bits, d};
-  return launch_finish(kind, a, 1, s);
+  TruncEvalArgs a{{d_key, d_key}, d_xhat, {d_y, d_y}, {tab, tab}, n, frac_bits, d};
+  return launch_finish(kind, prg_state, a, 1, s);
 }
 
 int sufhip_trunc_finish2(int kind, int frac_bits, const uint8_t* prg_state, const uint8_t* d_key0,
@@ -750,17 +764,14 @@ int sufhip_trunc_finish2(int kind, int frac_bits, const uint8_t* prg_state, cons
     return rc;
   if (n == 0) return SUFHIP_OK;
   SUFHIP_REQUIRE(d_xhat && d_y0 && d_y1, "sufhip_trunc_finish2: null pointer");
-  Prg4 prg;
-  fill_prg4(prg_state, &prg);
-  TruncEvalArgs a{prg,
-                  {d_key0, d_key1},
+  TruncEvalArgs a{{d_key0, d_key1},
                   d_xhat,
                   {d_y0, d_y1},
                   {static_cast<const uint4*>(d_work0), static_cast<const uint4*>(d_work1)},
                   n,
                   frac_bits,
                   frontier_bits(frac_bits, n)};
-  return launch_finish(kind, a, 2, as_stream(stream));
+  return launch_finish(kind, prg_state, a, 2, as_stream(stream));
 }
 
 int sufhip_trunc_prepare_batch(const uint8_t* prg_state, const sufhip_trunc_job* jobs, int count,

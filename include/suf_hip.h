@@ -797,7 +797,9 @@ int sufhip_beaver_matmul2_batched(const uint64_t* d_D_open, const uint64_t* d_E_
  * aligned.  sufhip_beaver_matmul2_mfma_batched: the planes of D, E, A_p,
  * B_p and C_p, out_p as in sufhip_beaver_matmul2_batched; M, K, N multiples
  * of 32, K <= 4096 (exact int32 accumulation).  planes_a0 (optional, with
- * a0): also the planes of src[i] + a0[i] (as in sufhip_kb_planes). */
+ * a0): also the planes of src[i] + a0[i] (as in sufhip_kb_planes).
+ * valid_rows, valid_cols (optional): src and a0 are [batches][valid_rows x
+ * valid_cols], and the planes' other rows and columns are zero. */
 #define SUFHIP_KB_SPLIT_JOBS 8
 typedef struct sufhip_kb_split_job {
   const uint64_t* src;
@@ -806,6 +808,7 @@ typedef struct sufhip_kb_split_job {
   int k_is_col;
   int8_t* planes_a0;
   const uint64_t* a0;
+  int valid_rows, valid_cols; /* the source's own extent; 0, 0: rows, cols */
 } sufhip_kb_split_job;
 /* sufhip_beaver_matmul2_mfma_ex: the same product with options.  merge_heads:
  * outputs at [m][b N + n] (heads side by side, as attention_forward merges
@@ -818,7 +821,10 @@ typedef struct sufhip_kb_split_job {
  * (party 0's own value after the open, sufhip_kb_planes.planes_a0).  With
  * it each party's share takes two operand products per k-step,
  *   out_0 = C_0 + (D + A_0) E + D B_0,   out_1 = C_1 + A_1 E + D B_1,
- * the same shares as the three-product form that runs without it. */
+ * the same shares as the three-product form that runs without it.  valid_m,
+ * valid_n (optional, with Xp, without merge_heads and out_planes): C_p and the
+ * outputs are [batches][valid_m x valid_n], M and N the padded extents of
+ * planes written with valid_rows / valid_cols. */
 typedef struct sufhip_beaver_mfma2_args {
   const int8_t* Dp;
   const int8_t* Ep;
@@ -832,6 +838,7 @@ typedef struct sufhip_beaver_mfma2_args {
   uint64_t mask;
   sufhip_x_planes out_planes;
   const int8_t* Xp;
+  int valid_m, valid_n;
 } sufhip_beaver_mfma2_args;
 int sufhip_beaver_matmul2_mfma_ex(const sufhip_beaver_mfma2_args* args, void* stream);
 size_t sufhip_kb_planes_bytes(int batches, int rows, int cols);
@@ -858,6 +865,7 @@ typedef struct sufhip_kb_open_job {
   int8_t* planes_a0; /* optional, with a0: planes of the open + a0[i] */
   const uint64_t* a0;
   int64_t a_stride[3];
+  int valid_rows, valid_cols; /* as in sufhip_kb_split_job, without a_stride */
 } sufhip_kb_open_job;
 int sufhip_kb_open_split_batch(const sufhip_kb_open_job* jobs, int count, void* stream);
 /* sufhip_kb_open_split_prepare: sufhip_trunc_prepare_batch(prg_state, tjobs,

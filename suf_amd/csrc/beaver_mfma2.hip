@@ -42,6 +42,8 @@ struct SplitArgs {
   int8_t* planes_a0[kSplitJobs];       // optional: planes of the value + a0[i]
   const uint64_t* a0[kSplitJobs];
   int batches[kSplitJobs], rows[kSplitJobs], cols[kSplitJobs], k_is_col[kSplitJobs];
+  // The source's own extent; rows and cols past it are zero digits.
+  int vrows[kSplitJobs], vcols[kSplitJobs];
   // src and add read through a strided view (batch, row, col strides; all
   // zero: the plain [batches][rows][cols] index of the other arrays).
   size_t view[kSplitJobs][3];
@@ -105,7 +107,8 @@ __device__ __forceinline__ void write_k(int8_t* planes, size_t plane, size_t off
 }
 
 // Lanes first, first + stride, ... of a split launch over `a`.
-template <int kColK, int kRowK>
+// kRagged: some job's source is smaller than its planes (never with a view).
+template <int kColK, int kRowK, bool kRagged>
 __device__ __forceinline__ void split_lanes(const SplitArgs& a, size_t first, size_t stride) {
   const size_t total = a.begin[a.count];
   for (size_t g = first; g < total; g += stride) {
@@ -120,17 +123,20 @@ __device__ __forceinline__ void split_lanes(const SplitArgs& a, size_t first, si
       const size_t per_batch = size_t(R) * (K / kRowK);
       const size_t b = q / per_batch, rem = q % per_batch;
       const int r = int(rem / (K / kRowK)), k = kRowK * int(rem % (K / kRowK));
-      const size_t src = b * size_t(rows) * cols + size_t(r) * cols + k;
+      const size_t vc = kRagged ? size_t(a.vcols[j]) : size_t(cols);
+      const size_t vr = kRagged ? size_t(a.vrows[j]) : size_t(rows);
+      const size_t src = b * vr * vc + size_t(r) * vc + k;
+      const auto in = [&](int t) { return !kRagged || (size_t(r) < vr && size_t(k + t) < vc); };
       const size_t off = b * size_t(R) * K + kblock_off(size_t(r), k, size_t(R));
       const size_t sv = view_index(a, j, b, size_t(r), size_t(k), src);
       const size_t cs = (a.view[j][0] | a.view[j][1] | a.view[j][2]) ? a.view[j][2] : 1;
       uint64_t v[kRowK];
 #pragma unroll
-      for (int t = 0; t < kRowK; ++t) v[t] = split_val(a, j, src + t, sv + t * cs);
+      for (int t = 0; t < kRowK; ++t) v[t] = in(t) ? split_val(a, j, src + t, sv + t * cs) : 0;
       write_k<kRowK>(a.planes[j], plane, off, v);
       if (a.planes_a0[j]) {
 #pragma unroll
-        for (int t = 0; t < kRowK; ++t) v[t] += a.a0[j][src + t];
+        for (int t = 0; t < kRowK; ++t) v[t] += in(t) ? a.a0[j][src + t] : 0;
         write_k<kRowK>(a.planes_a0[j], plane, off, v);
       }
     } else {
@@ -140,27 +146,30 @@ __device__ __forceinline__ void split_lanes(const SplitArgs& a, size_t first, si
       const int kq = int(rem % kSeg), kb = int(rem / (kSeg * size_t(R)));
       const int r = int((rem / kSeg) % size_t(R));
       const int k0 = 32 * kb + kColK * kq;
-      const size_t src = b * size_t(rows) * cols + size_t(k0) * cols + r;
+      const size_t vc = kRagged ? size_t(a.vcols[j]) : size_t(cols);
+      const size_t vr = kRagged ? size_t(a.vrows[j]) : size_t(rows);
+      const size_t src = b * vr * vc + size_t(k0) * vc + r;
+      const auto in = [&](int t) { return !kRagged || (size_t(r) < vc && size_t(k0 + t) < vr); };
       const size_t off = b * size_t(R) * K + kblock_off(size_t(r), k0, size_t(R));
       const size_t sv = view_index(a, j, b, size_t(k0), size_t(r), src);
-      const size_t rs = (a.view[j][0] | a.view[j][1] | a.view[j][2]) ? a.view[j][1] : size_t(cols);
+      const size_t rs = (a.view[j][0] | a.view[j][1] | a.view[j][2]) ? a.view[j][1] : vc;
       uint64_t v[kColK];
 #pragma unroll
       for (int t = 0; t < kColK; ++t)
-        v[t] = split_val(a, j, src + size_t(t) * cols, sv + size_t(t) * rs);
+        v[t] = in(t) ? split_val(a, j, src + size_t(t) * vc, sv + size_t(t) * rs) : 0;
       write_k<kColK>(a.planes[j], plane, off, v);
       if (a.planes_a0[j]) {
 #pragma unroll
-        for (int t = 0; t < kColK; ++t) v[t] += a.a0[j][src + size_t(t) * cols];
+        for (int t = 0; t < kColK; ++t) v[t] += in(t) ? a.a0[j][src + size_t(t) * vc] : 0;
         write_k<kColK>(a.planes_a0[j], plane, off, v);
       }
     }
   }
 }
 
-template <int kColK, int kRowK>
+template <int kColK, int kRowK, bool kRagged>
 __global__ void __launch_bounds__(256) kb_split_kernel(SplitArgs a) {
-  split_lanes<kColK, kRowK>(a, size_t(blockIdx.x) * 256 + threadIdx.x, size_t(gridDim.x) * 256);
+  split_lanes<kColK, kRowK, kRagged>(a, size_t(blockIdx.x) * 256 + threadIdx.x, size_t(gridDim.x) * 256);
 }
 
 // The opens' digit planes and the key-only walks of truncation gates in one
@@ -194,6 +203,7 @@ struct SplitWalkArgs {
 constexpr int kTileK = 32, kTileN = 64;
 using SplitTile = uint64_t[kTileK][kTileN + 1];  // + 1: the column reads spread over banks
 
+template <bool kRagged>
 __device__ __forceinline__ void split_tile(const SplitArgs& a, int j, uint32_t tile,
                                            SplitTile& E) {
   const int K = a.rows[j], N = a.cols[j];
@@ -201,13 +211,17 @@ __device__ __forceinline__ void split_tile(const SplitArgs& a, int j, uint32_t t
   const uint32_t b = tile / per_b, rem = tile - b * per_b;
   const int kb = int(rem / tn), nb = int(rem - (rem / tn) * tn);
   const size_t bk = size_t(b) * size_t(K) * size_t(N);
-  const size_t base = bk + size_t(kb) * kTileK * N + size_t(nb) * kTileN;
+  const size_t vk = kRagged ? size_t(a.vrows[j]) : size_t(K);
+  const size_t vn = kRagged ? size_t(a.vcols[j]) : size_t(N);
+  const size_t base = size_t(b) * vk * vn + size_t(kb) * kTileK * vn + size_t(nb) * kTileN;
   uint64_t v[kTileK * kTileN / 256];
 #pragma unroll
   for (int i = 0; i < kTileK * kTileN / 256; ++i) {
     const int e = int(threadIdx.x) + 256 * i;
-    const size_t idx = base + size_t(e / kTileN) * N + (e % kTileN);
-    v[i] = split_val(a, j, idx, idx);
+    const int r = e / kTileN, c = e % kTileN;
+    const size_t idx = base + size_t(r) * vn + c;
+    const bool in = !kRagged || (size_t(kb) * kTileK + r < vk && size_t(nb) * kTileN + c < vn);
+    v[i] = in ? split_val(a, j, idx, idx) : 0;
   }
   __syncthreads();  // the previous tile's column reads are done
 #pragma unroll
@@ -238,7 +252,7 @@ __device__ __forceinline__ void split_tile(const SplitArgs& a, int j, uint32_t t
 // lane form (25.7 against 26.6 us at config 3's shape); alone they do not
 // (22.0 against 20.6 us for the triples' planes), so only the launch with
 // walks uses them.
-template <bool kWalk>
+template <bool kWalk, bool kRagged>
 __global__ void __launch_bounds__(256) kb_split_tiled_kernel(SplitWalkArgs a) {
   __shared__ SplitTile E;
   const uint32_t wg = kWalk ? a.walk_groups : 0u;
@@ -263,18 +277,18 @@ __global__ void __launch_bounds__(256) kb_split_tiled_kernel(SplitWalkArgs a) {
     for (uint32_t t = blockIdx.x - wg; t < total; t += a.tile_groups) {
       int u = 0;
       while (u + 1 < a.tcount && t >= a.tbegin[u + 1]) ++u;
-      split_tile(a.s, a.tjob[u], t - a.tbegin[u], E);
+      split_tile<kRagged>(a.s, a.tjob[u], t - a.tbegin[u], E);
     }
     return;
   }
   const uint32_t first = wg + a.tile_groups;
-  split_lanes<4, 4>(a.s, size_t(blockIdx.x - first) * 256 + threadIdx.x,
+  split_lanes<4, 4, kRagged>(a.s, size_t(blockIdx.x - first) * 256 + threadIdx.x,
                     size_t(gridDim.x - first) * 256);
 }
 
 static_assert(sizeof(SplitWalkArgs) <= 4096, "kernel argument block must fit in 4 KB");
 
-template <int kColK, int kRowK>
+template <int kColK, int kRowK, bool kRagged>
 __global__ void __launch_bounds__(256) kb_split_walk_kernel(SplitWalkArgs a) {
   __shared__ __align__(16) uint32_t tab[FusedAes::kWords];
   __shared__ uint4 rkl[4 * 11];
@@ -290,7 +304,7 @@ __global__ void __launch_bounds__(256) kb_split_walk_kernel(SplitWalkArgs a) {
     walk_leaf_path(aes, rkl, a.w.key[j], a.w.out[j], a.w.geo[j], g - a.w.begin[j], gl);
     return;
   }
-  split_lanes<kColK, kRowK>(a.s, size_t(blockIdx.x - a.walk_groups) * 256 + threadIdx.x,
+  split_lanes<kColK, kRowK, kRagged>(a.s, size_t(blockIdx.x - a.walk_groups) * 256 + threadIdx.x,
                             size_t(gridDim.x - a.walk_groups) * 256);
 }
 
@@ -307,19 +321,23 @@ struct Bm2Args {
   uint64_t mask;
   sufhip_x_planes xp;  // optional digit planes of the (truncated) outputs, merged layout
   const int8_t* X;     // balanced form: LHS planes of D + A_0
+  int vM, vN;          // balanced form: extent of C and the outputs (M, N padded)
 };
 
 // Party p's finished 32 x 32 tile values (lane l: column l % 32, rows of
 // the accumulator layout) to out_p, and to the output digit planes.
+// kRagged: rows and columns past vM and vN are padding (no merge, no planes).
+template <bool kRagged = false>
 __device__ __forceinline__ void bm2_store(const Bm2Args& a, int p, int l, int m0, int n0, size_t b,
                                           const uint64_t (&v)[16]) {
-  const int M = a.M, N = a.N;
+  const int M = kRagged ? a.vM : a.M, N = kRagged ? a.vN : a.N;
   const int col = n0 + (l & 31);
   const size_t ob = b * size_t(M) * N;
   const size_t ld = size_t(a.batches) * N;  // merged row length
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
+    if (kRagged && (row >= M || col >= N)) continue;
     const size_t o = a.merge ? size_t(row) * ld + b * N + col : ob + size_t(row) * N + col;
     a.out[p][o] = v[r];
     if (a.xp.planes) put_x_digits(a.xp, size_t(M), o, p, v[r]);
@@ -330,10 +348,11 @@ __device__ __forceinline__ void bm2_store(const Bm2Args& a, int p, int l, int m0
 // wave p opens rows r in [8p, 8p + 8) and writes both parties' outputs.
 // eh: the gate's key headers, read before the kernel's first global store;
 // every table read is issued before the first output store.
+template <bool kRagged = false>
 __device__ __forceinline__ void bm2_trunc_rows(const Bm2Args& a, const EpiHdrs& eh, int p, int l,
                                                int m0, int n0, size_t b,
                                                const uint64_t (*both)[16][64]) {
-  const int M = a.M, N = a.N;
+  const int M = kRagged ? a.vM : a.M, N = kRagged ? a.vN : a.N;
   const int col = n0 + (l & 31);
   const size_t ob = b * size_t(M) * N;
   const size_t ld = size_t(a.batches) * N;
@@ -350,6 +369,7 @@ __device__ __forceinline__ void bm2_trunc_rows(const Bm2Args& a, const EpiHdrs& 
   }
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
+    if (kRagged && (m0 + 8 * ((8 * p + q) >> 2) + 4 * (l >> 5) + (q & 3) >= M || col >= N)) continue;
     const uint64_t y0 = trunc_table_out(eh.h[0], a.epi.f, open[q], w[q][0]);
     const uint64_t y1 = trunc_table_out(eh.h[1], a.epi.f, open[q], w[q][1]);
     a.epi.y[0][o[q]] = y0;
@@ -466,7 +486,7 @@ __global__ void __launch_bounds__(128 * kKWaves) beaver_mfma2_kernel(Bm2Args a) 
 // wave's 16 C_p words are loaded with the first operand pairs, so the tile
 // needs no memory round trip after the k-loop (four stages leave no
 // registers for them).
-template <int kStages, bool kPrefC>
+template <int kStages, bool kPrefC, bool kRagged>
 __global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
   __shared__ uint64_t both[2][16][64];
   const int l = threadIdx.x & 63;
@@ -485,12 +505,17 @@ __global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
   const int8_t* Re = a.E + rb0;
   const int8_t* Rb = (p == 0 ? a.B[0] : a.B[1]) + rb0;
   const int col = n0 + (l & 31);
-  const size_t ob = b * size_t(M) * N;
+  const int vM = kRagged ? a.vM : M, vN = kRagged ? a.vN : N;
+  const size_t ob = b * size_t(vM) * vN;
+  const auto c_word = [&](int r) -> uint64_t {
+    const int row = m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
+    if (kRagged && (row >= vM || col >= vN)) return 0;
+    return a.C[p][ob + size_t(row) * vN + col];
+  };
   uint64_t cpre[16];
   if constexpr (kPrefC) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      cpre[r] = a.C[p][ob + size_t(m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3)) * N + col];
+    for (int r = 0; r < 16; ++r) cpre[r] = c_word(r);
   }
   v16i acc[kDigitPlanes];
 #pragma unroll
@@ -538,17 +563,16 @@ __global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
     v[r] = 0;
 #pragma unroll
     for (int s = 0; s < kDigitPlanes; ++s) v[r] += uint64_t(int64_t(acc[s][r])) << (8 * s);
-    const int row = m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-    v[r] += kPrefC ? cpre[r] : a.C[p][ob + size_t(row) * N + col];
+    v[r] += kPrefC ? cpre[r] : c_word(r);
   }
   if (!a.epi.on) {
-    bm2_store(a, p, l, m0, n0, b, v);
+    bm2_store<kRagged>(a, p, l, m0, n0, b, v);
     return;
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) both[p][r][l] = v[r];
   __syncthreads();
-  bm2_trunc_rows(a, eh, p, l, m0, n0, b, both);
+  bm2_trunc_rows<kRagged>(a, eh, p, l, m0, n0, b, both);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -563,7 +587,8 @@ namespace {
 
 // Shape checks and lane count of split job j (sources already set).
 int split_job(SplitArgs& a, int j, int8_t* planes, int batches, int rows, int cols,
-              int k_is_col, int8_t* planes_a0, const uint64_t* a0, const char* what) {
+              int k_is_col, int8_t* planes_a0, const uint64_t* a0, int valid_rows, int valid_cols,
+              const char* what) {
   const bool shape = batches >= 1 && rows >= 32 && cols >= 32 && rows % 32 == 0 &&
                      cols % 32 == 0;
   if (!shape || !planes || !aligned16(planes) || !aligned16(planes_a0)) {
@@ -575,6 +600,15 @@ int split_job(SplitArgs& a, int j, int8_t* planes, int batches, int rows, int co
     set_error(std::string(what) + ": planes_a0 and a0 go together");
     return SUFHIP_ERR_INVALID;
   }
+  const bool whole = valid_rows == 0 && valid_cols == 0;
+  if (!whole && (valid_rows < 1 || valid_rows > rows || valid_cols < 1 || valid_cols > cols ||
+                 (a.view[j][0] | a.view[j][1] | a.view[j][2]))) {
+    set_error(std::string(what) +
+              ": valid_rows in [1, rows] and valid_cols in [1, cols], without a_stride");
+    return SUFHIP_ERR_INVALID;
+  }
+  a.vrows[j] = whole ? rows : valid_rows;
+  a.vcols[j] = whole ? cols : valid_cols;
   a.planes[j] = planes;
   a.planes_a0[j] = planes_a0;
   a.a0[j] = a0;
@@ -605,7 +639,7 @@ int open_split_args(const sufhip_kb_open_job* jobs, int count, SplitArgs& a, con
     a.sub[j][1] = jb.b[1];
     for (int t = 0; t < 3; ++t) a.view[j][t] = size_t(jb.a_stride[t]);
     if (int rc = split_job(a, j, jb.planes, jb.batches, jb.rows, jb.cols, jb.k_is_col,
-                           jb.planes_a0, jb.a0, what))
+                           jb.planes_a0, jb.a0, jb.valid_rows, jb.valid_cols, what))
       return rc;
   }
   return SUFHIP_OK;
@@ -674,13 +708,24 @@ bool plan_tiles(SplitWalkArgs& f, int count, int ck) {
   return true;
 }
 
+bool split_ragged(const SplitArgs& a) {
+  for (int j = 0; j < a.count; ++j)
+    if (a.vrows[j] != a.rows[j] || a.vcols[j] != a.cols[j]) return true;
+  return false;
+}
+
 template <bool kWalk>
 int launch_tiled(SplitWalkArgs& f, void* stream) {
   size_t g = (f.s.begin[f.s.count] + 255) / 256;
   if (g > 4096) g = 4096;
   const size_t wg = kWalk ? f.walk_groups : 0;
-  hipLaunchKernelGGL((kb_split_tiled_kernel<kWalk>), dim3(unsigned(wg + f.tile_groups + g)),
-                     dim3(256), 0, as_stream(stream), f);
+  const dim3 grid(unsigned(wg + f.tile_groups + g));
+  if (split_ragged(f.s))
+    hipLaunchKernelGGL((kb_split_tiled_kernel<kWalk, true>), grid, dim3(256), 0,
+                       as_stream(stream), f);
+  else
+    hipLaunchKernelGGL((kb_split_tiled_kernel<kWalk, false>), grid, dim3(256), 0,
+                       as_stream(stream), f);
   return check_launch("kb_split_tiled_kernel");
 }
 
@@ -690,15 +735,21 @@ int launch_split(SplitArgs& a, int count, void* stream) {
   if (a.begin[count] == 0) return SUFHIP_OK;
   size_t g = (a.begin[count] + 255) / 256;
   if (g > 4096) g = 4096;
-  if (ck == 16)
-    hipLaunchKernelGGL((kb_split_kernel<16, 4>), dim3(unsigned(g)), dim3(256), 0,
-                       as_stream(stream), a);
+  const dim3 grid{unsigned(g)}, block(256);
+  const hipStream_t st = as_stream(stream);
+  const bool ragged = split_ragged(a);
+  if (ck == 16 && ragged)
+    hipLaunchKernelGGL((kb_split_kernel<16, 4, true>), grid, block, 0, st, a);
+  else if (ck == 16)
+    hipLaunchKernelGGL((kb_split_kernel<16, 4, false>), grid, block, 0, st, a);
+  else if (ck == 4 && ragged)
+    hipLaunchKernelGGL((kb_split_kernel<4, 4, true>), grid, block, 0, st, a);
   else if (ck == 4)
-    hipLaunchKernelGGL((kb_split_kernel<4, 4>), dim3(unsigned(g)), dim3(256), 0,
-                       as_stream(stream), a);
+    hipLaunchKernelGGL((kb_split_kernel<4, 4, false>), grid, block, 0, st, a);
+  else if (ragged)
+    hipLaunchKernelGGL((kb_split_kernel<1, 1, true>), grid, block, 0, st, a);
   else
-    hipLaunchKernelGGL((kb_split_kernel<1, 1>), dim3(unsigned(g)), dim3(256), 0,
-                       as_stream(stream), a);
+    hipLaunchKernelGGL((kb_split_kernel<1, 1, false>), grid, block, 0, st, a);
   return check_launch("kb_split_kernel");
 }
 
@@ -713,13 +764,21 @@ int launch_split_walk(SplitWalkArgs& f, int count, void* stream) {
   size_t g = (f.s.begin[count] + 255) / 256;
   if (g > 4096) g = 4096;
   if (wg + g == 0) return SUFHIP_OK;
-  const dim3 grid(unsigned(wg + (g > 0 ? g : 0)));
-  if (ck == 16)
-    hipLaunchKernelGGL((kb_split_walk_kernel<16, 4>), grid, dim3(256), 0, as_stream(stream), f);
+  const dim3 grid(unsigned(wg + (g > 0 ? g : 0))), block(256);
+  const hipStream_t st = as_stream(stream);
+  const bool ragged = split_ragged(f.s);
+  if (ck == 16 && ragged)
+    hipLaunchKernelGGL((kb_split_walk_kernel<16, 4, true>), grid, block, 0, st, f);
+  else if (ck == 16)
+    hipLaunchKernelGGL((kb_split_walk_kernel<16, 4, false>), grid, block, 0, st, f);
+  else if (ck == 4 && ragged)
+    hipLaunchKernelGGL((kb_split_walk_kernel<4, 4, true>), grid, block, 0, st, f);
   else if (ck == 4)
-    hipLaunchKernelGGL((kb_split_walk_kernel<4, 4>), grid, dim3(256), 0, as_stream(stream), f);
+    hipLaunchKernelGGL((kb_split_walk_kernel<4, 4, false>), grid, block, 0, st, f);
+  else if (ragged)
+    hipLaunchKernelGGL((kb_split_walk_kernel<1, 1, true>), grid, block, 0, st, f);
   else
-    hipLaunchKernelGGL((kb_split_walk_kernel<1, 1>), grid, dim3(256), 0, as_stream(stream), f);
+    hipLaunchKernelGGL((kb_split_walk_kernel<1, 1, false>), grid, block, 0, st, f);
   return check_launch("kb_split_walk_kernel");
 }
 
@@ -742,7 +801,8 @@ int sufhip_kb_split_batch(const sufhip_kb_split_job* jobs, int count, void* stre
     SUFHIP_REQUIRE(jb.src, "sufhip_kb_split_batch: null source");
     a.src[j] = jb.src;
     if (int rc = split_job(a, j, jb.planes, jb.batches, jb.rows, jb.cols, jb.k_is_col,
-                           jb.planes_a0, jb.a0, "sufhip_kb_split_batch"))
+                           jb.planes_a0, jb.a0, jb.valid_rows, jb.valid_cols,
+                           "sufhip_kb_split_batch"))
       return rc;
   }
   return launch_split(a, count, stream);
@@ -787,10 +847,15 @@ int sufhip_beaver_matmul2_mfma_ex(const sufhip_beaver_mfma2_args* args, void* st
   SUFHIP_REQUIRE(aligned16(g.Dp) && aligned16(g.Ep) && aligned16(g.Ap[0]) &&
                      aligned16(g.Ap[1]) && aligned16(g.Bp[0]) && aligned16(g.Bp[1]),
                  "sufhip_beaver_matmul2_mfma_ex: planes must be 16-byte aligned");
-  const size_t n = size_t(g.batches) * g.M * g.N;
+  const bool ragged = g.valid_m != 0 || g.valid_n != 0;
+  SUFHIP_REQUIRE(!ragged || (g.valid_m >= 1 && g.valid_m <= g.M && g.valid_n >= 1 &&
+                             g.valid_n <= g.N && g.Xp && !g.merge_heads && !g.out_planes.planes),
+                 "sufhip_beaver_matmul2_mfma_ex: valid_m in [1, M] and valid_n in [1, N], with Xp "
+                 "and neither merge_heads nor out_planes");
+  const size_t n = size_t(g.batches) * (ragged ? g.valid_m : g.M) * (ragged ? g.valid_n : g.N);
   Bm2Args a{g.Dp, g.Ep, {g.Ap[0], g.Ap[1]}, {g.Bp[0], g.Bp[1]}, {g.C[0], g.C[1]},
             {g.out[0], g.out[1]}, g.batches, g.M, g.K, g.N, g.merge_heads ? 1 : 0, TruncEpi{},
-            g.mask, g.out_planes, g.Xp};
+            g.mask, g.out_planes, g.Xp, ragged ? g.valid_m : g.M, ragged ? g.valid_n : g.N};
   if (int rc = make_epi(g.trunc, n, what, &a.epi)) return rc;
   SUFHIP_REQUIRE(a.epi.on || (g.out[0] && g.out[1]),
                  "sufhip_beaver_matmul2_mfma_ex: outputs (or a truncation) needed");
@@ -806,12 +871,20 @@ int sufhip_beaver_matmul2_mfma_ex(const sufhip_beaver_mfma2_args* args, void* st
   const uint64_t plane_set = uint64_t(kDigitPlanes) * uint64_t(g.batches) * uint64_t(g.K) *
                              uint64_t(g.M > g.N ? g.M : g.N);
   if (g.Xp && plane_set < (uint64_t(1) << 32)) {
-    if (g.K <= 128)  // at most 8 operand pairs
-      hipLaunchKernelGGL((beaver_bal_kernel<3, true>), grid, dim3(128), 0, as_stream(stream), a);
-    else
-      hipLaunchKernelGGL((beaver_bal_kernel<4, false>), grid, dim3(128), 0, as_stream(stream), a);
+    const hipStream_t st = as_stream(stream);
+    if (g.K <= 128) {  // at most 8 operand pairs
+      if (ragged)
+        hipLaunchKernelGGL((beaver_bal_kernel<3, true, true>), grid, dim3(128), 0, st, a);
+      else
+        hipLaunchKernelGGL((beaver_bal_kernel<3, true, false>), grid, dim3(128), 0, st, a);
+    } else if (ragged) {
+      hipLaunchKernelGGL((beaver_bal_kernel<4, false, true>), grid, dim3(128), 0, st, a);
+    } else {
+      hipLaunchKernelGGL((beaver_bal_kernel<4, false, false>), grid, dim3(128), 0, st, a);
+    }
     return check_launch("beaver_bal_kernel");
   }
+  SUFHIP_REQUIRE(!ragged, "sufhip_beaver_matmul2_mfma_ex: valid_m / valid_n with planes of 4 GiB");
   const int steps = g.K / 32;
   const int kws = steps < 2 ? 2 : (steps < kKWaves ? steps : kKWaves);
   hipLaunchKernelGGL(beaver_mfma2_kernel, grid, dim3(128 * kws), 0, as_stream(stream), a);

@@ -128,21 +128,32 @@ def kb_planes(batches, rows, cols, device="cuda"):
     return torch.empty(max(2, (nb + 15) // 8), dtype=torch.int64, device=device)
 
 
-def kb_split(jobs):
+def _extent(job, rows, cols, pad):
+    """A split job's plane extents: rows x cols, or with pad the next
+    multiples of 32, the planes' other rows and columns zero."""
+    job.rows, job.cols = rows, cols
+    if pad and (rows % 32 or cols % 32):
+        job.rows, job.cols = (-(-v // 32) * 32 for v in (rows, cols))
+        job.valid_rows, job.valid_cols = rows, cols
+
+
+def kb_split(jobs, pad=False):
     """Digit planes of up to 8 operands in one launch: jobs of (src, planes,
     batches, rows, cols, k_is_col[, planes_a0, a0]); with the last two also
-    the planes of src + a0."""
+    the planes of src + a0.  pad: rows and cols may be any, in planes of the
+    next multiples of 32, padded with zeros."""
     arr = (native.KbSplitJob * len(jobs))()
     for i, jb in enumerate(jobs):
         src, planes, b, r, c, kc = jb[:6]
         arr[i].src, arr[i].planes = ptr(src), ptr(planes)
-        arr[i].batches, arr[i].rows, arr[i].cols, arr[i].k_is_col = b, r, c, int(kc)
+        arr[i].batches, arr[i].k_is_col = b, int(kc)
+        _extent(arr[i], r, c, pad)
         if len(jb) > 6:
             arr[i].planes_a0, arr[i].a0 = ptr(jb[6]), ptr(jb[7])
     native.call("sufhip_kb_split_batch", arr, len(jobs), stream_ptr())
 
 
-def kb_open_split(jobs, prepare=None):
+def kb_open_split(jobs, prepare=None, pad=False):
     """Masked opens written straight as digit planes, up to 8 in one launch:
     jobs of (a, b, planes, batches, rows, cols, k_is_col[, planes_a0, a0[,
     view]]) with a and b pairs of share arrays (b may be None); element i is
@@ -151,7 +162,8 @@ def kb_open_split(jobs, prepare=None):
     element (batch, row, col) of a[p] is a[p][offset + strides . index].
     prepare: optional truncation gates (tasks.Trunc, one PRG state) whose
     key-only halves run in the same launch when they fit beside the split
-    (sufhip_kb_open_split_prepare), else in their own launches first."""
+    (sufhip_kb_open_split_prepare), else in their own launches first.  pad: as
+    in kb_split (jobs without a view)."""
     arr = (native.KbOpenJob * len(jobs))()
     for i, jb in enumerate(jobs):
         a, b, planes, nb, r, c, kc = jb[:7]
@@ -166,7 +178,8 @@ def kb_open_split(jobs, prepare=None):
         if b is not None:
             arr[i].b[0], arr[i].b[1] = ptr(b[0]), ptr(b[1])
         arr[i].planes = ptr(planes)
-        arr[i].batches, arr[i].rows, arr[i].cols, arr[i].k_is_col = nb, r, c, int(kc)
+        arr[i].batches, arr[i].k_is_col = nb, int(kc)
+        _extent(arr[i], r, c, pad)
         if len(jb) > 7 and jb[7] is not None:
             arr[i].planes_a0, arr[i].a0 = ptr(jb[7]), ptr(jb[8])
         if len(jb) > 9 and jb[9] is not None:

@@ -81,8 +81,11 @@ class BeaverMatmulTrunc:
         # the truncation folded in, the triple shares' digit planes made here.
         # The launch-per-step form's buffers (u64 opens, products, masked open,
         # truncation workspaces) exist only when it is the form in use.
-        self.fused = (use_mfma and M % 32 == 0 and K % 32 == 0 and N % 32 == 0 and K <= 4096 and
-                      frac_bits <= 13)
+        # Extents that are no multiple of 32 are padded with zero digits.
+        Mp, Kp, Np = (-(-v // 32) * 32 for v in (M, K, N))
+        whole = (Mp, Kp, Np) == (M, K, N)
+        self.fused = (use_mfma and Kp <= 4096 and frac_bits <= 13 and min(M, K, N) > 0 and
+                      (whole or 8 * Kp * max(Mp, Np) < 1 << 32))
         self.mm_work = None
         if not self.fused:
             self.work_bytes = lib.sufhip_trunc_work_bytes(frac_bits, M * N)
@@ -99,12 +102,13 @@ class BeaverMatmulTrunc:
         else:
             from . import layer, tasks
             self.tr = tasks.Trunc(None, frac_bits, M * N, self.prg_state, rnd=rnd)
-            self.Ap = tuple(layer.kb_planes(1, M, K) for _ in range(2))
-            self.Bp = tuple(layer.kb_planes(1, K, N) for _ in range(2))
-            self.Dp, self.Ep = layer.kb_planes(1, M, K), layer.kb_planes(1, K, N)
-            self.Xp = layer.kb_planes(1, M, K)  # D + A_0, party 0's left operand with E
+            self.padded = (Mp, Kp, Np)
+            self.Ap = tuple(layer.kb_planes(1, Mp, Kp) for _ in range(2))
+            self.Bp = tuple(layer.kb_planes(1, Kp, Np) for _ in range(2))
+            self.Dp, self.Ep = layer.kb_planes(1, Mp, Kp), layer.kb_planes(1, Kp, Np)
+            self.Xp = layer.kb_planes(1, Mp, Kp)  # D + A_0, party 0's left operand with E
             layer.kb_split([(self.A[p], self.Ap[p], 1, M, K, 1) for p in (0, 1)] +
-                           [(self.B[p], self.Bp[p], 1, K, N, 0) for p in (0, 1)])
+                           [(self.B[p], self.Bp[p], 1, K, N, 0) for p in (0, 1)], pad=True)
 
     def eval2(self, X, W, out, events=None):
         """X, W, out: pairs of device int64 tensors (party shares).  events:
@@ -158,7 +162,10 @@ class BeaverMatmulTrunc:
         a.Dp, a.Ep, a.Xp = _p(self.Dp), _p(self.Ep), _p(self.Xp)
         for p in (0, 1):
             a.Ap[p], a.Bp[p], a.C[p] = _p(self.Ap[p]), _p(self.Bp[p]), _p(self.C[p])
-        a.batches, a.M, a.K, a.N = 1, M, K, N
+        a.batches = 1
+        a.M, a.K, a.N = self.padded
+        if self.padded != (M, K, N):
+            a.valid_m, a.valid_n = M, N
         epi = self.tr.epilogue(out)
         a.trunc = native.ctypes.pointer(epi)
         a.mask = self.tr.mask & M64
@@ -166,7 +173,7 @@ class BeaverMatmulTrunc:
             events[0].record()
         # The truncation's key-only walks run in the opens' launch.
         layer.kb_open_split([(X, self.A, self.Dp, 1, M, K, 1, self.Xp, self.A[0]),
-                             (W, self.B, self.Ep, 1, K, N, 0)], prepare=[self.tr])
+                             (W, self.B, self.Ep, 1, K, N, 0)], prepare=[self.tr], pad=True)
         if events and len(events) > 2:
             events[1].record()
         native.call("sufhip_beaver_matmul2_mfma_ex", native.ctypes.byref(a), _stream())

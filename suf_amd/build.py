@@ -41,14 +41,7 @@ HIPCC_FLAGS = [
 
 # Kernels allowed a private segment, with the reason.  Every other kernel
 # must report ScratchSize 0, or the build fails.
-SCRATCH_ALLOWED = {
-    # SGPR spill slots only: the block's ~100 uniform pointers exceed the
-    # SGPR file, and the compiler keeps the overflow in VGPR lanes
-    # (v_writelane / v_readlane).  The frame size is reported, but the kernel
-    # has no scratch memory instruction (tests/test_build_scratch.py).
-    "softmax2_kernel": "SGPR spill slots in VGPR lanes, no scratch memory access",
-    "softmax2_team_kernel": "SGPR spill slots in VGPR lanes, no scratch memory access",
-}
+SCRATCH_ALLOWED = {}
 RESOURCE_REPORT = os.path.join(LIBDIR, "kernel_resources.txt")
 
 

@@ -9,7 +9,7 @@
 //
 //   layernorm2_kernel  LayerNormTask (include/runtime/phase_tasks.hpp:
 //                      2186-2668) with RsqrtTask (:1383-1700)
-//   softmax2_kernel    SoftmaxBlockTask (include/nn/softmax_block_task.hpp:
+//   softmax2_team_kernel    SoftmaxBlockTask (include/nn/softmax_block_task.hpp:
 //                      97-450) with RowMaxDiffTask, nExp, row sum, Recip
 #include <hip/hip_runtime.h>
 
@@ -271,21 +271,22 @@ __global__ void __launch_bounds__(kBlock) layernorm2_kernel(LnArgs A) {
   }
 }
 
-// Softmax rows: one wavefront per row, groups of `waves` rows per workgroup.
-// The row's scores go to registers and to level 0 of the max tree in LDS;
-// after the tree every step is wave-local (the row sum is a wave reduction,
-// the reciprocal runs on lane 0 and is broadcast by a lane shuffle).
+// Softmax rows: up to kSmSlots rows per workgroup of 768 lanes, every phase
+// flat over the workgroup: a max-tree level's pairs, the scores' nExp chains
+// and the normalisation are dealt to the lanes whatever row they belong to.
+// What bounds a row is its chain of dependent steps (7 to 9 tree levels, two
+// LUT chains), so a workgroup's rows go through it together: with rows of
+// very different lengths (causal attention) a wave or two per row leaves most
+// lanes idle, and a long row's levels run in turn on its own wave.
+//   12 x 128 causal rows: 53 us (60 with two waves per row);
+//   4 x 300 causal rows: 75 us (166 with one wave per row).
 constexpr int kSmRounds = 10;
 constexpr int kSmMaxRow = 512;
-// Six rows per workgroup, one workgroup per CU: the 64 KB two-table AES
-// span, the staged keys and six rows of up to 512 elements fit the CU's
-// 160 KB of LDS, and the config's 1536 rows are one workgroup on each of
-// 256 CUs.
-constexpr int kSmWaves = 6;
-constexpr int kSmThreads = 64 * kSmWaves;
+constexpr int kSmSlots = 8;
+constexpr int kSmThreads = 768;
+constexpr int kSmPer = 4;  // scores per lane: 6 rows of 512 or 8 of 384
 using SmAes = AesLds2<32>;
 constexpr size_t kSmLdsCap = 160 * 1024;
-constexpr int kSmLock = 2;  // nExp chains per lane evaluated in lockstep
 
 struct SmArgs {
   sufhip_operand2 x;
@@ -295,7 +296,7 @@ struct SmArgs {
   const int32_t* offs;
   const int32_t* round_off;
   TreeKeys<kSmRounds> keys;
-  int rows, max_row, waves;
+  int rows, max_row, slots, groups;
   ChainArgs nexp, recip;
   sufhip_triple2 norm;
   TruncEpi tr_norm;
@@ -312,15 +313,17 @@ struct SmStatic {
   TreeLds<kSmRounds> t;
   ChainLds nexp, recip;
   TruncHdr thn[3][2], thr[3][2];  // the chains' truncation key headers
-  ChainPreN<3> rpre[kSmWaves];  // each row's reciprocal triples
-  uint32_t j0[kSmWaves][kSmRounds];  // each row's tree slot offsets
+  ChainPreN<3> rpre[kSmSlots];  // each row's reciprocal triples
+  uint32_t j0[kSmSlots][kSmRounds];  // each row's tree slot offsets
+  // The group's rows: global row (-1: none), first score, length, levels of
+  // the max tree, and where the row's scores (even levels) and odd levels
+  // start in the level buffers.
+  int row[kSmSlots], first[kSmSlots], len[kSmSlots], levels[kSmSlots];
+  int even0[kSmSlots + 1], odd0[kSmSlots];
+  int pairs0[kSmRounds][kSmSlots + 1];  // first pair of each row in a level
+  uint64_t sum[kSmSlots][2];   // row sums of e
+  uint64_t inv[kSmSlots][2];   // their reciprocals
 };
-
-__device__ __forceinline__ uint64_t bcast_lane0(uint64_t v) {
-  const uint32_t lo = __shfl(uint32_t(v), 0, 64);
-  const uint32_t hi = __shfl(uint32_t(v >> 32), 0, 64);
-  return uint64_t(lo) | uint64_t(hi) << 32;
-}
 
 // Everything the block keeps in LDS for the whole launch -- the AES span,
 // every tree round's keys, both chains' keys -- in one staging pass: a
@@ -331,7 +334,7 @@ __device__ __forceinline__ uint64_t bcast_lane0(uint64_t v) {
 // loads go in between; the caller syncs after store().
 template <int kThreads>
 struct SmStagerT {
-  static constexpr int kChainPer = (3 * kSmThreads + kThreads - 1) / kThreads;
+  static constexpr int kChainPer = 2;
   typename SmAes::template Filler<kThreads> tf;
   TreeStager<kSmRounds, 2> ts;
   TruncHdrStager<3> hn, hr;
@@ -386,323 +389,237 @@ struct SmStagerT {
     }
   }
 };
-using SmStager = SmStagerT<kSmThreads>;
+// The kernel's argument read afresh from the kernarg segment: an opaque copy
+// of its address per phase, so that a phase's pointers are scalar loads where
+// they are used.  The block's ~100 uniform pointers exceed the scalar
+// registers, and held over the whole kernel they are moved to vector lanes
+// and back.
+__device__ __forceinline__ const SmArgs& sm_args() {
+  typedef const __attribute__((address_space(4))) SmArgs* Ptr;
+  Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const SmArgs*)p;
+}
+
+// kN values of a lane in registers, indexed by a (uniform) loop variable.
+// (One or two are named members: the compiler puts a short indexed vector or
+// array in private memory.)
+template <int kN>
+struct LaneVals {
+  typedef uint64_t Vec __attribute__((ext_vector_type(kN)));
+  Vec v = 0;
+  __device__ __forceinline__ uint64_t get(int k) const { return v[k]; }
+  __device__ __forceinline__ void set(int k, uint64_t x) { v[k] = x; }
+};
+template <>
+struct LaneVals<1> {
+  uint64_t a = 0;
+  __device__ __forceinline__ uint64_t get(int) const { return a; }
+  __device__ __forceinline__ void set(int, uint64_t x) { a = x; }
+};
+template <>
+struct LaneVals<2> {
+  uint64_t a = 0, b = 0;
+  __device__ __forceinline__ uint64_t get(int k) const { return k ? b : a; }
+  __device__ __forceinline__ void set(int k, uint64_t x) {
+    a = k ? a : x;
+    b = k ? x : b;
+  }
+};
+
+// The slot whose range [start[s], start[s + 1]) holds x (the last one whose
+// start is at most x; empty slots share their start with the next).
+__device__ __forceinline__ int sm_slot(const int* start, int x) {
+  int s = 0;
+#pragma unroll
+  for (int k = 1; k < kSmSlots; ++k) s += x >= start[k] ? 1 : 0;
+  return s;
+}
+
+// Pairs p0 + Q + 192 u (Q the lane's quad, u < U) of level k over the
+// workgroup's rows: tree_chunk's step with each pair's row looked up.  The
+// AES block of a pair is spread over its quad; lane q then finishes the
+// quad's pair u = q.
+template <int U>
+__device__ __forceinline__ void tree_flat(const SmArgs& a, const SmStatic& st, const SmAes& aes,
+                                          int k, const uint64_t* src, int sw, const int* src0,
+                                          uint64_t* dst, int dw, const int* dst0, int p0,
+                                          int pairs, bool one_ks) {
+  constexpr int kQuads = kSmThreads / 4;
+  const TreeLds<kSmRounds>& L = st.t;
+  const int Q = int(threadIdx.x >> 2), q = int(threadIdx.x & 3);
+  uint64_t xh[U], xb[U][2];
+  int iv[U][2], at[U];
+  uint32_t blk[2][U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int p = p0 + Q + kQuads * u < pairs ? p0 + Q + kQuads * u : pairs - 1;
+    const int r = sm_slot(st.pairs0[k], p);
+    const int t = p - st.pairs0[k][r];
+    const uint64_t* s = src + src0[r] + 2 * t;
+    at[u] = dst0[r] + t;
+    const uint64_t xa0 = s[0], xb0 = s[1], xa1 = s[sw], xb1 = s[sw + 1];
+    xh[u] = (xa0 - xb0) + (xa1 - xb1) + a.keys.mask[k];
+    xb[u][0] = xb0;
+    xb[u][1] = xb1;
+    const uint32_t j = st.j0[r][k] + uint32_t(t);
+#pragma unroll
+    for (int p2 = 0; p2 < 2; ++p2) {
+      iv[u][p2] = (p2 == 1 && one_ks) ? iv[u][0] : tree_interval(a.keys, L, k, p2, xh[u]);
+      const uint64_t ctr = L.nonce[k][p2] ^ (uint64_t(j) << 32) ^ (uint64_t(iv[u][p2]) * 2);
+      blk[p2][u] = q == 0 ? uint32_t(ctr) : (q == 1 ? uint32_t(ctr >> 32) : 0u);
+    }
+  }
+  tree_keystream<U>(aes, L, k, q, one_ks, blk);
+  // Lane q takes block q: column c of it is lane c's word of blk[.][q].
+  uint32_t w[2][4];
+  uint64_t x = 0, b[2] = {0, 0};
+  int ivq[2] = {0, 0}, o0 = 0;
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) w[p][c] = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    uint32_t c[2][4];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const uint32_t v = blk[p][u];
+      c[p][0] = quad_bcast<0>(v);
+      c[p][1] = quad_bcast<1>(v);
+      c[p][2] = quad_bcast<2>(v);
+      c[p][3] = quad_bcast<3>(v);
+    }
+    if (q == u) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[p][j] = c[p][j];
+        b[p] = xb[u][p];
+        ivq[p] = iv[u][p];
+      }
+      x = xh[u];
+      o0 = at[u];
+    }
+  }
+  if (q < U && p0 + Q + kQuads * q < pairs) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const uint64_t k0 = uint64_t(w[p][0]) | uint64_t(w[p][1]) << 32;
+      const uint64_t k1 = uint64_t(w[p][2]) | uint64_t(w[p][3]) << 32;
+      const bool zero = L.party[k][p] == 0;
+      const uint64_t q0 = zero ? k0 : L.pay[k][p][2 * ivq[p]] - k0;
+      const uint64_t q1 = zero ? k1 : L.pay[k][p][2 * ivq[p] + 1] - k1;
+      dst[(p ? dw : 0) + o0] = b[p] + q0 + q1 * x;
+    }
+  }
+}
 
 template <int kPer>
-__global__ void __launch_bounds__(kSmThreads) softmax2_kernel(SmArgs a) {
+__global__ void __launch_bounds__(kSmThreads) softmax2_team_kernel(SmArgs) {
+  const SmArgs& a = sm_args();
   __shared__ __align__(16) SmStatic st;
   extern __shared__ uint64_t rowbuf[];
-  const int mr = a.max_row;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint64_t* even = rowbuf + size_t(wave) * tree_row_words(mr);
-  uint64_t* odd = even + 2 * size_t(mr);
-  constexpr bool kPre = kPer <= 2;
-  int b = 0, len = 0;
-  uint64_t na[kPre ? kPer : 1][2], nc[kPre ? kPer : 1][2];
-  uint64_t s[kPer][2];
-  // Group g's row loads: offsets, the loads that need no open (issued now
-  // to land while the tree runs: the reciprocal's triples, one word per
-  // lane, to LDS, and for short rows every element's normalisation triple),
-  // and the scores through the optional truncations of their open, into
-  // registers and level 0 of the tree.  They touch no staged LDS, so for
-  // rows of up to 128 elements the first group's run before the staging and
-  // overlap its loads (longer rows keep too many scores in registers).
-  auto load_rows = [&](int g) {
-    const int r = g * a.waves + wave;
-    b = 0;
-    len = 0;
-    if (r < a.rows) {
-      b = a.offs[r];
-      len = a.offs[r + 1] - b;
-      if (len < 1 || len > mr) len = 0;  // refused on the host
-    }
-    if (len > 0 && lane < 18) st.rpre[wave].word(lane) = chain_triple_word(a.recip, lane, size_t(r));
-    tree_row_offsets(a.keys, a.round_off, a.rows, r, len, st.j0[wave]);
-    if constexpr (kPre) {
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        const int j = lane + 64 * k;
-        const size_t i = size_t(b) + size_t(j < len ? j : 0);
-        na[k][0] = j < len ? a.norm.a[0][i] : 0;
-        na[k][1] = j < len ? a.norm.a[1][i] : 0;
-        nc[k][0] = j < len ? a.norm.c[0][i] : 0;
-        nc[k][1] = j < len ? a.norm.c[1][i] : 0;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int j = lane + 64 * k;
-      s[k][0] = s[k][1] = 0;
-      if (j < len) {
-        const size_t i = size_t(b) + size_t(j);
-        uint64_t v0 = operand_at(a.x, 0, i), v1 = operand_at(a.x, 1, i);
-        // Compile-time gate indices: a runtime index into the by-value
-        // argument block would copy it to private scratch memory.
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          if (q >= a.pre) break;
-          const uint64_t o = v0 + v1 + a.pre_mask[q];
-          v0 = trunc_table_eval(a.pre_tr[q].key[0], a.pre_tr[q].table[0], a.pre_tr[q].f, o);
-          v1 = trunc_table_eval(a.pre_tr[q].key[1], a.pre_tr[q].table[1], a.pre_tr[q].f, o);
-        }
-        s[k][0] = v0;
-        s[k][1] = v1;
-        even[j] = v0;
-        even[mr + j] = v1;
-      }
-    }
+  const int mr = a.max_row, half = (mr + 1) / 2;
+  const int we = a.slots * mr, wo = a.slots * half;  // party strides of the level buffers
+  uint64_t* even = rowbuf;
+  uint64_t* odd = rowbuf + 2 * we;
+  const int tid = int(threadIdx.x), lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // This lane's scores, one in every 768 of the group's; the loops over them
+  // stay loops (unrolled, the chains' code outgrows the instruction cache).
+  LaneVals<kPer> s0, s1;
+  // Group g's rows: slot k takes row k G + g or, for odd k, (k + 1) G - 1 - g,
+  // which evens out the lengths of causal rows.  The offsets are uniform
+  // (scalar) loads; every lane then loads its scores -- through the optional
+  // truncations of their open -- into registers and level 0 of the tree, its
+  // first score's normalisation triple, and (one wave per row) the
+  // reciprocal's triples and the row's tree slots.  Before the first barrier
+  // nothing staged is read, so the first group's loads overlap the staging.
+  // Length of slot k's row r and its first score f (0: none).
+  auto row_len = [&](const SmArgs& a, int k, int r, int& f) {
+    if (k >= a.slots || r >= a.rows) return 0;
+    f = a.offs[r];
+    const int n = a.offs[r + 1] - f;
+    return n < 1 || n > mr ? 0 : n;  // refused on the host
   };
-  {
-    SmStager stager;
-    stager.load(a);
-    if constexpr (kPre) load_rows(blockIdx.x);
-    stager.store(a, st);
-  }
-  __syncthreads();
-  tree_compare(a.keys, st.t);
-  chain_compare(a.nexp, st.nexp);
-  chain_compare(a.recip, st.recip);
-  __syncthreads();
-  const SmAes aes = SmAes::make(st.tab);
-  const ChainKeyInfo Kn = chain_key_info(a.nexp, st.nexp);
-  const ChainKeyInfo Kr = chain_key_info(a.recip, st.recip);
-  const uint32_t shared = ~st.t.diff;
-  for (int g = blockIdx.x; g * a.waves < a.rows; g += gridDim.x) {
-    if (!kPre || g != int(blockIdx.x)) {
-      load_rows(g);
-      __syncthreads();
-    }
-    const int r = g * a.waves + wave;
-    const int level =
-        tree_row<kSmRounds, SmAes>(a.keys, st.t, aes, even, odd, mr, len, st.j0[wave], shared);
-    const uint64_t* fin = (level & 1) ? odd : even;
-    const int fw = (level & 1) ? (mr + 1) / 2 : mr;
-    const uint64_t m0 = len > 0 ? fin[0] : 0, m1 = len > 0 ? fin[fw] : 0;
-    // e = nExp(max - s), summed over the row; the lane's elements kSmLock at
-    // a time, their chains in lockstep (elements past the row end compute on
-    // clamped indices and are dropped).
-    uint64_t e[kPer][2];
-    uint64_t es0 = 0, es1 = 0;
-#pragma unroll
-    for (int k0 = 0; k0 < kPer; k0 += kSmLock) {
-      size_t ii[kSmLock];
-      Two dl[kSmLock], ev[kSmLock];
-      plain_loader<SUFHIP_CHAIN_CUBIC> pl[kSmLock] = {};
-#pragma unroll
-      for (int u = 0; u < kSmLock; ++u) {
-        const int j = lane + 64 * (k0 + u);
-        ii[u] = size_t(b) + size_t(j < len ? j : 0);
-        dl[u] = Two{{m0 - s[k0 + u][0], m1 - s[k0 + u][1]}};
-        pl[u] = plain_loader<SUFHIP_CHAIN_CUBIC>{&a.nexp, ii[u]};
-      }
-      chain_eval_m<SUFHIP_CHAIN_CUBIC, SmAes, kSmLock>(a.nexp, st.nexp, Kn, aes, ii, dl, pl,
-                                                        ev, st.thn);
-#pragma unroll
-      for (int u = 0; u < kSmLock; ++u) {
-        const bool ok = lane + 64 * (k0 + u) < len;
-        e[k0 + u][0] = ok ? ev[u].v[0] : 0;
-        e[k0 + u][1] = ok ? ev[u].v[1] : 0;
-        es0 += e[k0 + u][0];
-        es1 += e[k0 + u][1];
-      }
-    }
-    es0 = wave_sum_u64(es0);
-    es1 = wave_sum_u64(es1);
-    // inv = Recip(row sum) on the whole wave (its keystream blocks
-    // column-parallel on eight lanes, every lane ends with the result).
-    uint64_t inv0 = 0, inv1 = 0;
-    if (len > 0) {
-      const Two iv = chain_eval_quad<SUFHIP_CHAIN_RECIP, SmAes, ChainPreN<3>>(
-          a.recip, st.recip, Kr, aes, size_t(r), Two{{es0, es1}}, st.rpre[wave], st.thr);
-      inv0 = iv.v[0];
-      inv1 = iv.v[1];
-    }
-    // prob = tr_norm(e * inv[row]) (row-broadcast Beaver), and the next
-    // product's open over the dense row.
-    if (len > 0) {
-      const uint64_t nb0 = a.norm.b[0][r], nb1 = a.norm.b[1][r];
-      const uint64_t ee = (inv0 - nb0) + (inv1 - nb1);
-      const size_t drow = size_t(r) * size_t(a.dense_cols);
-#pragma unroll
-      for (int k = 0; k < kPer; ++k) {
-        const int j = lane + 64 * k;
-        if (j < len) {
-          const size_t i = size_t(b) + size_t(j);
-          uint64_t a0, a1, c0, c1;
-          if constexpr (kPre) {
-            a0 = na[k][0];
-            a1 = na[k][1];
-            c0 = nc[k][0];
-            c1 = nc[k][1];
-          } else {
-            a0 = a.norm.a[0][i];
-            a1 = a.norm.a[1][i];
-            c0 = a.norm.c[0][i];
-            c1 = a.norm.c[1][i];
-          }
-          const uint64_t dd = (e[k][0] - a0) + (e[k][1] - a1);
-          const uint64_t z0 = c0 + dd * nb0 + ee * a0 + dd * ee;
-          const uint64_t z1 = c1 + dd * nb1 + ee * a1;
-          const uint64_t o = z0 + z1 + a.norm_mask;
-          const uint64_t p0 =
-              trunc_table_eval(a.tr_norm.key[0], a.tr_norm.table[0], a.tr_norm.f, o);
-          const uint64_t p1 =
-              trunc_table_eval(a.tr_norm.key[1], a.tr_norm.table[1], a.tr_norm.f, o);
-          if (a.out[0]) {
-            a.out[0][i] = p0;
-            a.out[1][i] = p1;
-          }
-          if (a.dense) {
-            const size_t di = drow + size_t(j);
-            const uint64_t dv = (p0 - a.dense_a[0][di]) + (p1 - a.dense_a[1][di]);
-            a.dense[di] = dv;
-            if (a.dkb.planes) put_kb_digits(a.dkb, di, dv);
-          }
-        }
-      }
-      if (a.dense)
-        for (int j = len + lane; j < a.dense_cols; j += 64) {
-          const size_t di = drow + size_t(j);
-          const uint64_t dv = (uint64_t(0) - a.dense_a[0][di]) + (uint64_t(0) - a.dense_a[1][di]);
-          a.dense[di] = dv;
-          if (a.dkb.planes) put_kb_digits(a.dkb, di, dv);
-        }
-    }
-    __syncthreads();  // the row buffers are rewritten by the next group
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Rows of up to 128 elements on a team of two waves: six rows per
-// workgroup of 768 lanes (twelve waves, three per SIMD; the LDS is the
-// six-row kernel's).  Wave t of a row's team holds element lane + 64 t.
-// The max tree's first two levels (up to 64 and 32 pairs) are split between
-// the team's waves, with a workgroup barrier after each; the shorter levels
-// run on the team's first wave.  Each lane then runs one element's nExp
-// chain with both parties' keystream blocks in one lockstep group, the
-// row sum adds the two waves' partial sums through LDS, the reciprocal runs
-// on the first wave's lane 0, and each wave normalises its elements.  The
-// per-wave work of the tree's wide levels, of the nExp chain and of the
-// normalisation halves; every output equals the one-wave-per-row kernel's.
-constexpr int kSmTeam = 2;
-constexpr int kSmTeamThreads = 64 * kSmWaves * kSmTeam;
-constexpr int kSmTeamMaxRow = 128;
-
-// Levels 0 and 1 split over the team (pairs [32 t, 32 t + 32) and
-// [16 t, 16 t + 16)), a workgroup barrier after each; later levels on wave
-// t = 0 only (its wave-local ordering as in tree_row).  Every thread of the
-// workgroup runs the same number of barriers.  Returns the level count (the
-// same in both waves).
-template <class Aes>
-__device__ __forceinline__ int tree_row_team(const TreeKeys<kSmRounds>& K,
-                                             const TreeLds<kSmRounds>& L, const Aes& aes,
-                                             uint64_t* even, uint64_t* odd, int mr, int len,
-                                             const uint32_t* j0s, uint32_t shared, int tw) {
-  const int lane = threadIdx.x & 63, half = (mr + 1) / 2;
-  int level = 0;
-  for (int k = 0; k < K.rounds; ++k) {
-    const bool split = k < 2;
-    if (len > 1) {
-      const uint64_t* src = (level & 1) ? odd : even;
-      const int sw = (level & 1) ? half : mr;
-      uint64_t* dst = (level & 1) ? even : odd;
-      const int dw = (level & 1) ? mr : half;
-      const int pairs = len >> 1;
-      const uint32_t j0 = j0s[k];
-      const bool one_ks = (shared >> k) & 1u;
-      if (split) {
-        const int per = k == 0 ? 32 : 16;
-        const int t0 = per * tw;
-        const int nb = pairs - t0 < per ? pairs - t0 : per;
-        if (nb > 16)
-          tree_chunk<2>(K, L, aes, k, src, sw, dst, dw, j0, t0, nb, one_ks);
-        else if (nb > 0)
-          tree_chunk<1>(K, L, aes, k, src, sw, dst, dw, j0, t0, nb, one_ks);
-      } else if (tw == 0) {
-        for (int t0 = 0; t0 < pairs; t0 += 64) {
-          const int nb = pairs - t0 < 64 ? pairs - t0 : 64;
-          if (nb > 48)
-            tree_chunk<4>(K, L, aes, k, src, sw, dst, dw, j0, t0, nb, one_ks);
-          else if (nb > 32)
-            tree_chunk<3>(K, L, aes, k, src, sw, dst, dw, j0, t0, nb, one_ks);
-          else if (nb > 16)
-            tree_chunk<2>(K, L, aes, k, src, sw, dst, dw, j0, t0, nb, one_ks);
-          else
-            tree_chunk<1>(K, L, aes, k, src, sw, dst, dw, j0, t0, nb, one_ks);
-        }
-      }
-      if ((len & 1) && lane == 0 && tw == 0) {
-        dst[pairs] = src[2 * pairs];
-        dst[dw + pairs] = src[sw + 2 * pairs];
-      }
-      len = (len + 1) >> 1;
-      ++level;
-    }
-    if (split) {
-      __syncthreads();
-    } else if (tw == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-  }
-  return level;
-}
-
-__global__ void __launch_bounds__(kSmTeamThreads) softmax2_team_kernel(SmArgs a) {
-  __shared__ __align__(16) SmStatic st;
-  __shared__ uint64_t part[kSmWaves][kSmTeam][2];  // the team's partial row sums
-  __shared__ uint64_t invs[kSmWaves][2];           // the row's reciprocal shares
-  extern __shared__ uint64_t rowbuf[];
-  const int mr = a.max_row;
-  // Wave-uniform (a scalar register): the row offsets then load through the
-  // scalar cache and the team's branches are scalar branches.
-  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-  const int lane = threadIdx.x & 63;
-  const int slot = wave >> 1, tw = wave & 1;  // row slot in the group, wave in the team
-  const int j = lane + 64 * tw;               // this lane's element of the row
-  uint64_t* even = rowbuf + size_t(slot) * tree_row_words(mr);
-  uint64_t* odd = even + 2 * size_t(mr);
-  int b = 0, len = 0;
-  uint64_t na0 = 0, na1 = 0, nc0 = 0, nc1 = 0, s0 = 0, s1 = 0;
-  // The row group's loads, as in softmax2_kernel (one element per lane).
   auto load_rows = [&](int g) {
-    const int r = g * a.waves + slot;
-    b = 0;
-    len = 0;
-    if (r < a.rows) {
-      b = a.offs[r];
-      len = a.offs[r + 1] - b;
-      if (len < 1 || len > mr) len = 0;  // refused on the host
+    const SmArgs& a = sm_args();
+    const auto row_of = [&](int k) {
+      return (k & 1) ? (k + 1) * a.groups - 1 - g : k * a.groups + g;
+    };
+    int total = 0, ototal = 0;
+    int e0[kSmSlots], f0[kSmSlots], ln[kSmSlots];
+#pragma unroll
+    for (int k = 0; k < kSmSlots; ++k) {
+      const int r = row_of(k);
+      int f = 0;
+      const int n = row_len(a, k, r, f);
+      e0[k] = total;
+      f0[k] = f;
+      ln[k] = n;
+      if (tid == k) {
+        st.row[k] = n > 0 ? r : -1;
+        st.first[k] = f;
+        st.len[k] = n;
+        st.levels[k] = n > 1 ? 32 - __builtin_clz(uint32_t(n - 1)) : 0;
+        st.even0[k] = total;
+        st.odd0[k] = ototal;
+        st.sum[k][0] = st.sum[k][1] = 0;
+      }
+      total += n;
+      ototal += (n + 1) >> 1;
     }
-    if (tw == 0) {
-      if (len > 0 && lane < 18)
-        st.rpre[slot].word(lane) = chain_triple_word(a.recip, lane, size_t(r));
-      tree_row_offsets(a.keys, a.round_off, a.rows, r, len, st.j0[slot]);
+    if (tid == 0) st.even0[kSmSlots] = total;
+    if (wave < kSmSlots) {
+      const int r = row_of(wave);
+      int f = 0;
+      const int n = row_len(a, wave, r, f);
+      if (n > 0 && lane < 18)
+        st.rpre[wave].word(lane) = chain_triple_word(a.recip, lane, size_t(r));
+      tree_row_offsets(a.keys, a.round_off, a.rows, r, n, st.j0[wave]);
     }
-    const size_t i = size_t(b) + size_t(j < len ? j : 0);
-    na0 = j < len ? a.norm.a[0][i] : 0;
-    na1 = j < len ? a.norm.a[1][i] : 0;
-    nc0 = j < len ? a.norm.c[0][i] : 0;
-    nc1 = j < len ? a.norm.c[1][i] : 0;
-    s0 = s1 = 0;
-    if (j < len) {
+    // Lane k of the wave after the rows': level k's pairs.
+    if (wave == kSmSlots && lane < kSmRounds) {
+      int p = 0;
+#pragma unroll
+      for (int k = 0; k < kSmSlots; ++k) {
+        st.pairs0[lane][k] = p;
+        const int n = ln[k] > 0 ? ((ln[k] - 1) >> lane) + 1 : 0;  // the level's length
+        p += n >> 1;
+      }
+      st.pairs0[lane][kSmSlots] = p;
+    }
+#pragma unroll 1
+    for (int k = 0; k < kPer && kSmThreads * k < total; ++k) {
+      const int e = tid + kSmThreads * k;
+      if (e >= total) continue;
+      int base = 0, f = f0[0];
+#pragma unroll
+      for (int j = 1; j < kSmSlots; ++j)
+        if (e >= e0[j]) {
+          base = e0[j];
+          f = f0[j];
+        }
+      const size_t i = size_t(f) + size_t(e - base);
       uint64_t v0 = operand_at(a.x, 0, i), v1 = operand_at(a.x, 1, i);
+      // Compile-time gate indices: a runtime index into the argument block
+      // would copy it to private scratch memory.
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        if (q >= a.pre) break;
-        const uint64_t o = v0 + v1 + a.pre_mask[q];
-        v0 = trunc_table_eval(a.pre_tr[q].key[0], a.pre_tr[q].table[0], a.pre_tr[q].f, o);
-        v1 = trunc_table_eval(a.pre_tr[q].key[1], a.pre_tr[q].table[1], a.pre_tr[q].f, o);
+      for (int t = 0; t < 2; ++t) {
+        if (t >= a.pre) break;
+        const uint64_t o = v0 + v1 + a.pre_mask[t];
+        v0 = trunc_table_eval(a.pre_tr[t].key[0], a.pre_tr[t].table[0], a.pre_tr[t].f, o);
+        v1 = trunc_table_eval(a.pre_tr[t].key[1], a.pre_tr[t].table[1], a.pre_tr[t].f, o);
       }
-      s0 = v0;
-      s1 = v1;
-      even[j] = v0;
-      even[mr + j] = v1;
+      s0.set(k, v0);
+      s1.set(k, v1);
+      even[e] = v0;
+      even[we + e] = v1;
     }
   };
   {
-    SmStagerT<kSmTeamThreads> stager;
+    SmStagerT<kSmThreads> stager;
     stager.load(a);
     load_rows(blockIdx.x);
     stager.store(a, st);
@@ -716,78 +633,137 @@ __global__ void __launch_bounds__(kSmTeamThreads) softmax2_team_kernel(SmArgs a)
   const ChainKeyInfo Kn = chain_key_info(a.nexp, st.nexp);
   const ChainKeyInfo Kr = chain_key_info(a.recip, st.recip);
   const uint32_t shared = ~st.t.diff;
-  for (int g = blockIdx.x; g * a.waves < a.rows; g += gridDim.x) {
+  for (int g = blockIdx.x; g < a.groups; g += gridDim.x) {
     if (g != int(blockIdx.x)) {
       load_rows(g);
       __syncthreads();
     }
-    const int r = g * a.waves + slot;
-    const int level = tree_row_team<SmAes>(a.keys, st.t, aes, even, odd, mr, len, st.j0[slot],
-                                           shared, tw);
-    __syncthreads();  // the first wave's later levels, for the second wave
-    const uint64_t* fin = (level & 1) ? odd : even;
-    const int fw = (level & 1) ? (mr + 1) / 2 : mr;
-    const uint64_t m0 = len > 0 ? fin[0] : 0, m1 = len > 0 ? fin[fw] : 0;
-    // e = nExp(max - s) for this lane's element, both parties' keystream
-    // blocks in one lockstep group (elements past the row end compute on a
-    // clamped index and are dropped).
-    const bool ok = j < len;
-    const size_t ii = size_t(b) + size_t(ok ? j : 0);
-    const Two ev = chain_eval<SUFHIP_CHAIN_CUBIC, SmAes, plain_loader<SUFHIP_CHAIN_CUBIC>, true>(
-        a.nexp, st.nexp, Kn, aes, ii, Two{{m0 - s0, m1 - s1}},
-        plain_loader<SUFHIP_CHAIN_CUBIC>{&a.nexp, ii}, st.thn);
-    const uint64_t e0 = ok ? ev.v[0] : 0, e1 = ok ? ev.v[1] : 0;
-    const uint64_t ps0 = wave_sum_u64(e0), ps1 = wave_sum_u64(e1);
-    if (lane == 0) {
-      part[slot][tw][0] = ps0;
-      part[slot][tw][1] = ps1;
+    // The max tree, level by level over all rows.
+    for (int k = 0; k < a.keys.rounds; ++k) {
+      const SmArgs& a = sm_args();
+      const int pairs = __builtin_amdgcn_readfirstlane(st.pairs0[k][kSmSlots]);
+      if (pairs == 0) break;  // every row is down to one element
+      const uint64_t* src = (k & 1) ? odd : even;
+      uint64_t* dst = (k & 1) ? even : odd;
+      const int sw = (k & 1) ? wo : we, dw = (k & 1) ? we : wo;
+      const int* src0 = (k & 1) ? st.odd0 : st.even0;
+      const int* dst0 = (k & 1) ? st.even0 : st.odd0;
+      const bool one_ks = (shared >> k) & 1u;
+      for (int p0 = 0; p0 < pairs; p0 += kSmThreads / 2) {
+        const int left = pairs - p0;
+        if (left <= 16 * wave) break;  // no pair for this wave's quads
+        if (left > kSmThreads / 4)
+          tree_flat<2>(a, st, aes, k, src, sw, src0, dst, dw, dst0, p0, pairs, one_ks);
+        else
+          tree_flat<1>(a, st, aes, k, src, sw, src0, dst, dw, dst0, p0, pairs, one_ks);
+      }
+      // An odd level's last element passes through.
+      if (tid < kSmSlots && k < st.levels[tid]) {
+        const int n = ((st.len[tid] - 1) >> k) + 1;
+        if (n & 1) {
+          dst[dst0[tid] + (n >> 1)] = src[src0[tid] + n - 1];
+          dst[dw + dst0[tid] + (n >> 1)] = src[sw + src0[tid] + n - 1];
+        }
+      }
+      __syncthreads();
     }
+    // e = nExp(max - s) for the lane's scores, both parties' keystream blocks
+    // in one lockstep group, and the row sums: a wave adds its lanes of a row,
+    // then the waves meet in LDS.
+    const int total = __builtin_amdgcn_readfirstlane(st.even0[kSmSlots]);
+    LaneVals<kPer> ex0, ex1;
+#pragma unroll 1
+    for (int k = 0; k < kPer; ++k) {
+      const SmArgs& a = sm_args();
+      const int w0 = kSmThreads * k + 64 * wave;  // the wave's first score
+      if (w0 >= total) break;
+      const bool ok = w0 + lane < total;
+      const int x = ok ? w0 + lane : total - 1;  // past the end: dropped
+      const int q = sm_slot(st.even0, x);
+      const uint64_t* fin = (st.levels[q] & 1) ? odd + st.odd0[q] : even + st.even0[q];
+      const int fw = (st.levels[q] & 1) ? wo : we;
+      const size_t i = size_t(st.first[q]) + size_t(x - st.even0[q]);
+      const Two d{{fin[0] - s0.get(k), fin[fw] - s1.get(k)}};
+      const Two ev = chain_eval<SUFHIP_CHAIN_CUBIC, SmAes, plain_loader<SUFHIP_CHAIN_CUBIC>,
+                                kPer <= 2>(
+          a.nexp, st.nexp, Kn, aes, i, d, plain_loader<SUFHIP_CHAIN_CUBIC>{&a.nexp, i}, st.thn);
+      const uint64_t v0 = ok ? ev.v[0] : 0, v1 = ok ? ev.v[1] : 0;
+      ex0.set(k, v0);
+      ex1.set(k, v1);
+      const int lo = __builtin_amdgcn_readfirstlane(q), hi = __builtin_amdgcn_readlane(q, 63);
+      for (int r = lo; r <= hi; ++r) {
+        const uint64_t p0 = wave_sum_u64(q == r ? v0 : 0);
+        const uint64_t p1 = wave_sum_u64(q == r ? v1 : 0);
+        if (lane < 2)
+          atomicAdd(reinterpret_cast<unsigned long long*>(&st.sum[r][lane]),
+                    static_cast<unsigned long long>(lane ? p1 : p0));
+      }
+    }
+    // The normalisation triple of score x of the group (its row q): the first
+    // pass's loads are issued here, to land under the reciprocal.
+    uint64_t na[2], nb[2], nc[2];
+    auto load_norm = [&](const SmArgs& a, int x, int q) {
+      const size_t i = size_t(st.first[q]) + size_t(x - st.even0[q]);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        na[p] = a.norm.a[p][i];
+        nb[p] = a.norm.b[p][st.row[q]];
+        nc[p] = a.norm.c[p][i];
+      }
+    };
+    if (tid < total) load_norm(sm_args(), tid, sm_slot(st.even0, tid));
     __syncthreads();
-    // inv = Recip(row sum) on the first wave (its keystream blocks
+    // inv = Recip(row sum), one wave per row (its keystream blocks
     // column-parallel on eight lanes).
-    if (tw == 0 && len > 0) {
-      const Two es{{part[slot][0][0] + part[slot][1][0], part[slot][0][1] + part[slot][1][1]}};
+    if (wave < kSmSlots && st.row[wave] >= 0) {
+      const SmArgs& a = sm_args();
       const Two iv = chain_eval_quad<SUFHIP_CHAIN_RECIP, SmAes, ChainPreN<3>>(
-          a.recip, st.recip, Kr, aes, size_t(r), es, st.rpre[slot], st.thr);
+          a.recip, st.recip, Kr, aes, size_t(st.row[wave]),
+          Two{{st.sum[wave][0], st.sum[wave][1]}}, st.rpre[wave], st.thr);
       if (lane == 0) {
-        invs[slot][0] = iv.v[0];
-        invs[slot][1] = iv.v[1];
+        st.inv[wave][0] = iv.v[0];
+        st.inv[wave][1] = iv.v[1];
       }
     }
     __syncthreads();
     // prob = tr_norm(e * inv[row]) (row-broadcast Beaver), and the next
     // product's open over the dense row.
-    if (len > 0) {
-      const uint64_t inv0 = invs[slot][0], inv1 = invs[slot][1];
-      const uint64_t nb0 = a.norm.b[0][r], nb1 = a.norm.b[1][r];
-      const uint64_t ee = (inv0 - nb0) + (inv1 - nb1);
-      const size_t drow = size_t(r) * size_t(a.dense_cols);
-      if (ok) {
-        const size_t i = size_t(b) + size_t(j);
-        const uint64_t dd = (e0 - na0) + (e1 - na1);
-        const uint64_t z0 = nc0 + dd * nb0 + ee * na0 + dd * ee;
-        const uint64_t z1 = nc1 + dd * nb1 + ee * na1;
-        const uint64_t o = z0 + z1 + a.norm_mask;
-        const uint64_t p0 = trunc_table_eval(a.tr_norm.key[0], a.tr_norm.table[0], a.tr_norm.f, o);
-        const uint64_t p1 = trunc_table_eval(a.tr_norm.key[1], a.tr_norm.table[1], a.tr_norm.f, o);
-        if (a.out[0]) {
-          a.out[0][i] = p0;
-          a.out[1][i] = p1;
-        }
-        if (a.dense) {
-          const size_t di = drow + size_t(j);
-          const uint64_t dv = (p0 - a.dense_a[0][di]) + (p1 - a.dense_a[1][di]);
-          a.dense[di] = dv;
-          if (a.dkb.planes) put_kb_digits(a.dkb, di, dv);
-        }
+#pragma unroll 1
+    for (int k = 0; k < kPer; ++k) {
+      const SmArgs& a = sm_args();
+      const int x = tid + kSmThreads * k;
+      if (x >= total) break;
+      const int q = sm_slot(st.even0, x), r = st.row[q], j = x - st.even0[q];
+      const size_t i = size_t(st.first[q]) + size_t(j);
+      if (k > 0) load_norm(a, x, q);
+      const uint64_t ee = (st.inv[q][0] - nb[0]) + (st.inv[q][1] - nb[1]);
+      const uint64_t dd = (ex0.get(k) - na[0]) + (ex1.get(k) - na[1]);
+      const uint64_t z0 = nc[0] + dd * nb[0] + ee * na[0] + dd * ee;
+      const uint64_t z1 = nc[1] + dd * nb[1] + ee * na[1];
+      const uint64_t o = z0 + z1 + a.norm_mask;
+      const uint64_t p0 = trunc_table_eval(a.tr_norm.key[0], a.tr_norm.table[0], a.tr_norm.f, o);
+      const uint64_t p1 = trunc_table_eval(a.tr_norm.key[1], a.tr_norm.table[1], a.tr_norm.f, o);
+      if (a.out[0]) {
+        a.out[0][i] = p0;
+        a.out[1][i] = p1;
       }
-      if (a.dense)
-        for (int jj = len + j; jj < a.dense_cols; jj += 64 * kSmTeam) {
-          const size_t di = drow + size_t(jj);
-          const uint64_t dv = (uint64_t(0) - a.dense_a[0][di]) + (uint64_t(0) - a.dense_a[1][di]);
-          a.dense[di] = dv;
-          if (a.dkb.planes) put_kb_digits(a.dkb, di, dv);
-        }
+      if (a.dense) {
+        const size_t di = size_t(r) * size_t(a.dense_cols) + size_t(j);
+        const uint64_t dv = (p0 - a.dense_a[0][di]) + (p1 - a.dense_a[1][di]);
+        a.dense[di] = dv;
+        if (a.dkb.planes) put_kb_digits(a.dkb, di, dv);
+      }
+    }
+    if (a.dense) {
+      // Past the rows' ends the probability is 0.
+      for (int x = tid; x < a.slots * a.dense_cols; x += kSmThreads) {
+        const int q = x / a.dense_cols, j = x - q * a.dense_cols;
+        if (st.row[q] < 0 || j < st.len[q]) continue;
+        const size_t di = size_t(st.row[q]) * size_t(a.dense_cols) + size_t(j);
+        const uint64_t dv = (uint64_t(0) - a.dense_a[0][di]) + (uint64_t(0) - a.dense_a[1][di]);
+        a.dense[di] = dv;
+        if (a.dkb.planes) put_kb_digits(a.dkb, di, dv);
+      }
     }
     __syncthreads();  // the row buffers are rewritten by the next group
   }
@@ -798,19 +774,9 @@ __global__ void __launch_bounds__(kSmTeamThreads) softmax2_team_kernel(SmArgs a)
 template <int kPer>
 bool sm_lds_allowed() {
   static const bool ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&softmax2_kernel<kPer>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&softmax2_team_kernel<kPer>),
                           hipFuncAttributeMaxDynamicSharedMemorySize,
                           int(kSmLdsCap - sizeof(SmStatic))) == hipSuccess;
-  return ok;
-}
-
-constexpr size_t kSmTeamStatic = sizeof(SmStatic) + sizeof(uint64_t) * kSmWaves * (2 * kSmTeam + 2);
-
-bool sm_team_lds_allowed() {
-  static const bool ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&softmax2_team_kernel),
-                          hipFuncAttributeMaxDynamicSharedMemorySize,
-                          int(kSmLdsCap - kSmTeamStatic)) == hipSuccess;
   return ok;
 }
 
@@ -998,37 +964,33 @@ int sufhip_softmax2(const sufhip_softmax2_args* args, void* stream) {
                      (g.d_dense && kb_planes_ok(g.dense_planes, size_t(g.rows) * g.dense_cols)),
                  "sufhip_softmax2: dense_planes need d_dense and cover rows x dense_cols");
   A.dkb = g.d_dense ? g.dense_planes : sufhip_kb_planes{};
-  const size_t row_bytes = tree_row_words(g.max_row) * sizeof(uint64_t);
-  const int waves = kSmWaves;
-  const size_t dyn = size_t(waves) * row_bytes;
-  SUFHIP_REQUIRE(sizeof(SmStatic) + dyn <= kSmLdsCap,
-                 "sufhip_softmax2: rows too long for the workgroup's LDS");
-  A.waves = waves;
+  // Rows per workgroup: 8 while their scores fit kSmPer per lane (and their
+  // level buffers the LDS), 6 of the longest.
+  A.slots = g.max_row <= kSmThreads * kSmPer / kSmSlots ? kSmSlots : 6;
+  const size_t dyn = size_t(A.slots) * tree_row_words(g.max_row) * sizeof(uint64_t);
+  // Scores per lane at most: 1, 2 or kSmPer.
+  const int scores = A.slots * g.max_row;
+  const bool lds_ok = scores <= kSmThreads       ? sm_lds_allowed<1>()
+                      : scores <= 2 * kSmThreads ? sm_lds_allowed<2>()
+                                                 : sm_lds_allowed<kSmPer>();
+  SUFHIP_REQUIRE(sizeof(SmStatic) + dyn <= kSmLdsCap && lds_ok,
+                 "sufhip_softmax2: the kernel's LDS size was refused");
   int dev = 0, cus = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  const int per_cu = int(kSmLdsCap / (sizeof(SmStatic) + dyn));
-  const int groups = (g.rows + waves - 1) / waves;
-  const int grid = groups < cus * per_cu ? groups : cus * per_cu;
-  const dim3 block(kSmThreads);
-  hipStream_t s = as_stream(stream);
-  if (g.max_row <= kSmTeamMaxRow) {
-    SUFHIP_REQUIRE(kSmTeamStatic + dyn <= kSmLdsCap && sm_team_lds_allowed(),
-                   "sufhip_softmax2: the kernel's LDS size was refused");
-    hipLaunchKernelGGL(softmax2_team_kernel, dim3(grid), dim3(kSmTeamThreads), dyn, s, A);
-    return check_launch("softmax2_team_kernel");
-  }
-  const bool lds_ok = g.max_row <= 128   ? sm_lds_allowed<2>()
-                      : g.max_row <= 256 ? sm_lds_allowed<4>()
-                                         : sm_lds_allowed<8>();
-  SUFHIP_REQUIRE(lds_ok, "sufhip_softmax2: the kernel's LDS size was refused");
-  if (g.max_row <= 128)
-    hipLaunchKernelGGL(softmax2_kernel<2>, dim3(grid), block, dyn, s, A);
-  else if (g.max_row <= 256)
-    hipLaunchKernelGGL(softmax2_kernel<4>, dim3(grid), block, dyn, s, A);
+  // Rows dealt evenly to whole passes of one workgroup per CU.
+  const size_t passes = (size_t(g.rows) + size_t(A.slots) * cus - 1) / (size_t(A.slots) * cus);
+  const size_t groups = passes * size_t(cus);
+  A.groups = int(groups < size_t(g.rows) ? groups : size_t(g.rows));
+  const int grid = A.groups < cus ? A.groups : cus;
+  const hipStream_t s = as_stream(stream);
+  if (scores <= kSmThreads)
+    hipLaunchKernelGGL(softmax2_team_kernel<1>, dim3(grid), dim3(kSmThreads), dyn, s, A);
+  else if (scores <= 2 * kSmThreads)
+    hipLaunchKernelGGL(softmax2_team_kernel<2>, dim3(grid), dim3(kSmThreads), dyn, s, A);
   else
-    hipLaunchKernelGGL(softmax2_kernel<8>, dim3(grid), block, dyn, s, A);
-  return check_launch("softmax2_kernel");
+    hipLaunchKernelGGL(softmax2_team_kernel<kSmPer>, dim3(grid), dim3(kSmThreads), dyn, s, A);
+  return check_launch("softmax2_team_kernel");
 }
 
 }  // extern "C"

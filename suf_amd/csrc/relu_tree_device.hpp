@@ -218,6 +218,45 @@ __device__ __forceinline__ int tree_interval(const TreeKeys<kRounds>& K,
   return lo - 1 < 0 ? 0 : lo - 1;
 }
 
+// Keystream blocks blk[p][u] (column q, counter in, block out) of round k for
+// both parties; one_ks: party 0's serve both.
+template <int U, int kRounds, class Aes>
+__device__ __forceinline__ void tree_keystream(const Aes& aes, const TreeLds<kRounds>& L, int k,
+                                               int q, bool one_ks, uint32_t (&blk)[2][U]) {
+  const uint32_t* rk0 = reinterpret_cast<const uint32_t*>(L.rk[k][0]) + q;
+  const uint32_t* rk1 = reinterpret_cast<const uint32_t*>(L.rk[k][1]) + q;
+  const uint32_t* rks[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) rks[u] = rk0;
+  if (one_ks) {
+    aes.template encrypt_quad_n<U>(blk[0], rks);
+#pragma unroll
+    for (int u = 0; u < U; ++u) blk[1][u] = blk[0][u];
+  } else if constexpr (U <= 2) {
+    // Both parties' blocks in one lockstep group: one quad-AES latency.
+    uint32_t b2[2 * U];
+    const uint32_t* k2[2 * U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      b2[u] = blk[0][u];
+      b2[U + u] = blk[1][u];
+      k2[u] = rk0;
+      k2[U + u] = rk1;
+    }
+    aes.template encrypt_quad_n<2 * U>(b2, k2);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      blk[0][u] = b2[u];
+      blk[1][u] = b2[U + u];
+    }
+  } else {
+    aes.template encrypt_quad_n<U>(blk[0], rks);
+#pragma unroll
+    for (int u = 0; u < U; ++u) rks[u] = rk1;
+    aes.template encrypt_quad_n<U>(blk[1], rks);
+  }
+}
+
 // One chunk of a level: pair slots t0 .. t0 + nb - 1 (nb <= 64), each AES
 // block spread over a lane quad (AesLds::encrypt_quad_n).  Quad m = lane / 4
 // encrypts slots t0 + m + 16u for u < U (U = ceil(nb / 16)), so a level of
@@ -252,40 +291,7 @@ __device__ __forceinline__ void tree_chunk(const TreeKeys<kRounds>& K, const Tre
       blk[p][u] = q == 0 ? uint32_t(ctr) : (q == 1 ? uint32_t(ctr >> 32) : 0u);
     }
   }
-  {
-    const uint32_t* rk0 = reinterpret_cast<const uint32_t*>(L.rk[k][0]) + q;
-    const uint32_t* rk1 = reinterpret_cast<const uint32_t*>(L.rk[k][1]) + q;
-    const uint32_t* rks[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) rks[u] = rk0;
-    if (one_ks) {
-      aes.template encrypt_quad_n<U>(blk[0], rks);
-#pragma unroll
-      for (int u = 0; u < U; ++u) blk[1][u] = blk[0][u];
-    } else if constexpr (U <= 2) {
-      // Both parties' blocks in one lockstep group: one quad-AES latency.
-      uint32_t b2[2 * U];
-      const uint32_t* k2[2 * U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        b2[u] = blk[0][u];
-        b2[U + u] = blk[1][u];
-        k2[u] = rk0;
-        k2[U + u] = rk1;
-      }
-      aes.template encrypt_quad_n<2 * U>(b2, k2);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        blk[0][u] = b2[u];
-        blk[1][u] = b2[U + u];
-      }
-    } else {
-      aes.template encrypt_quad_n<U>(blk[0], rks);
-#pragma unroll
-      for (int u = 0; u < U; ++u) rks[u] = rk1;
-      aes.template encrypt_quad_n<U>(blk[1], rks);
-    }
-  }
+  tree_keystream<U>(aes, L, k, q, one_ks, blk);
   // Lane q takes block q: column c of it is lane c's word of blk[.][q].
   uint32_t w[2][4];
   uint64_t x = 0, b[2] = {0, 0};

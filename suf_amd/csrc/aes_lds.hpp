@@ -345,6 +345,22 @@ struct AesLds {
              rkq[n][40];
   }
 
+  // One column of a quad (encrypt_quad_n's scheme): the terms its four bytes
+  // give to output columns q, q - 1, q - 2 and q - 3 of a middle round, and
+  // the S-box bytes they give in the last one.
+  __device__ __forceinline__ void quad_terms(uint32_t s, uint32_t (&a)[4]) const {
+    a[0] = b0(s);
+    a[1] = rotl32(b1(s), 8);
+    a[2] = rotl32(b2(s), 16);
+    a[3] = rotl32(b3(s), 24);
+  }
+  __device__ __forceinline__ void quad_last(uint32_t s, uint32_t (&u)[4]) const {
+    u[0] = (b0(s) >> 8) & 0xffu;
+    u[1] = b1(s) & 0xff00u;
+    u[2] = b2(s) & 0xff0000u;
+    u[3] = (b3(s) << 8) & 0xff000000u;
+  }
+
   // Only byte 0 of the ciphertext: rounds 1-8 in full, column 0 of round 9,
   // one S-box lookup in round 10.
   __device__ __forceinline__ uint32_t encrypt_byte0(uint32_t s0, uint32_t s1, uint32_t s2,
@@ -592,11 +608,17 @@ struct AesLds4 {
       s[n] = (lo | hi) ^ rkq[n][40];
     }
   }
-  __device__ __forceinline__ uint32_t encrypt_quad(uint32_t pt, const uint32_t* rkq) const {
-    uint32_t s[1] = {pt};
-    const uint32_t* const k[1] = {rkq};
-    encrypt_quad_n<1>(s, k);
-    return s[0];
+  __device__ __forceinline__ void quad_terms(uint32_t s, uint32_t (&a)[4]) const {
+    a[0] = t<0, 0>(s);
+    a[1] = t<1, 1>(s);
+    a[2] = t<2, 2>(s);
+    a[3] = t<3, 3>(s);
+  }
+  __device__ __forceinline__ void quad_last(uint32_t s, uint32_t (&u)[4]) const {
+    u[0] = t<3, 0>(s) & 0xffu;
+    u[1] = t<0, 1>(s) & 0xff00u;
+    u[2] = t<0, 2>(s) & 0xff0000u;
+    u[3] = t<1, 3>(s) & 0xff000000u;
   }
   // Ciphertext words 0 and 1 only (the final round skips columns 2 and 3).
   __device__ __forceinline__ void encrypt_lo2(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3,

@@ -258,17 +258,16 @@ __global__ void __launch_bounds__(256) kb_split_tiled_kernel(SplitWalkArgs a) {
   const uint32_t wg = kWalk ? a.walk_groups : 0u;
   if constexpr (kWalk) {
     __shared__ __align__(16) uint32_t tab[FusedAes::kWords];
-    __shared__ uint4 rkl[4 * 11];
     if (blockIdx.x < wg) {
       fill_ttable<kFusedCopies>(tab, kTDev.v);
-      fill_round_keys(rkl, a.w.prg.rk, 4);
+      const QuadKeys keys = load_quad_keys(a.w.prg);
       __syncthreads();
       const FusedAes aes{tab, threadIdx.x % kFusedCopies};
       const uint32_t gl = blockIdx.x * 256 + threadIdx.x;
       const uint32_t g = gl >> 3;  // walk; whole 8-lane groups leave together
       if (g >= a.w.begin[a.w.count]) return;
       const int j = batch_job<kFusedWalkJobs>(a.w.begin, a.w.count, g);
-      walk_leaf_path(aes, rkl, a.w.key[j], a.w.out[j], a.w.geo[j], g - a.w.begin[j], gl);
+      walk_leaf_path(aes, keys, a.w.key[j], a.w.out[j], a.w.geo[j], g - a.w.begin[j], gl);
       return;
     }
   }
@@ -291,17 +290,16 @@ static_assert(sizeof(SplitWalkArgs) <= 4096, "kernel argument block must fit in 
 template <int kColK, int kRowK, bool kRagged>
 __global__ void __launch_bounds__(256) kb_split_walk_kernel(SplitWalkArgs a) {
   __shared__ __align__(16) uint32_t tab[FusedAes::kWords];
-  __shared__ uint4 rkl[4 * 11];
   if (blockIdx.x < a.walk_groups) {
     fill_ttable<kFusedCopies>(tab, kTDev.v);
-    fill_round_keys(rkl, a.w.prg.rk, 4);
+    const QuadKeys keys = load_quad_keys(a.w.prg);
     __syncthreads();
     const FusedAes aes{tab, threadIdx.x % kFusedCopies};
     const uint32_t gl = blockIdx.x * 256 + threadIdx.x;
     const uint32_t g = gl >> 3;  // walk; whole 8-lane groups leave together
     if (g >= a.w.begin[a.w.count]) return;
     const int j = batch_job<kFusedWalkJobs>(a.w.begin, a.w.count, g);
-    walk_leaf_path(aes, rkl, a.w.key[j], a.w.out[j], a.w.geo[j], g - a.w.begin[j], gl);
+    walk_leaf_path(aes, keys, a.w.key[j], a.w.out[j], a.w.geo[j], g - a.w.begin[j], gl);
     return;
   }
   split_lanes<kColK, kRowK, kRagged>(a.s, size_t(blockIdx.x - a.walk_groups) * 256 + threadIdx.x,

@@ -56,24 +56,46 @@ __device__ __forceinline__ QuadKeys load_quad_keys(KeySelPtr sel) {
   return K;
 }
 
-// AES_{K_{2b + h}} of the group's seed (column q in s), b chosen by m = -b.
-__device__ __forceinline__ uint32_t quad_encrypt(const AesLds4& aes, const QuadKeys& K,
-                                                 uint32_t m, uint32_t s) {
-  s ^= xor_and(K.k[0], m, K.d[0]);
+// The same keys from a Prg4 in the kernel argument.
+__device__ __forceinline__ QuadKeys load_quad_keys(const Prg4& prg) {
+  QuadKeys K;
+  const uint32_t h = (threadIdx.x >> 2) & 1u, q = threadIdx.x & 3u;
+#pragma unroll
+  for (int r = 0; r < 11; ++r) {
+    K.k[r] = prg.rk[h][4 * r + q];
+    K.d[r] = K.k[r] ^ prg.rk[2 + h][4 * r + q];
+  }
+  return K;
+}
+
+// AES_{K_{2b + h}} of N seeds in lockstep (column q of seed n in s[n]).
+// N = 1: b = b0; else b = (b0 + n) & 1, with b0 known at compile time.
+template <int N, class Aes>
+__device__ __forceinline__ void quad_encrypt_n(const Aes& aes, const QuadKeys& K, uint32_t b0,
+                                               uint32_t (&s)[N]) {
+  const auto key = [&](int r, int n) {
+    if (N == 1) return xor_and(K.k[r], 0u - b0, K.d[r]);
+    return ((b0 + n) & 1u) ? K.k[r] ^ K.d[r] : K.k[r];
+  };
+#pragma unroll
+  for (int n = 0; n < N; ++n) s[n] ^= key(0, n);
 #pragma unroll
   for (int r = 1; r < 10; ++r) {
-    const uint32_t a0 = aes.t<0, 0>(s);
-    const uint32_t a1 = aes.t<1, 1>(s);
-    const uint32_t a2 = aes.t<2, 2>(s);
-    const uint32_t a3 = aes.t<3, 3>(s);
-    const uint32_t kr = xor_and(K.k[r], m, K.d[r]);
-    s = a0 ^ kr ^ quad_rot<1>(a1) ^ quad_rot<2>(a2) ^ quad_rot<3>(a3);
+    uint32_t a[N][4];
+#pragma unroll
+    for (int n = 0; n < N; ++n) aes.quad_terms(s[n], a[n]);
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      s[n] = a[n][0] ^ key(r, n) ^ quad_rot<1>(a[n][1]) ^ quad_rot<2>(a[n][2]) ^
+             quad_rot<3>(a[n][3]);
   }
-  // Final round: S(x) is byte 0 of T3[x], bytes 1 and 2 of T0[x] and byte 3
-  // of T1[x].
-  const uint32_t u0 = aes.t<3, 0>(s) & 0xffu, u1 = aes.t<0, 1>(s) & 0xff00u;
-  const uint32_t u2 = aes.t<0, 2>(s) & 0xff0000u, u3 = aes.t<1, 3>(s) & 0xff000000u;
-  return u0 ^ xor_and(K.k[10], m, K.d[10]) ^ quad_rot<1>(u1) ^ quad_rot<2>(u2) ^ quad_rot<3>(u3);
+  uint32_t u[N][4];
+#pragma unroll
+  for (int n = 0; n < N; ++n) aes.quad_last(s[n], u[n]);
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+    s[n] = u[n][0] ^ key(10, n) ^ quad_rot<1>(u[n][1]) ^ quad_rot<2>(u[n][2]) ^
+           quad_rot<3>(u[n][3]);
 }
 
 // What a walk accumulates: bit 0 of the share, its low 64 bits (additive
@@ -120,7 +142,9 @@ __device__ __forceinline__ void quad_level(const AesLds4& aes, const QuadKeys& K
                                            const QuadCw<kVal>& c, uint32_t xi, uint32_t party,
                                            QuadState& st) {
   const uint32_t l = threadIdx.x & 7u, q = l & 3u;
-  uint32_t on = quad_encrypt(aes, K, 0u - xi, st.s) ^ st.s;
+  uint32_t enc[1] = {st.s};
+  quad_encrypt_n<1>(aes, K, xi, enc);
+  uint32_t on = enc[0] ^ st.s;
   const uint32_t tmask = 0u - st.t;
   if constexpr (kVal == kQuadBit) {
     st.v.lo ^= (on ^ ((c.v[0] >> (8 * c.sh)) & tmask)) & 1u;

@@ -303,9 +303,11 @@ __global__ void __launch_bounds__(256) trunc_eval_table_kernel(TruncEvalArgs a) 
 // blocks stay under 4 KB.
 constexpr int kWalkJobs = 96;
 constexpr int kBatchJobs = 32;
-// Up to 1024 lanes per workgroup: the walk's 8 lanes per node and one
-// workgroup per CU (128 KB of AES tables) must cover a batch in one round.
-constexpr int kWalkBlock = 1024;
+// Up to 768 lanes per workgroup (one per CU: 128 KB of AES tables): the walk's
+// 8 lanes per node cover a batch in one round (plan_walk), and three waves
+// per SIMD leave the lanes the registers for their round keys and the
+// expansion's lockstep groups.
+constexpr int kWalkBlock = 768;
 
 using WalkArgs = WalkJobs<kWalkJobs>;
 
@@ -324,25 +326,31 @@ static_assert(sizeof(WalkArgs) <= 4096 && sizeof(BatchLevelArgs) <= 4096,
               "kernel argument blocks must fit in 4 KB");
 
 __global__ void __launch_bounds__(kWalkBlock) trunc_batch_walk_kernel(WalkArgs a) {
-  SUFHIP_DCF_LDS_SETUP(a.prg);
-  const uint32_t gl = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t g = gl >> 3;  // walk; whole 8-lane groups leave together
-  if (g >= a.begin[a.count]) return;
+  // The walk's job, key header and seed are loaded under the tables' staging.
+  const uint32_t gl = blockIdx.x * uint32_t(a.lanes) + threadIdx.x;
+  const uint32_t total = a.begin[a.count];
+  const bool mine = threadIdx.x < uint32_t(a.lanes) && (gl >> 3) < total;
+  const uint32_t g = (gl >> 3) < total ? gl >> 3 : total - 1;  // walk
   const int j = batch_job<kWalkJobs>(a.begin, a.count, g);
   const uint8_t* key = a.key[j];
   const uint32_t v = g - a.begin[j];
-  if (!(key[7] & 1)) return;
   const uint32_t geo = a.geo[j];
   const int f = int(geo & 0xff), d = int((geo >> 8) & 0xff), e = int(geo >> 16);
   const uint8_t* chunk = key + kHdrBytes + 8;
+  const uint32_t flags = key[7], party = key[6] & 1u;
+  const uint32_t seed = word_at(chunk, int(gl & 3u));
+  const uint64_t last = walk8_last(chunk, f);
+  const QuadKeys keys = load_quad_keys(a.prg);
+  SUFHIP_DCF_TABLE_SETUP();
+  if (!mine || !(flags & 1)) return;  // whole 8-lane groups leave together
   // The body stays in the kernel: passed through a helper function, the same
   // steps spill at the 1024-lane register limit.
-  const Walk8Ctx<DcfAes> c{aes, rkl, chunk, a.out[j], f, uint32_t(key[6] & 1u),
-                           (gl >> 2) & 1u, gl & 3u};
+  const Walk8Ctx<DcfAes> c{aes,   keys,           chunk,   a.out[j], f,
+                           party, (gl >> 2) & 1u, gl & 3u, last};
   const int dw = d - e;  // depth walked before the local expansion
   const uint64_t x = uint64_t(v) << (f - dw);
   Walk8 w;
-  w.s = word_at(chunk, int(c.q));
+  w.s = seed;
   if (c.q == 3) w.s &= 0x7fffffffu;
   w.t = c.party;
   w.v = 0;
@@ -418,14 +426,16 @@ int spread_grid(size_t count, unsigned int* grid, unsigned int* block) {
 }
 
 // Launch shape for the batched walk (8 lanes per walk, no grid stride): the
-// lanes spread over every CU, 128..kWalkBlock per workgroup.
-int walk_grid(size_t count, unsigned int* grid, unsigned int* block) {
+// lanes spread over every CU, 128..kWalkBlock walk lanes per workgroup, in
+// workgroups of 512 threads at least (all of them stage the AES tables).
+int walk_grid(size_t count, unsigned int* grid, unsigned int* block, int* lanes) {
   int cus = 0;
   if (int rc = cu_count(&cus)) return rc;
   size_t per = (count + size_t(cus) - 1) / size_t(cus);
   per = (per + 63) / 64 * 64;
   const size_t b = per < 128 ? 128 : (per > size_t(kWalkBlock) ? size_t(kWalkBlock) : per);
-  *block = unsigned(b);
+  *lanes = int(b);
+  *block = unsigned(b < 512 ? 512 : b);
   *grid = unsigned((count + b - 1) / b);
   return SUFHIP_OK;
 }
@@ -522,13 +532,13 @@ int plan_walk(const uint8_t* prg_state, const sufhip_trunc_job* jobs, int m, con
   // Local levels of the full-domain walks: a walk level costs about as
   // much as one lockstep group of the expansion, so the walks go as deep as
   // the lanes allow -- the fewest local levels whose walks take less than
-  // three quarters of one full workgroup per CU (at most kWalkLocal; past
-  // that the extra waves per SIMD slow every level more than a local level
-  // costs).  A hosted walk (lanes_cap > 0) takes the fewest whose walks fit
+  // one full workgroup per CU (at most kWalkLocal; with 1024 lanes per
+  // workgroup the extra waves per SIMD slowed every level more than a local
+  // level costs).  A hosted walk (lanes_cap > 0) takes the fewest whose walks fit
   // in the host's room.
   int cus = 0;
   if (int rc = cu_count(&cus)) return rc;
-  const size_t cap = lanes_cap > 0 ? lanes_cap + 1 : 3 * size_t(cus) * kWalkBlock / 4;
+  const size_t cap = lanes_cap > 0 ? lanes_cap + 1 : size_t(cus) * kWalkBlock;
   p.el = 0;
   for (; p.el < kWalkLocal; ++p.el) {
     size_t lanes = 0;
@@ -796,7 +806,7 @@ int sufhip_trunc_prepare_batch(const uint8_t* prg_state, const sufhip_trunc_job*
     wa.count = m;
     if (wa.begin[m] > 0) {
       unsigned int g = 0, b = 0;
-      if (int rc = walk_grid(8 * size_t(wa.begin[m]), &g, &b)) return rc;
+      if (int rc = walk_grid(8 * size_t(wa.begin[m]), &g, &b, &wa.lanes)) return rc;
       hipLaunchKernelGGL(trunc_batch_walk_kernel, dim3(g), dim3(b), 0, s, wa);
       if (int rc = check_launch("trunc_batch_walk_kernel")) return rc;
     }

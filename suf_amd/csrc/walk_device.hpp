@@ -62,6 +62,7 @@ template <int kJobs>
 struct WalkJobs {
   Prg4 prg;
   int count;
+  int lanes;  // walk lanes per workgroup (trunc_batch_walk_kernel)
   uint32_t begin[kJobs + 1];
   const uint8_t* key[kJobs];
   uint4* out[kJobs];
@@ -70,18 +71,28 @@ struct WalkJobs {
 
 // The job of lane g: the last j < count with begin[j] <= g (jobs with no
 // lanes share their begin with the next job, so the last such j owns g).
+// g grows with the lane: a scalar search for the wave's first lane, then the
+// wave advances together (a search per lane was a chain of vector loads of
+// the kernel argument, a microsecond or two before the walk could start).
 template <int kJobs>
 __device__ __forceinline__ int batch_job(const uint32_t (&begin)[kJobs + 1], int count,
                                          uint32_t g) {
+  const uint32_t g0 = uint32_t(__builtin_amdgcn_readfirstlane(int(g)));
   int lo = 0, hi = count - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (begin[mid] <= g)
+    if (begin[mid] <= g0)
       lo = mid;
     else
       hi = mid - 1;
   }
-  return lo;
+  int j = lo;
+  for (int k = lo + 1; k < count; ++k) {
+    const bool past = begin[k] <= g;
+    if (__ballot(past) == 0) break;
+    if (past) j = k;
+  }
+  return j;
 }
 
 // One walk per 8 lanes.  Lanes 0-3 of the group compute the next-seed block
@@ -96,14 +107,23 @@ struct Walk8 {
   uint64_t v;  // accumulated value, low 64 bits (value half)
 };
 
+// Words 0 and 1 of a key's last correction word (cw_np1).
+__device__ __forceinline__ uint64_t walk8_last(const uint8_t* chunk, int f) {
+  const uint8_t* np1 = chunk + 16 + 33 * f;
+  return uint64_t(word_at(np1, 0)) | uint64_t(word_at(np1, 1)) << 32;
+}
+
 template <class Aes>
 struct Walk8Ctx {
   const Aes& aes;
-  const uint4* rkl;
+  const QuadKeys& keys;
   const uint8_t* chunk;
   uint4* nodes;
   int f;
   uint32_t party, h, q;
+  // cw_np1, read before the first entry is stored: read entry by entry, each
+  // entry waited for a load that the previous one's store kept behind it.
+  uint64_t last;
 };
 
 // One level (record cw) of N independent walks in lockstep: walk n goes
@@ -116,14 +136,9 @@ __device__ __forceinline__ void walk8_step_n(const Ctx& c, const uint8_t* cw, ui
   const uint64_t cv = uint64_t(word_at(cw, 4)) | uint64_t(word_at(cw, 5)) << 32;
   const uint32_t tb = cw[32];
   uint32_t o[N];
-  const uint32_t* rkq[N];
 #pragma unroll
-  for (int n = 0; n < N; ++n) {
-    const uint32_t b = N == 1 ? b0 : ((b0 + n) & 1u);
-    o[n] = par[N == 1 ? 0 : (b0 + n) >> 1].s;
-    rkq[n] = reinterpret_cast<const uint32_t*>(c.rkl + 11 * (2 * b + c.h)) + c.q;
-  }
-  c.aes.template encrypt_quad_n<N>(o, rkq);
+  for (int n = 0; n < N; ++n) o[n] = par[N == 1 ? 0 : (b0 + n) >> 1].s;
+  quad_encrypt_n<N>(c.aes, c.keys, b0, o);
 #pragma unroll
   for (int n = 0; n < N; ++n) {
     const Walk8& w = par[N == 1 ? 0 : (b0 + n) >> 1];
@@ -150,10 +165,8 @@ __device__ __forceinline__ void walk8_step_n(const Ctx& c, const uint8_t* cw, ui
 // of the value half, which holds the seed, t and v.
 template <class Ctx>
 __device__ __forceinline__ void walk8_leaf(const Ctx& c, const Walk8& w, uint32_t leaf) {
-  const uint8_t* np1 = c.chunk + 16 + 33 * c.f;
   const uint64_t s64 = uint64_t(quad_bcast<0>(w.s)) | uint64_t(quad_bcast<1>(w.s)) << 32;
-  const uint64_t n64 = uint64_t(word_at(np1, 0)) | uint64_t(word_at(np1, 1)) << 32;
-  const uint64_t sv = s64 + (w.t ? n64 : 0);
+  const uint64_t sv = s64 + (w.t ? c.last : 0);
   const uint64_t out = w.v + (c.party ? 0 - sv : sv);
   if (c.h == 1 && c.q == 0)
     c.nodes[2 * leaf + 1] = make_uint4(uint32_t(out), uint32_t(out >> 32), 0, 0);
@@ -195,13 +208,14 @@ __device__ __forceinline__ void walk8_expand(const Ctx& c, const uint8_t* cw,
 // (trunc_batch_walk_kernel runs the same steps with local levels and
 // frontier nodes.)
 template <class Aes>
-__device__ __forceinline__ void walk_leaf_path(const Aes& aes, const uint4* rkl,
+__device__ __forceinline__ void walk_leaf_path(const Aes& aes, const QuadKeys& keys,
                                                const uint8_t* key, uint4* out, uint32_t geo,
                                                uint32_t v, uint32_t gl) {
   if (!(key[7] & 1)) return;
   const int f = int(geo & 0xff);
   const uint8_t* chunk = key + kTruncHdrBytes + 8;
-  const Walk8Ctx<Aes> c{aes, rkl, chunk, out, f, uint32_t(key[6] & 1u), (gl >> 2) & 1u, gl & 3u};
+  const Walk8Ctx<Aes> c{aes, keys, chunk, out, f, uint32_t(key[6] & 1u), (gl >> 2) & 1u, gl & 3u,
+                        walk8_last(chunk, f)};
   Walk8 w;
   w.s = word_at(chunk, int(c.q));
   if (c.q == 3) w.s &= 0x7fffffffu;
@@ -223,12 +237,13 @@ __device__ __forceinline__ void walk_leaf_path(const Aes& aes, const uint4* rkl,
 // fewer (the expansion's lockstep groups need more than the 128 registers
 // of a 1024-lane workgroup when passed through this function).
 template <class Aes>
-__device__ __forceinline__ void walk_table(const Aes& aes, const uint4* rkl, const uint8_t* key,
+__device__ __forceinline__ void walk_table(const Aes& aes, const QuadKeys& keys, const uint8_t* key,
                                            uint4* out, uint32_t geo, uint32_t v, uint32_t gl) {
   if (!(key[7] & 1)) return;
   const int f = int(geo & 0xff), e = int(geo >> 16);
   const uint8_t* chunk = key + kTruncHdrBytes + 8;
-  const Walk8Ctx<Aes> c{aes, rkl, chunk, out, f, uint32_t(key[6] & 1u), (gl >> 2) & 1u, gl & 3u};
+  const Walk8Ctx<Aes> c{aes, keys, chunk, out, f, uint32_t(key[6] & 1u), (gl >> 2) & 1u, gl & 3u,
+                        walk8_last(chunk, f)};
   Walk8 w;
   w.s = word_at(chunk, int(c.q));
   if (c.q == 3) w.s &= 0x7fffffffu;
@@ -266,14 +281,13 @@ template <int kJobs, bool kFour>
 __device__ __forceinline__ void hosted_walk_role(const WalkJobs<kJobs>& w, uint32_t gl) {
   using Aes = std::conditional_t<kFour, DcfAes, AesLds<kHostedWalkCopies>>;
   __shared__ __align__(16) uint32_t wtab[Aes::kWords];
-  __shared__ uint4 rkl[4 * 11];
   if constexpr (kFour) {
     __shared__ uint32_t stage[256];
     DcfAes::fill(wtab, stage, kTDev.v);
   } else {
     fill_ttable<kHostedWalkCopies>(wtab, kTDev.v);
   }
-  fill_round_keys(rkl, w.prg.rk, 4);
+  const QuadKeys keys = load_quad_keys(w.prg);
   __syncthreads();
   const Aes aes = [&] {
     if constexpr (kFour)
@@ -284,7 +298,7 @@ __device__ __forceinline__ void hosted_walk_role(const WalkJobs<kJobs>& w, uint3
   const uint32_t g = gl >> 3;
   if (g >= w.begin[w.count]) return;
   const int j = batch_job<kJobs>(w.begin, w.count, g);
-  walk_table(aes, rkl, w.key[j], w.out[j], w.geo[j], g - w.begin[j], gl);
+  walk_table(aes, keys, w.key[j], w.out[j], w.geo[j], g - w.begin[j], gl);
 }
 
 // Host side of a hosted walk: w for `count` jobs walked by a launch with

@@ -324,18 +324,15 @@ struct Bm2Args {
 
 // Party p's finished 32 x 32 tile values (lane l: column l % 32, rows of
 // the accumulator layout) to out_p, and to the output digit planes.
-// kRagged: rows and columns past vM and vN are padding (no merge, no planes).
-template <bool kRagged = false>
 __device__ __forceinline__ void bm2_store(const Bm2Args& a, int p, int l, int m0, int n0, size_t b,
                                           const uint64_t (&v)[16]) {
-  const int M = kRagged ? a.vM : a.M, N = kRagged ? a.vN : a.N;
+  const int M = a.M, N = a.N;
   const int col = n0 + (l & 31);
   const size_t ob = b * size_t(M) * N;
   const size_t ld = size_t(a.batches) * N;  // merged row length
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-    if (kRagged && (row >= M || col >= N)) continue;
     const size_t o = a.merge ? size_t(row) * ld + b * N + col : ob + size_t(row) * N + col;
     a.out[p][o] = v[r];
     if (a.xp.planes) put_x_digits(a.xp, size_t(M), o, p, v[r]);
@@ -346,11 +343,10 @@ __device__ __forceinline__ void bm2_store(const Bm2Args& a, int p, int l, int m0
 // wave p opens rows r in [8p, 8p + 8) and writes both parties' outputs.
 // eh: the gate's key headers, read before the kernel's first global store;
 // every table read is issued before the first output store.
-template <bool kRagged = false>
 __device__ __forceinline__ void bm2_trunc_rows(const Bm2Args& a, const EpiHdrs& eh, int p, int l,
                                                int m0, int n0, size_t b,
                                                const uint64_t (*both)[16][64]) {
-  const int M = kRagged ? a.vM : a.M, N = kRagged ? a.vN : a.N;
+  const int M = a.M, N = a.N;
   const int col = n0 + (l & 31);
   const size_t ob = b * size_t(M) * N;
   const size_t ld = size_t(a.batches) * N;
@@ -367,7 +363,6 @@ __device__ __forceinline__ void bm2_trunc_rows(const Bm2Args& a, const EpiHdrs& 
   }
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    if (kRagged && (m0 + 8 * ((8 * p + q) >> 2) + 4 * (l >> 5) + (q & 3) >= M || col >= N)) continue;
     const uint64_t y0 = trunc_table_out(eh.h[0], a.epi.f, open[q], w[q][0]);
     const uint64_t y1 = trunc_table_out(eh.h[1], a.epi.f, open[q], w[q][1]);
     a.epi.y[0][o[q]] = y0;
@@ -473,22 +468,29 @@ __global__ void __launch_bounds__(128 * kKWaves) beaver_mfma2_kernel(Bm2Args a) 
   if (kw == 0) bm2_trunc_rows(a, eh, p, l, m0, n0, b, both);
 }
 
-// Balanced form (Xp given): wave p computes party p's tile over every
-// k-step as two operand products, (L_p, E) with L_0 = D + A_0 and L_1 = A_1,
-// then (D, B_p): 72 MFMAs per party and step, so the two waves of a tile
-// finish together.  The operand pairs run through a register pipeline
-// kStages deep (a pair's planes are loaded kStages - 1 pairs before its
-// MFMAs), which keeps loads in flight while the wave -- the only one on its
-// SIMD -- multiplies.  Bases are wave-uniform (scalar registers) plus each
-// lane's 32-bit fragment offset.  kPrefC (short K, three stages): the
-// wave's 16 C_p words are loaded with the first operand pairs, so the tile
-// needs no memory round trip after the k-loop (four stages leave no
-// registers for them).
-template <int kStages, bool kPrefC, bool kRagged>
-__global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
-  __shared__ uint64_t both[2][16][64];
+// Balanced form (Xp given): party p's tile as two operand products per k-step,
+// (L_p, E) with L_0 = D + A_0 and L_1 = A_1, then (D, B_p): 72 MFMAs per party
+// and step, so the two parties' waves of a tile finish together.  The operand
+// pairs run through a register pipeline kStages deep (a pair's planes are
+// loaded kStages - 1 pairs before its MFMAs), which keeps loads in flight
+// while the wave -- the only one on its SIMD -- multiplies.  Bases are
+// wave-uniform (scalar registers) plus each lane's 32-bit fragment offset.
+//
+// kKW waves per party and tile take a share of the pairs each (1, or 2: a
+// tile then fills its CU's four SIMDs), for products of few tiles (77 x 300 x
+// 1000: 96 tiles, 192 waves on 1024 SIMDs: 23.7 -> 15.7 us; the layer's QK^T
+// 12.5 -> 9.8, PV 18.4 -> 13.1).  The partial tiles meet in LDS, where wave w of the
+// 2 kKW finishes rows [16 / (2 kKW) w, ...) of both parties.  kPrefC: the
+// finishing rows' C words are loaded with the first operand pairs, so the
+// tile needs no memory round trip after the k-loop (four stages leave no
+// registers for 16 of them).
+template <int kStages, bool kPrefC, int kKW, bool kRagged>
+__global__ void __launch_bounds__(128 * kKW, 1) beaver_bal_kernel(Bm2Args a) {
+  constexpr int kRows = 8 / kKW;
+  __shared__ uint64_t part[kKW][2][16][64];
   const int l = threadIdx.x & 63;
-  const int p = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int p = w & 1, kh = w >> 1;
   const int M = a.M, K = a.K, N = a.N;
   const int n0 = blockIdx.x * 32, m0 = blockIdx.y * 32;
   const size_t b = blockIdx.z;
@@ -505,29 +507,37 @@ __global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
   const int col = n0 + (l & 31);
   const int vM = kRagged ? a.vM : M, vN = kRagged ? a.vN : N;
   const size_t ob = b * size_t(vM) * vN;
-  const auto c_word = [&](int r) -> uint64_t {
-    const int row = m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-    if (kRagged && (row >= vM || col >= vN)) return 0;
-    return a.C[p][ob + size_t(row) * vN + col];
+  const auto row_of = [&](int q) {
+    const int r = kRows * w + q;
+    return m0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
   };
-  uint64_t cpre[16];
+  const auto c_word = [&](int party, int q) -> uint64_t {
+    const int row = row_of(q);
+    if (kRagged && (row >= vM || col >= vN)) return 0;
+    return a.C[party][ob + size_t(row) * vN + col];
+  };
+  uint64_t cpre[2][kRows];
   if constexpr (kPrefC) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) cpre[r] = c_word(r);
+    for (int q = 0; q < kRows; ++q) {
+      cpre[0][q] = c_word(0, q);
+      cpre[1][q] = c_word(1, q);
+    }
   }
   v16i acc[kDigitPlanes];
 #pragma unroll
   for (int s = 0; s < kDigitPlanes; ++s)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[s][r] = 0;
-  // Operand pairs u = 2 step + (0: (L_p, E), 1: (D, B_p)).  The loop runs
-  // over whole groups of kStages pairs; loads past the last pair repeat it
-  // (in bounds) and their MFMAs are skipped.
+  // Operand pairs u = 2 step + (0: (L_p, E), 1: (D, B_p)); this wave's are
+  // [u0, u1).  The loop runs over whole groups of kStages pairs; loads past
+  // the last pair repeat it (in bounds) and their MFMAs are skipped.
   const int U = 2 * (K / 32);
-  const int Ug = (U + kStages - 1) / kStages * kStages;
+  const int u0 = U * kh / kKW, u1 = U * (kh + 1) / kKW;
   v4i L[kStages][kDigitPlanes], R[kStages][kDigitPlanes];
   auto issue = [&](int q, int u) {
-    u = u < U ? u : U - 1;
+    u = u < u1 ? u : u1 - 1;
+    u = u > 0 ? u : 0;
     const uint32_t st = uint32_t(u >> 1);
     const int8_t* lb = (u & 1) ? Ld : Lx;
     const int8_t* rb = (u & 1) ? Rb : Re;
@@ -538,13 +548,13 @@ __global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
     }
   };
 #pragma unroll
-  for (int q = 0; q < kStages - 1; ++q) issue(q, q);
-  for (int u0 = 0; u0 < Ug; u0 += kStages) {
+  for (int q = 0; q < kStages - 1; ++q) issue(q, u0 + q);
+  for (int v0 = u0; v0 < u1; v0 += kStages) {
 #pragma unroll
     for (int h = 0; h < kStages; ++h) {
-      const int u = u0 + h;
+      const int u = v0 + h;
       issue((h + kStages - 1) % kStages, u + kStages - 1);
-      if (u < U) {
+      if (u < u1) {
 #pragma unroll
         for (int i = 0; i < kDigitPlanes; ++i)
 #pragma unroll
@@ -555,22 +565,73 @@ __global__ void __launch_bounds__(128, 1) beaver_bal_kernel(Bm2Args a) {
     }
   }
   const EpiHdrs eh = epi_hdrs(a.epi);
-  uint64_t v[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
-    v[r] = 0;
+    uint64_t v = 0;
 #pragma unroll
-    for (int s = 0; s < kDigitPlanes; ++s) v[r] += uint64_t(int64_t(acc[s][r])) << (8 * s);
-    v[r] += kPrefC ? cpre[r] : c_word(r);
+    for (int s = 0; s < kDigitPlanes; ++s) v += uint64_t(int64_t(acc[s][r])) << (8 * s);
+    part[kh][p][r][l] = v;
   }
-  if (!a.epi.on) {
-    bm2_store<kRagged>(a, p, l, m0, n0, b, v);
-    return;
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) both[p][r][l] = v[r];
   __syncthreads();
-  bm2_trunc_rows<kRagged>(a, eh, p, l, m0, n0, b, both);
+  // Both parties' values of the wave's rows, then every table read before the
+  // first output store.
+  uint64_t z[2][kRows], wd[2][kRows];
+  size_t o[kRows];
+  bool in[kRows];
+  const size_t ld = size_t(a.batches) * vN;
+#pragma unroll
+  for (int q = 0; q < kRows; ++q) {
+    const int row = row_of(q);
+    in[q] = !kRagged || (row < vM && col < vN);
+    o[q] = a.merge ? size_t(row) * ld + b * vN + col : ob + size_t(row) * vN + col;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      z[t][q] = kPrefC ? cpre[t][q] : c_word(t, q);
+#pragma unroll
+      for (int g = 0; g < kKW; ++g) z[t][q] += part[g][t][kRows * w + q][l];
+    }
+  }
+  if (a.epi.on) {
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      const uint64_t open = z[0][q] + z[1][q] + a.mask;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        wd[t][q] = trunc_table_word(eh.h[t], a.epi.table[t], a.epi.f, open);
+    }
+#pragma unroll
+    for (int q = 0; q < kRows; ++q) {
+      const uint64_t open = z[0][q] + z[1][q] + a.mask;
+      z[0][q] = trunc_table_out(eh.h[0], a.epi.f, open, wd[0][q]);
+      z[1][q] = trunc_table_out(eh.h[1], a.epi.f, open, wd[1][q]);
+    }
+  }
+  uint64_t* const y[2] = {a.epi.on ? a.epi.y[0] : a.out[0], a.epi.on ? a.epi.y[1] : a.out[1]};
+#pragma unroll
+  for (int q = 0; q < kRows; ++q) {
+    if (!in[q]) continue;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      y[t][o[q]] = z[t][q];
+      if (a.xp.planes) put_x_digits(a.xp, size_t(M), o[q], t, z[t][q]);
+    }
+  }
+}
+
+// Launches the balanced product: waves per party by what its tiles leave idle
+// (one wave per SIMD is all the registers allow), and at least two operand
+// pairs to a wave.
+template <bool kRagged>
+void launch_bal(const Bm2Args& a, const dim3& grid, int cus, hipStream_t st) {
+  const size_t tiles = size_t(grid.x) * grid.y * grid.z;
+  const int pairs = 2 * (a.K / 32);
+  const size_t simds = 4 * size_t(cus);
+  if (pairs >= 4 && 4 * tiles <= simds)
+    hipLaunchKernelGGL((beaver_bal_kernel<3, true, 2, kRagged>), grid, dim3(256), 0, st, a);
+  else if (pairs <= 8)
+    hipLaunchKernelGGL((beaver_bal_kernel<3, true, 1, kRagged>), grid, dim3(128), 0, st, a);
+  else
+    hipLaunchKernelGGL((beaver_bal_kernel<4, false, 1, kRagged>), grid, dim3(128), 0, st, a);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -869,17 +930,12 @@ int sufhip_beaver_matmul2_mfma_ex(const sufhip_beaver_mfma2_args* args, void* st
   const uint64_t plane_set = uint64_t(kDigitPlanes) * uint64_t(g.batches) * uint64_t(g.K) *
                              uint64_t(g.M > g.N ? g.M : g.N);
   if (g.Xp && plane_set < (uint64_t(1) << 32)) {
-    const hipStream_t st = as_stream(stream);
-    if (g.K <= 128) {  // at most 8 operand pairs
-      if (ragged)
-        hipLaunchKernelGGL((beaver_bal_kernel<3, true, true>), grid, dim3(128), 0, st, a);
-      else
-        hipLaunchKernelGGL((beaver_bal_kernel<3, true, false>), grid, dim3(128), 0, st, a);
-    } else if (ragged) {
-      hipLaunchKernelGGL((beaver_bal_kernel<4, false, true>), grid, dim3(128), 0, st, a);
-    } else {
-      hipLaunchKernelGGL((beaver_bal_kernel<4, false, false>), grid, dim3(128), 0, st, a);
-    }
+    int cus = 0;
+    if (int rc = cu_count(&cus)) return rc;
+    if (ragged)
+      launch_bal<true>(a, grid, cus, as_stream(stream));
+    else
+      launch_bal<false>(a, grid, cus, as_stream(stream));
     return check_launch("beaver_bal_kernel");
   }
   SUFHIP_REQUIRE(!ragged, "sufhip_beaver_matmul2_mfma_ex: valid_m / valid_n with planes of 4 GiB");

@@ -18,7 +18,7 @@ STATE = ol.mt64_bytes(3, ol.PRG_STATE_BYTES).tobytes()
 @pytest.mark.parametrize("M,K,N,f", [
     (1, 1, 1, 12), (1, 16, 33, 8), (31, 33, 65, 13), (32, 100, 64, 12), (33, 64, 32, 12),
     (77, 300, 1000, 12), (3, 129, 2000, 12), (40, 1023, 2050, 12), (5, 1023, 2100, 12),
-    (250, 160, 31, 12)])
+    (250, 160, 31, 12), (64, 64, 64, 12), (32, 96, 480, 12), (31, 32, 33, 12)])
 def test_ragged_gate_equals_step_form(M, K, N, f):
     say("matmul gate ragged %dx%dx%d f=%d" % (M, K, N, f))
     native.call("sufhip_init", 0)

@@ -31,6 +31,7 @@ namespace {
 constexpr int kLnBlock = 512;
 constexpr int kLnWideBlock = 256;
 constexpr int kLnMaxPer = 2;      // elements per thread at kLnBlock: cols <= 1024
+constexpr int kLnPairPer = 4;     // at kLnWideBlock, two rows per CU: cols <= 1024
 constexpr int kLnWidePer = 8;     // at kLnWideBlock: cols <= 2048
 constexpr int kLnCopies = 4;  // the T table serves one lane per workgroup
 using LnAes = AesLds<kLnCopies>;  // one lane's chain: the small table fills fastest
@@ -67,7 +68,8 @@ constexpr int kLnMaxInPer = kLnMaxPer;  // in_slices rows of up to 1024 elements
 // instantiation, so that launches without walks keep the rows' own register
 // allocation and LDS).
 template <int kPer, bool kIn, int kBlock, bool kWalk>
-__global__ void __launch_bounds__(kBlock) layernorm2_kernel(LnArgs A) {
+__global__ void __launch_bounds__(kBlock, kBlock == kLnWideBlock && kPer <= kLnPairPer ? 2 : 1)
+    layernorm2_kernel(LnArgs A) {
   constexpr int kLnWaves = kBlock / 64;
   if constexpr (kWalk) {
     if (int(blockIdx.x) >= A.row_groups) {
@@ -864,11 +866,15 @@ int sufhip_layernorm2(const sufhip_layernorm2_args* args, void* stream) {
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   const int grid = g.rows < cus * 8 ? g.rows : cus * 8;
   const int per = (g.cols + kLnBlock - 1) / kLnBlock;
-  const int block = per <= kLnMaxPer || A.in_slices ? kLnBlock : kLnWideBlock;
+  // More rows than CUs: 256 lanes per row leave the registers for two rows on
+  // a CU, where 512 hold one (300 x 1001: 38 -> 25 us, 256 rows then 44 before;
+  // a row alone takes about 1 us longer).
+  const bool pair = g.rows > cus && per <= kLnMaxPer && !A.in_slices;
+  const int block = (per <= kLnMaxPer || A.in_slices) && !pair ? kLnBlock : kLnWideBlock;
   A.row_groups = grid;
   // The walks: one workgroup per CU fits beside the rows' (the kernel's
   // registers allow one), so the CUs without a row hold one pass of them.
-  // The 256-lane form for rows past 1024 elements walks nothing itself.
+  // The 256-lane forms walk nothing themselves.
   size_t walk_lanes = 0;
   if (block == kLnBlock) {
     if (int rc = plan_hosted_walk(g.walk_prg_state, g.walk_jobs, g.walk_count,
@@ -894,7 +900,10 @@ int sufhip_layernorm2(const sufhip_layernorm2_args* args, void* stream) {
                          s, A);
   };
   using PerOne = std::integral_constant<int, 1>;
-  if (A.in_slices) {
+  if (pair) {
+    hipLaunchKernelGGL((layernorm2_kernel<kLnPairPer, false, kLnWideBlock, false>), launch,
+                       dim3(kLnWideBlock), 0, s, A);
+  } else if (A.in_slices) {
     if (per <= 1)
       rows512(PerOne{}, std::true_type{});
     else

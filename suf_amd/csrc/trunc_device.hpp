@@ -22,6 +22,17 @@ constexpr int kTruncHdrBytes = 64;
 // read per element at evaluation).
 constexpr int kTruncTableBits = 14;
 
+// The prepared carry share at point v.  Tables of up to kTruncTableBits bits
+// are 8-byte entries (32 KB at 12 bits, an L1's worth, where whole frontier
+// nodes take four times that: a gather's 64 lanes share fewer lines; spline
+// gate at 2^20 98.9 -> 96.9 us, the secure layer 289 -> 282); deeper full
+// domains keep the nodes of the frontier they are expanded from.
+__device__ __forceinline__ uint64_t trunc_table_at(const uint4* table, int f, uint64_t v) {
+  if (f <= kTruncTableBits) return reinterpret_cast<const uint64_t*>(table)[v];
+  const uint4 q = table[2 * v + 1];
+  return uint64_t(q.x) | uint64_t(q.y) << 32;
+}
+
 struct TruncHdr {
   uint32_t tag, kind, f, party, flags;
   uint64_t r_hi, base, cw, sw, m;
@@ -97,10 +108,8 @@ __device__ __forceinline__ uint64_t trunc_table_eval_h(const TruncHdr& h, const 
                                                        int f, uint64_t xhat) {
   if (h.tag != kTruncTag || h.kind != SUFHIP_TRUNC_GAPARS || int(h.f) != f) return 0;
   uint64_t carry = 0;
-  if (h.flags & 1) {
-    const uint4 q = table[2 * (xhat & ((uint64_t(1) << f) - 1)) + 1];
-    carry = trunc_carry_from(h, uint64_t(q.x) | uint64_t(q.y) << 32);
-  }
+  if (h.flags & 1)
+    carry = trunc_carry_from(h, trunc_table_at(table, f, xhat & ((uint64_t(1) << f) - 1)));
   return trunc_postproc<SUFHIP_TRUNC_GAPARS>(h, f, xhat, carry, 0, 0);
 }
 
@@ -128,8 +137,7 @@ __device__ __forceinline__ bool trunc_table_key_ok(const TruncHdr& h, int f) {
 __device__ __forceinline__ uint64_t trunc_table_word(const TruncHdr& h, const uint4* table, int f,
                                                      uint64_t xhat) {
   if (!trunc_table_key_ok(h, f) || !(h.flags & 1)) return 0;
-  const uint4 q = table[2 * (xhat & ((uint64_t(1) << f) - 1)) + 1];
-  return uint64_t(q.x) | uint64_t(q.y) << 32;
+  return trunc_table_at(table, f, xhat & ((uint64_t(1) << f) - 1));
 }
 __device__ __forceinline__ uint64_t trunc_table_out(const TruncHdr& h, int f, uint64_t xhat,
                                                     uint64_t word) {

@@ -264,8 +264,7 @@ __global__ void __launch_bounds__(kForestBlock) trunc_eval_aes_kernel(TruncEvalA
         if (carry_walk) {
           c = share[kDcf * span + i];
         } else {
-          const uint4 q = nodes[2 * (x & low) + 1];
-          c = uint64_t(q.x) | uint64_t(q.y) << 32;
+          c = trunc_table_at(nodes, a.f, x & low);
         }
         carry = carry_from(h, c);
       }
@@ -289,10 +288,7 @@ __global__ void __launch_bounds__(256) trunc_eval_table_kernel(TruncEvalArgs a) 
   for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) {
     const uint64_t x = a.xhat[e];
     uint64_t carry = 0;
-    if (h.flags & 1) {
-      const uint4 q = nodes[2 * (x & low) + 1];
-      carry = carry_from(h, uint64_t(q.x) | uint64_t(q.y) << 32);
-    }
+    if (h.flags & 1) carry = carry_from(h, trunc_table_at(nodes, a.f, x & low));
     y[e] = postproc<SUFHIP_TRUNC_GAPARS>(h, a.f, x, carry, 0, 0);
   }
 }

@@ -168,8 +168,13 @@ __device__ __forceinline__ void walk8_leaf(const Ctx& c, const Walk8& w, uint32_
   const uint64_t s64 = uint64_t(quad_bcast<0>(w.s)) | uint64_t(quad_bcast<1>(w.s)) << 32;
   const uint64_t sv = s64 + (w.t ? c.last : 0);
   const uint64_t out = w.v + (c.party ? 0 - sv : sv);
-  if (c.h == 1 && c.q == 0)
-    c.nodes[2 * leaf + 1] = make_uint4(uint32_t(out), uint32_t(out >> 32), 0, 0);
+  if (c.h == 1 && c.q == 0) {
+    // trunc_table_at's entries.
+    if (c.f <= kTruncTableBits)
+      reinterpret_cast<uint64_t*>(c.nodes)[leaf] = out;
+    else
+      c.nodes[2 * leaf + 1] = make_uint4(uint32_t(out), uint32_t(out >> 32), 0, 0);
+  }
 }
 
 // Breadth-first expansion of the subtree below a depth-(f - E) node: the

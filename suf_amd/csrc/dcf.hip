@@ -13,7 +13,7 @@
 // only on bit 0 of the terms, and bit 0 of -v equals bit 0 of v, so this
 // holds for both output groups.
 //
-// Batches of more than 256 keys per CU: one element per lane; each lane streams its own key front to back
+// Batches of more than 320 keys per CU: one element per lane; each lane streams its own key front to back
 // (33 bytes per level), so successive levels hit the same cache lines.
 //
 // The evaluation kernels run 1024 lanes per CU (four waves per SIMD): their
@@ -179,6 +179,52 @@ __global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_quad_bytes_kernel(DcfEv
   }
 }
 
+// Middling batches: 2 lanes per walk (dcf_quad_device.hpp).  The group only
+// matters for the bits past bit 0.
+template <int kMode, int kGroup>
+__global__ void __launch_bounds__(kPairBlock) dcf_eval_pair_kernel(DcfEvalArgs a) {
+  SUFHIP_DCF_TABLE_SETUP();
+  const PairKeys K = load_pair_keys(kernarg_key_sel(offsetof(DcfEvalArgs, key_sel)));
+  const size_t chunk_bytes = 32 + 33 * size_t(a.in_bits);
+  const size_t walks = a.n * size_t(a.chunks);
+  const size_t stride = size_t(gridDim.x) * (kPairBlock / 2);
+  const uint32_t lane = threadIdx.x & 63u;
+  // A wave takes 32 consecutive walks (a half word of packed bits); the last
+  // packed word's missing elements are 0.
+  const size_t end = kMode == SUFHIP_DCF_OUT_PACKED ? (walks + 63) / 64 * 64 : walks;
+  for (size_t base = (size_t(blockIdx.x) + size_t(gridDim.x) * (threadIdx.x >> 6)) * 32;
+       base < end; base += stride) {
+    const size_t w = base + (lane >> 1);
+    const bool in = w < walks;
+    const size_t wc = in ? w : walks - 1;  // whole lane pairs keep walking
+    const size_t e = wc / size_t(a.chunks);
+    const int c = int(wc - e * size_t(a.chunks));
+    const uint8_t* key = a.broadcast ? a.keys : a.keys + e * a.key_bytes;
+    const uint8_t* chunk = key + 8 + size_t(c) * chunk_bytes;
+    const bool more = size_t(c + 1) * chunk_bytes + 8 < a.key_bytes;
+    const U128 r =
+        pair_walk<kGroup>(aes, K, chunk, a.in_bits, a.xs[e], key[2] & 1u, more);
+    const bool mine = in && (lane & 1u);
+    if constexpr (kMode == SUFHIP_DCF_OUT_BIT) {
+      if (mine) static_cast<uint8_t*>(a.out)[e] = uint8_t(r.lo & 1u);
+    } else if constexpr (kMode == SUFHIP_DCF_OUT_PACKED) {
+      // Bit 2 g + 1 of the ballot is element g: the odd bits, gathered.
+      uint64_t b = (__ballot(mine && (r.lo & 1u)) >> 1) & 0x5555555555555555ull;
+      b = (b | b >> 1) & 0x3333333333333333ull;
+      b = (b | b >> 2) & 0x0f0f0f0f0f0f0f0full;
+      b = (b | b >> 4) & 0x00ff00ff00ff00ffull;
+      b = (b | b >> 8) & 0x0000ffff0000ffffull;
+      b = (b | b >> 16) & 0xffffffffull;
+      if (lane == 0) static_cast<uint32_t*>(a.out)[base >> 5] = uint32_t(b);
+    } else {
+      uint8_t* out = static_cast<uint8_t*>(a.out) + e * size_t(a.out_bytes) + 16 * c;
+      const int take = a.out_bytes - 16 * c < 16 ? a.out_bytes - 16 * c : 16;
+      if (mine)
+        for (int b = 0; b < take; ++b) out[b] = uint8_t((b < 8 ? r.lo : r.hi) >> (8 * (b & 7)));
+    }
+  }
+}
+
 // ---------------------------------------------------------------- keygen --
 
 struct DcfGenArgs {
@@ -305,38 +351,53 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
   const size_t walks = n * size_t(a.chunks);
   int cus = 0;
   if (int rc = cu_count(&cus)) return rc;
-  // 8 lanes per walk up to two full passes of them (256 walks per CU), one
-  // lane above: at 300, 32768 and 65536 keys of 64 levels 42, 77 and 140 us
-  // against 134, 138 and 155; at 131072, 276 against 205.  The quad walks are
-  // bound by their serial chain up to one pass and by VALU issue beyond.
-  const bool quad = walks <= 256 * size_t(cus);
-  // Waves of 64 elements, or of 8 quad walks, one workgroup per CU at most.
-  const size_t waves = quad ? (walks + 7) / 8 : (n + 63) / 64;
-  const dim3 grid(unsigned(waves < size_t(cus) ? waves : size_t(cus))), block(kDcfBitBlock);
-  if (out_mode != SUFHIP_DCF_OUT_BYTES) {
-    if (out_mode == SUFHIP_DCF_OUT_BIT) {
-      if (quad)
-        hipLaunchKernelGGL((dcf_eval_quad_bit_kernel<SUFHIP_DCF_OUT_BIT>), grid, block, 0, s, a);
-      else
-        hipLaunchKernelGGL((dcf_eval_bit_kernel<SUFHIP_DCF_OUT_BIT>), grid, block, 0, s, a);
-    } else {
-      SUFHIP_REQUIRE((reinterpret_cast<uintptr_t>(d_out) & 7) == 0,
-                     "sufhip_dcf_eval: packed output must be 8-byte aligned");
-      if (quad)
-        hipLaunchKernelGGL((dcf_eval_quad_bit_kernel<SUFHIP_DCF_OUT_PACKED>), grid, block, 0, s, a);
-      else
-        hipLaunchKernelGGL((dcf_eval_bit_kernel<SUFHIP_DCF_OUT_PACKED>), grid, block, 0, s, a);
-    }
-  } else {
-    if (quad && group == SUFHIP_GROUP_XOR)
-      hipLaunchKernelGGL((dcf_eval_quad_bytes_kernel<SUFHIP_GROUP_XOR>), grid, block, 0, s, a);
-    else if (quad)
-      hipLaunchKernelGGL((dcf_eval_quad_bytes_kernel<SUFHIP_GROUP_ADD>), grid, block, 0, s, a);
-    else if (group == SUFHIP_GROUP_XOR)
-      hipLaunchKernelGGL((dcf_eval_bytes_kernel<SUFHIP_GROUP_XOR>), grid, block, 0, s, a);
+  // Lanes per walk by walks per CU: 8 up to 160, 2 up to 320, then one.
+  // Bits of 64-level keys on 256 CUs, us with 8 / 2 / 1 lanes: 16384 walks 52 /
+  // 83 / 135, 32768 73 / 83 / 136, 40000 91 / 97 / 151, 50021 113 / 104 / 151,
+  // 65536 137 / 105 / 153, 80000 151 / 160 / 173, 131072 270 / 206 / 200,
+  // 262144 533 / 406 / 365.  Fewer lanes do less exchange per walk; more have
+  // a shorter serial chain.
+  const size_t full = size_t(cus);
+  const bool quad = walks <= 160 * full, pair = !quad && walks <= 320 * full;
+  // Waves of 64 elements, or of 8 or 32 walks, one workgroup per CU at most.
+  const size_t per = quad ? 8 : (pair ? 32 : 64);
+  const size_t waves = ((quad || pair ? walks : n) + per - 1) / per;
+  const dim3 grid(unsigned(waves < full ? waves : full));
+  const dim3 block(unsigned(pair ? kPairBlock : kDcfBitBlock));
+  const bool xor_group = group == SUFHIP_GROUP_XOR;
+  SUFHIP_REQUIRE(out_mode != SUFHIP_DCF_OUT_PACKED || (reinterpret_cast<uintptr_t>(d_out) & 7) == 0,
+                 "sufhip_dcf_eval: packed output must be 8-byte aligned");
+#define SUFHIP_DCF_LAUNCH(...) hipLaunchKernelGGL((__VA_ARGS__), grid, block, 0, s, a)
+  if (out_mode == SUFHIP_DCF_OUT_BIT) {
+    if (quad)
+      SUFHIP_DCF_LAUNCH(dcf_eval_quad_bit_kernel<SUFHIP_DCF_OUT_BIT>);
+    else if (pair)
+      SUFHIP_DCF_LAUNCH(dcf_eval_pair_kernel<SUFHIP_DCF_OUT_BIT, SUFHIP_GROUP_XOR>);
     else
-      hipLaunchKernelGGL((dcf_eval_bytes_kernel<SUFHIP_GROUP_ADD>), grid, block, 0, s, a);
+      SUFHIP_DCF_LAUNCH(dcf_eval_bit_kernel<SUFHIP_DCF_OUT_BIT>);
+  } else if (out_mode == SUFHIP_DCF_OUT_PACKED) {
+    if (quad)
+      SUFHIP_DCF_LAUNCH(dcf_eval_quad_bit_kernel<SUFHIP_DCF_OUT_PACKED>);
+    else if (pair)
+      SUFHIP_DCF_LAUNCH(dcf_eval_pair_kernel<SUFHIP_DCF_OUT_PACKED, SUFHIP_GROUP_XOR>);
+    else
+      SUFHIP_DCF_LAUNCH(dcf_eval_bit_kernel<SUFHIP_DCF_OUT_PACKED>);
+  } else if (xor_group) {
+    if (quad)
+      SUFHIP_DCF_LAUNCH(dcf_eval_quad_bytes_kernel<SUFHIP_GROUP_XOR>);
+    else if (pair)
+      SUFHIP_DCF_LAUNCH(dcf_eval_pair_kernel<SUFHIP_DCF_OUT_BYTES, SUFHIP_GROUP_XOR>);
+    else
+      SUFHIP_DCF_LAUNCH(dcf_eval_bytes_kernel<SUFHIP_GROUP_XOR>);
+  } else {
+    if (quad)
+      SUFHIP_DCF_LAUNCH(dcf_eval_quad_bytes_kernel<SUFHIP_GROUP_ADD>);
+    else if (pair)
+      SUFHIP_DCF_LAUNCH(dcf_eval_pair_kernel<SUFHIP_DCF_OUT_BYTES, SUFHIP_GROUP_ADD>);
+    else
+      SUFHIP_DCF_LAUNCH(dcf_eval_bytes_kernel<SUFHIP_GROUP_ADD>);
   }
+#undef SUFHIP_DCF_LAUNCH
   return check_launch("dcf_eval kernel");
 }
 

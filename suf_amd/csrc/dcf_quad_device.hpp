@@ -8,8 +8,8 @@
 // a lane here issues 4 table reads a round where the one-lane walk issues 32,
 // so the chain is 0.65 us a level against 2.1 us (measured at 300 to 8192
 // keys, one or two waves per SIMD).  The exchanges make it 36 VALU operations
-// per block and round instead of 28, so the one-lane walk keeps the batches
-// that fill the chip.
+// per block and round instead of 28, so larger batches take fewer lanes per
+// walk (two, at the end of this file, then one).
 //
 // A lane only ever needs one column of two keys, K_h and K_{2+h} (h its
 // half), so the round keys live in 22 registers: nothing but table reads goes
@@ -225,6 +225,98 @@ __device__ __forceinline__ U128 quad_finish(const uint8_t* chunk, int in_bits, u
       return gadd<kGroup>(st.v, sv);
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// The same walk on 2 lanes, for batches between the 8-lane walks' and a full
+// chip of one-lane walks: the even lane forms the next-seed block, the odd
+// lane the value block.  A lane's two keys K_h and K_{2+h} (h its parity) are
+// 88 registers, so nothing but table reads goes through the LDS, and 512
+// lanes per CU (two waves per SIMD) have the registers for them.
+constexpr int kPairBlock = 512;
+
+struct PairKeys {
+  uint32_t k[44], d[44];  // K_h and K_h ^ K_{2+h}
+};
+
+__device__ __forceinline__ PairKeys load_pair_keys(KeySelPtr sel) {
+  PairKeys K;
+  const uint32_t at = (threadIdx.x & 1u) * 8u;
+#pragma unroll
+  for (int r = 0; r < 11; ++r)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      K.k[4 * r + j] = sel[16 * r + at + j];
+      K.d[4 * r + j] = sel[16 * r + at + 4 + j];
+    }
+  return K;
+}
+
+// The even lane's value of each lane pair, in both.
+__device__ __forceinline__ uint32_t pair_even(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0xa0, 0xf, 0xf, true));
+}
+
+// Walk of one chunk by a lane pair; the odd lane returns the 16-byte share.
+template <int kGroup>
+__device__ __forceinline__ U128 pair_walk(const AesLds4& aes, const PairKeys& K,
+                                          const uint8_t* chunk, int in_bits, uint64_t x,
+                                          uint32_t party, bool more_after) {
+  uint32_t s[4];
+  load16_bytes(chunk, true, s);
+  s[3] &= 0x7fffffffu;
+  uint32_t t = party;
+  U128 v{0, 0};
+  const uint8_t* cw = chunk + 16;
+#pragma unroll 1
+  for (int i = 0; i < in_bits; ++i, cw += 33) {
+    const CwRawFull cr = load_cw_raw_full(cw);
+    const uint32_t xi = uint32_t(x >> (in_bits - 1 - i)) & 1u;
+    const uint32_t m = 0u - xi;
+    uint32_t a[4], o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = xor_and(s[j], m, K.d[j]) ^ K.k[j];
+#pragma unroll
+    for (int r = 1; r < 10; ++r) {
+      uint32_t ad[16], tv[16];
+#pragma unroll
+      for (int n = 0; n < 16; ++n)
+        ad[n] = __builtin_amdgcn_perm(a[((n >> 2) + n) & 3], aes.base[n & 3], AesLds4::sel(n & 3));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < 16; ++n) tv[n] = lds_word(aes.lds, ad[n]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        a[c] = xor_and(SUFHIP_BITOP3(SUFHIP_BITOP3(tv[4 * c], tv[4 * c + 1], tv[4 * c + 2], 0x96),
+                                     tv[4 * c + 3], K.k[4 * r + c], 0x96),
+                       m, K.d[4 * r + c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      o[c] = xor_and(aes.last_col(a[c], a[(c + 1) & 3], a[(c + 2) & 3], a[(c + 3) & 3],
+                                  K.k[40 + c] ^ s[c]),
+                     m, K.d[40 + c]);
+    const CwFull c = decode_cw_full(cr);
+    const uint32_t tmask = 0u - t;
+    // The odd lane's value; the even lane's v is not used.
+    U128 vd = mk(o[0], o[1], o[2], o[3] & 0x7fffffffu);
+    if (t) vd = gadd<kGroup>(vd, mk(c.v[0], c.v[1], c.v[2], c.v[3]));
+    if (party) vd = gneg<kGroup>(vd);
+    v = gadd<kGroup>(v, vd);
+    // The even lane's next seed and control bit, to both.
+    uint32_t tn = (o[3] >> 31) ^ ((xi ? c.tb : (c.tb >> 1)) & t & 1u);
+    o[3] &= 0x7fffffffu;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] = pair_even(o[j] ^ (c.s[j] & tmask));
+    t = pair_even(tn);
+  }
+  uint32_t np1[4];
+  load16_bytes(cw, more_after, np1);
+  U128 sv = mk(s[0], s[1], s[2], s[3]);
+  if (t) sv = gadd<kGroup>(sv, mk(np1[0], np1[1], np1[2], np1[3]));
+  if (party) sv = gneg<kGroup>(sv);
+  return gadd<kGroup>(v, sv);
 }
 
 }  // namespace

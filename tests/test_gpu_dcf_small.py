@@ -1,7 +1,6 @@
-"""Small DCF batches on the GPU (8 lanes per walk up to 256 walks per CU, one
-lane per walk above): shares equal the oracle's at the edges of a wave's
-octet of walks, of one pass of the chip and of the rule that picks the
-kernel."""
+"""Small DCF batches on the GPU (8 lanes per walk up to 160 walks per CU, two
+up to 320, one above): shares equal the oracle's at the edges of a wave's
+walks, of one pass of the chip and of the rule that picks the kernel."""
 import numpy as np
 import pytest
 import torch
@@ -13,7 +12,7 @@ from suf_amd import native, pfss
 pytestmark = pytest.mark.gpu
 
 CUS = 256
-LIMIT = 256 * CUS  # the largest batch of quad walks on 256 CUs
+QUAD, PAIR = 160 * CUS, 320 * CUS  # the largest batches of 8-lane and 2-lane walks
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -23,8 +22,10 @@ def _init():
 
 @pytest.mark.parametrize("n,in_bits,plen,group", [
     (1, 64, 1, 0), (7, 1, 1, 1), (8, 13, 16, 1), (9, 64, 20, 0), (65, 32, 8, 1), (511, 37, 40, 1),
-    (128 * CUS + 1, 9, 8, 1), (LIMIT // 2 - 3, 8, 20, 0), (LIMIT, 8, 1, 0), (LIMIT + 1, 8, 8, 1),
-    (LIMIT + 64 * 7 + 5, 11, 1, 0)])
+(128 * CUS + 1, 9, 8, 1), (QUAD // 2 - 3, 8, 20, 0), (QUAD, 8, 1, 0), (QUAD + 1, 8, 8, 1),
+    (QUAD + 31, 11, 5, 0), (256 * CUS - 1, 7, 1, 1), (256 * CUS + 33, 10, 16, 0),
+    (QUAD // 2 + 1, 6, 33, 1), (PAIR, 9, 1, 0), (PAIR + 1, 8, 8, 1),
+    (PAIR + 64 * 7 + 5, 11, 1, 0)])
 @pytest.mark.parametrize("broadcast", [False, True])
 def test_small_batches_match_oracle(n, in_bits, plen, group, broadcast):
     say("dcf small n=%d in_bits=%d plen=%d group=%d bcast=%d" % (n, in_bits, plen, group, broadcast))

@@ -586,15 +586,5 @@ int cu_count(int* cus) {
   return SUFHIP_OK;
 }
 
-// Grid for the grid-stride DCF kernels: one workgroup per CU (LDS-limited),
-// never more workgroups than the batch needs.
-int dcf_grid(size_t n, unsigned int* grid, int block = kDcfBlock) {
-  int cus = 0;
-  if (int rc = cu_count(&cus)) return rc;
-  const size_t need = (n + size_t(block) - 1) / size_t(block);
-  *grid = static_cast<unsigned int>(need < size_t(cus) ? need : size_t(cus));
-  return SUFHIP_OK;
-}
-
 }  // namespace
 }  // namespace sufhip

@@ -3,7 +3,7 @@
 //
 // Lanes 0-3 of a group compute the next-seed block AES_{K_{2b}}(s) and lanes
 // 4-7 the value block AES_{K_{2b+1}}(s), one state column per lane
-// (AesLds4::encrypt_quad_n's scheme).  A level is bounded by its serial
+// (AesLds4::quad_terms' scheme).  A level is bounded by its serial
 // chain -- ten rounds of table address, LDS read, three quad exchanges -- and
 // a lane here issues 4 table reads a round where the one-lane walk issues 32,
 // so the chain is 0.65 us a level against 2.1 us (measured at 300 to 8192

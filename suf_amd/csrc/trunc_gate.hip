@@ -17,7 +17,7 @@
 // the first d levels depends only on the top d bits of x^_low, so for a
 // broadcast key and a large batch the 2^d frontier states are computed once
 // and every element continues from its prefix.  The first k0 = min(d, 12)
-// levels are walked one node per lane; deeper levels are expanded
+// levels are walked 8 lanes to a node; deeper levels are expanded
 // breadth-first, one child per lane (2 AES per node).  For f <= 14, d = f:
 // the frontier holds the final share of every point of the domain and an
 // element's carry is a single table read (the key-only work, 2^f walks, is

@@ -97,7 +97,7 @@ __device__ __forceinline__ int batch_job(const uint32_t (&begin)[kJobs + 1], int
 
 // One walk per 8 lanes.  Lanes 0-3 of the group compute the next-seed block
 // AES_{K_{2b}}(s) and lanes 4-7 the value block AES_{K_{2b+1}}(s), column-
-// parallel (encrypt_quad_n of the AES table type): lane q of either half
+// parallel (quad_encrypt_n over the AES table type): lane q of either half
 // holds word q of the seed.  A level is then about a quarter of the dependent
 // issue time of the one-lane walk (add64_walk), which bounds these
 // latency-bound launches.

@@ -531,13 +531,13 @@ __global__ void __launch_bounds__(128 * kKW, 1) beaver_bal_kernel(Bm2Args a) {
     for (int r = 0; r < 16; ++r) acc[s][r] = 0;
   // Operand pairs u = 2 step + (0: (L_p, E), 1: (D, B_p)); this wave's are
   // [u0, u1).  The loop runs over whole groups of kStages pairs; loads past
-  // the last pair repeat it (in bounds) and their MFMAs are skipped.
+  // the last pair repeat it (in bounds) and their MFMAs are skipped.  Without
+  // pairs (K = 0: the planes hold nothing) nothing is loaded.
   const int U = 2 * (K / 32);
   const int u0 = U * kh / kKW, u1 = U * (kh + 1) / kKW;
   v4i L[kStages][kDigitPlanes], R[kStages][kDigitPlanes];
   auto issue = [&](int q, int u) {
     u = u < u1 ? u : u1 - 1;
-    u = u > 0 ? u : 0;
     const uint32_t st = uint32_t(u >> 1);
     const int8_t* lb = (u & 1) ? Ld : Lx;
     const int8_t* rb = (u & 1) ? Rb : Re;
@@ -547,8 +547,10 @@ __global__ void __launch_bounds__(128 * kKW, 1) beaver_bal_kernel(Bm2Args a) {
       R[q][i] = load16(rb + (i * rplane + st * rstep) + fo);
     }
   };
+  if (u0 < u1) {
 #pragma unroll
-  for (int q = 0; q < kStages - 1; ++q) issue(q, u0 + q);
+    for (int q = 0; q < kStages - 1; ++q) issue(q, u0 + q);
+  }
   for (int v0 = u0; v0 < u1; v0 += kStages) {
 #pragma unroll
     for (int h = 0; h < kStages; ++h) {

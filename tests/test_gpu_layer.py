@@ -423,6 +423,28 @@ def test_beaver_balanced_form_equals_three_product_form(b, M, K, N):
                 assert np.array_equal(outs[0][p][i].ravel(), np.asarray(o).ravel()), (i, p)
 
 
+@pytest.mark.parametrize("M,N,vm,vn", [(32, 64, 0, 0), (64, 32, 33, 31)])
+def test_beaver_balanced_form_without_k(M, N, vm, vn):
+    """An empty k extent: the shares are C's, and the planes, which hold no
+    byte, are not read."""
+    say("beaver balanced form K=0 %dx%d" % (M, N))
+    rows, cols = (vm or M), (vn or N)
+    g = np.random.default_rng(M)
+    C = [g.integers(0, 2**64, rows * cols, dtype=np.uint64) for _ in range(2)]
+    Cd = [dev(c) for c in C]
+    planes = torch.zeros(1 << 14, dtype=torch.int64, device="cuda")  # covers every look-ahead load
+    a = native.BeaverMfma2Args()
+    a.Dp = a.Ep = a.Xp = planes.data_ptr()
+    out = [torch.full((rows * cols + 1,), 5, dtype=torch.int64, device="cuda") for _ in range(2)]
+    for p in (0, 1):
+        a.Ap[p] = a.Bp[p] = planes.data_ptr()
+        a.C[p], a.out[p] = Cd[p].data_ptr(), out[p].data_ptr()
+    a.batches, a.M, a.K, a.N, a.valid_m, a.valid_n = 1, M, 0, N, vm, vn
+    native.call("sufhip_beaver_matmul2_mfma_ex", native.ctypes.byref(a), 0)
+    for p in (0, 1):
+        assert np.array_equal(u64(out[p])[:-1], C[p]) and int(out[p][-1]) == 5
+
+
 @pytest.mark.parametrize("shape", [(1, 64, 96, 1), (2, 32, 64, 1), (1, 96, 64, 0)])
 def test_split_planes_a0_are_planes_of_value_plus_a0(shape):
     """planes_a0 of a split and of an open-split job are the planes of the

@@ -302,8 +302,14 @@ constexpr int kBatchJobs = 32;
 // Up to 768 lanes per workgroup (one per CU: 128 KB of AES tables): the walk's
 // 8 lanes per node cover a batch in one round (plan_walk), and three waves
 // per SIMD leave the lanes the registers for their round keys and the
-// expansion's lockstep groups.
+// expansion's lockstep groups.  Batches that take fewer rounds of 1024 lanes
+// run those, with the local levels depth first (walk8_descend: the lockstep
+// groups need more than 1024 lanes' 128 registers).  Us for both parties'
+// gates with 768 / 1024 lanes: 30 gates of 13 bits (960 lanes per CU) 73 /
+// 49, 64 of 14 bits 215 / 182, 4 of 16 bits (1024 lanes per CU, no local
+// levels) 33 / 23, 64 of 16 bits 308 / 269.
 constexpr int kWalkBlock = 768;
+constexpr int kWalkWideBlock = 1024;
 
 using WalkArgs = WalkJobs<kWalkJobs>;
 
@@ -321,7 +327,8 @@ struct BatchLevelArgs {
 static_assert(sizeof(WalkArgs) <= 4096 && sizeof(BatchLevelArgs) <= 4096,
               "kernel argument blocks must fit in 4 KB");
 
-__global__ void __launch_bounds__(kWalkBlock) trunc_batch_walk_kernel(WalkArgs a) {
+template <int kBlock>
+__global__ void __launch_bounds__(kBlock) trunc_batch_walk_kernel(WalkArgs a) {
   // The walk's job, key header and seed are loaded under the tables' staging.
   const uint32_t gl = blockIdx.x * uint32_t(a.lanes) + threadIdx.x;
   const uint32_t total = a.begin[a.count];
@@ -339,8 +346,6 @@ __global__ void __launch_bounds__(kWalkBlock) trunc_batch_walk_kernel(WalkArgs a
   const QuadKeys keys = load_quad_keys(a.prg);
   SUFHIP_DCF_TABLE_SETUP();
   if (!mine || !(flags & 1)) return;  // whole 8-lane groups leave together
-  // The body stays in the kernel: passed through a helper function, the same
-  // steps spill at the 1024-lane register limit.
   const Walk8Ctx<DcfAes> c{aes,   keys,           chunk,   a.out[j], f,
                            party, (gl >> 2) & 1u, gl & 3u, last};
   const int dw = d - e;  // depth walked before the local expansion
@@ -357,15 +362,27 @@ __global__ void __launch_bounds__(kWalkBlock) trunc_batch_walk_kernel(WalkArgs a
     w = n[0];
   }
   if (e > 0) {
-    const Walk8 root[1] = {w};
-    if (e == 1)
-      walk8_expand<0, 1>(c, cw, root, v);
-    else if (e == 2)
-      walk8_expand<0, 2>(c, cw, root, v);
-    else if (e == 3)
-      walk8_expand<0, 3>(c, cw, root, v);
-    else  // e == 4: the host picks e <= kWalkLocal <= 4 (static_assert above)
-      walk8_expand<0, 4>(c, cw, root, v);
+    // e <= kWalkLocal <= 4 (static_assert above)
+    if constexpr (kBlock > kWalkBlock) {
+      if (e == 1)
+        walk8_descend<1>(c, cw, w, v);
+      else if (e == 2)
+        walk8_descend<2>(c, cw, w, v);
+      else if (e == 3)
+        walk8_descend<3>(c, cw, w, v);
+      else
+        walk8_descend<4>(c, cw, w, v);
+    } else {
+      const Walk8 root[1] = {w};
+      if (e == 1)
+        walk8_expand<0, 1>(c, cw, root, v);
+      else if (e == 2)
+        walk8_expand<0, 2>(c, cw, root, v);
+      else if (e == 3)
+        walk8_expand<0, 3>(c, cw, root, v);
+      else
+        walk8_expand<0, 4>(c, cw, root, v);
+    }
   } else if (d == f) {
     walk8_leaf(c, w, v);
   } else {
@@ -422,14 +439,19 @@ int spread_grid(size_t count, unsigned int* grid, unsigned int* block) {
 }
 
 // Launch shape for the batched walk (8 lanes per walk, no grid stride): the
-// lanes spread over every CU, 128..kWalkBlock walk lanes per workgroup, in
+// lanes spread over every CU, 128 walk lanes per workgroup at least and
+// kWalkBlock at most -- kWalkWideBlock where that takes fewer rounds -- in
 // workgroups of 512 threads at least (all of them stage the AES tables).
 int walk_grid(size_t count, unsigned int* grid, unsigned int* block, int* lanes) {
   int cus = 0;
   if (int rc = cu_count(&cus)) return rc;
-  size_t per = (count + size_t(cus) - 1) / size_t(cus);
+  const auto rounds = [&](size_t b) { return (count + b * size_t(cus) - 1) / (b * size_t(cus)); };
+  const size_t cap =
+      rounds(kWalkWideBlock) < rounds(kWalkBlock) ? size_t(kWalkWideBlock) : size_t(kWalkBlock);
+  const size_t share = rounds(cap) * size_t(cus);
+  size_t per = (count + share - 1) / share;
   per = (per + 63) / 64 * 64;
-  const size_t b = per < 128 ? 128 : (per > size_t(kWalkBlock) ? size_t(kWalkBlock) : per);
+  const size_t b = per < 128 ? 128 : per;
   *lanes = int(b);
   *block = unsigned(b < 512 ? 512 : b);
   *grid = unsigned((count + b - 1) / b);
@@ -528,9 +550,9 @@ int plan_walk(const uint8_t* prg_state, const sufhip_trunc_job* jobs, int m, con
   // Local levels of the full-domain walks: a walk level costs about as
   // much as one lockstep group of the expansion, so the walks go as deep as
   // the lanes allow -- the fewest local levels whose walks take less than
-  // one full workgroup per CU (at most kWalkLocal; with 1024 lanes per
-  // workgroup the extra waves per SIMD slowed every level more than a local
-  // level costs).  A hosted walk (lanes_cap > 0) takes the fewest whose walks fit
+  // one workgroup of kWalkBlock lanes per CU (at most kWalkLocal; the extra
+  // waves per SIMD of kWalkWideBlock slow every level more than a local level
+  // costs).  A hosted walk (lanes_cap > 0) takes the fewest whose walks fit
   // in the host's room.
   int cus = 0;
   if (int rc = cu_count(&cus)) return rc;
@@ -803,7 +825,10 @@ int sufhip_trunc_prepare_batch(const uint8_t* prg_state, const sufhip_trunc_job*
     if (wa.begin[m] > 0) {
       unsigned int g = 0, b = 0;
       if (int rc = walk_grid(8 * size_t(wa.begin[m]), &g, &b, &wa.lanes)) return rc;
-      hipLaunchKernelGGL(trunc_batch_walk_kernel, dim3(g), dim3(b), 0, s, wa);
+      if (b > unsigned(kWalkBlock))
+        hipLaunchKernelGGL(trunc_batch_walk_kernel<kWalkWideBlock>, dim3(g), dim3(b), 0, s, wa);
+      else
+        hipLaunchKernelGGL(trunc_batch_walk_kernel<kWalkBlock>, dim3(g), dim3(b), 0, s, wa);
       if (int rc = check_launch("trunc_batch_walk_kernel")) return rc;
     }
     for (int level = kWalkFrontierBits; level < maxd; ++level) {

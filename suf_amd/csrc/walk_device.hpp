@@ -206,6 +206,22 @@ __device__ __forceinline__ void walk8_expand(const Ctx& c, const uint8_t* cw,
   }
 }
 
+// The same subtree depth first, a node's two children in lockstep: one state
+// per level is held instead of a level's, for workgroups of 1024 lanes (128
+// registers).
+template <int E, class Ctx>
+__device__ __forceinline__ void walk8_descend(const Ctx& c, const uint8_t* cw, const Walk8& w,
+                                              uint32_t v) {
+  if constexpr (E == 0) {
+    walk8_leaf(c, w, v);
+  } else {
+    Walk8 kid[2];
+    walk8_step_n<2>(c, cw, 0, &w, kid);
+    walk8_descend<E - 1>(c, cw + 33, kid[0], 2 * v);
+    walk8_descend<E - 1>(c, cw + 33, kid[1], 2 * v + 1);
+  }
+}
+
 // Lane gl's walk of every level: table entry v of the job with key `key`,
 // table `out` and geometry `geo` (WalkJobs::geo, d = f and no local levels,
 // as trunc_walk_plan gives).  The caller finds the job of lane gl (batch_job)
@@ -238,9 +254,8 @@ __device__ __forceinline__ void walk_leaf_path(const Aes& aes, const QuadKeys& k
 // Lane gl's walk of a table job with e = geo >> 16 local levels (0..4): the
 // depth-(f - e) node v, then its subtree's 2^e table entries (v << e) + i,
 // as trunc_batch_walk_kernel walks table jobs.  For kernels that run these
-// walks as a role beside their own work, at 512 lanes per workgroup or
-// fewer (the expansion's lockstep groups need more than the 128 registers
-// of a 1024-lane workgroup when passed through this function).
+// walks as a role beside their own work, at 512 lanes per workgroup or fewer
+// (walk8_expand's lockstep groups take about 150 registers).
 template <class Aes>
 __device__ __forceinline__ void walk_table(const Aes& aes, const QuadKeys& keys, const uint8_t* key,
                                            uint4* out, uint32_t geo, uint32_t v, uint32_t gl) {

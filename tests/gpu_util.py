@@ -42,3 +42,19 @@ class Pins:
         t = a if isinstance(a, torch.Tensor) else dev(a)
         self.held.append(t)
         return t.data_ptr()
+
+
+def best_us(fn, reps=10, tries=12):
+    """Shortest time of fn() in microseconds: the best of `tries` runs of
+    `reps` calls in a captured graph (no host time between them)."""
+    from suf_amd import tasks
+    graph = tasks.capture(lambda: [fn() for _ in range(reps)])
+    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    best = float("inf")
+    for _ in range(tries):
+        a.record()
+        graph.replay()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / reps)
+    return best

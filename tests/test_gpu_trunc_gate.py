@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle_lib as ol
-from gpu_util import dev, host, say, u64
+from gpu_util import best_us, dev, host, say, u64
 from suf_amd import native, pfss
 
 pytestmark = pytest.mark.gpu
@@ -164,7 +164,7 @@ def test_batched_prepare_matches_single_gate_path():
 @pytest.mark.parametrize("gates", [2, 4, 8, 16, 40])
 def test_batched_prepare_every_local_depth(gates):
     """One walk launch expands E local levels, the fewest whose walks take
-    less than three quarters of one full workgroup per CU: with f = 12 tables
+    less than one workgroup of 768 lanes per CU: with f = 12 tables
     (two per gate) and 256 CUs, 2 / 4 / 8 / 16 / 40 gates give E = 0 / 1 / 2
     / 3 / 4.  Every gate's shares equal the one-gate path's."""
     from suf_amd import tasks
@@ -181,3 +181,45 @@ def test_batched_prepare_every_local_depth(gates):
         for p in (0, 1):
             want = u64(pfss.trunc_eval(g.kind, g.f, STATE, g.keys[p], xd))
             assert np.array_equal(u64(out[p]), want), (gates, i, p)
+
+
+@pytest.mark.parametrize("gates,f", [(16, 4), (29, 13), (30, 13), (15, 14), (30, 14), (3, 16),
+                                     (4, 16), (9, 16)])
+def test_batched_prepare_wide_launches(gates, f):
+    """Batches on either side of one round of 768 and of 1024 lanes per CU,
+    with and without local levels: both parties' shares reconstruct x >> f at
+    every low-bit pattern (up to 2^14 of them), and equal the oracle's."""
+    from suf_amd import tasks
+    dealer = tasks.Dealer(7 * gates + f)
+    n = 1 << min(f, 14)
+    gs = [tasks.Trunc(dealer, f, n, STATE) for _ in range(gates)]
+    say("batched prepare, %d gates (f = %d)" % (gates, f))
+    for g in gs:
+        for w in g.work:
+            w.fill_(-1)
+    tasks.prepare_batch(gs)
+    x = np.arange(n, dtype=np.int64) - n // 2
+    picked = np.arange(0, n, max(1, n // 13))
+    for i, g in enumerate(gs):
+        xhat = x.view(np.uint64) + np.uint64(g.mask)
+        out = tuple(torch.empty(n, dtype=torch.int64, device="cuda") for _ in range(2))
+        g.finish(dev(xhat), out)
+        assert np.array_equal(host(out[0] + out[1]), x >> f), i
+        if i in (0, gates - 1):
+            for p in (0, 1):
+                ref = ol.trunc_eval(PRG, g.kind, f, host(g.keys[p]), xhat[picked])
+                assert np.array_equal(u64(out[p])[picked], ref), (i, p)
+
+
+def test_batched_prepare_past_one_round_of_768_lanes():
+    """A batch of 960 lanes per CU (15 gates of 14 bits: 30 tables of 2^10
+    walks) costs about what one of 768 (12 gates) does, not two rounds of it
+    (1.75 times)."""
+    from suf_amd import tasks
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the gate counts are those of 256 CUs")
+    dealer = tasks.Dealer(5)
+    gs = [tasks.Trunc(dealer, 14, 64, STATE) for _ in range(15)]
+    us = {m: best_us(lambda: tasks.prepare_batch(gs[:m])) for m in (11, 15)}
+    say("prepare of 11 / 15 gates: %s us" % us)
+    assert us[15] < 1.5 * us[11]

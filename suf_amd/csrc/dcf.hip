@@ -13,8 +13,9 @@
 // only on bit 0 of the terms, and bit 0 of -v equals bit 0 of v, so this
 // holds for both output groups.
 //
-// Batches of more than 320 keys per CU: one element per lane; each lane streams its own key front to back
-// (33 bytes per level), so successive levels hit the same cache lines.
+// Batches of more than 384 walks per CU: one walk per lane, a walk being one
+// 16-byte chunk of one element's payload; each lane streams its own key front
+// to back (33 bytes per level), so successive levels hit the same cache lines.
 //
 // The evaluation kernels run 1024 lanes per CU (four waves per SIMD): their
 // walks keep the round keys in scalar registers and fit in the 128 VGPRs
@@ -48,12 +49,12 @@ struct DcfEvalArgs {
 
 constexpr int kDcfBitBlock = 1024;
 
-// First element of this wave in the pass that starts at `pass`.  A full pass
-// gives each workgroup 1024 neighbouring keys; the last one deals its
-// elements out 64 at a time, so that what does not fill the chip spreads over
-// every CU (50021 keys of 32 levels: 182 -> 90 us) instead of filling the
-// first ones.  Dealing the full passes out too made 2^20 keys 4% slower (the
-// keys in flight on a CU then span the whole 2 GB).
+// First walk of this wave in the pass that starts at `pass`.  A full pass
+// gives each workgroup 1024 neighbouring keys; the last one deals its walks
+// out 64 at a time, so that what does not fill the chip spreads over every CU
+// (100000 keys of 64 levels: 318 -> 184 us) instead of filling the first ones.
+// Dealing the full passes out too made 2^20 keys 4% slower (the keys in flight
+// on a CU then span the whole 2 GB).
 __device__ __forceinline__ size_t wave_base(size_t pass, size_t n) {
   const size_t wave = threadIdx.x >> 6;
   return n - pass >= size_t(gridDim.x) * kDcfBitBlock
@@ -86,30 +87,29 @@ __global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_bit_kernel(DcfEvalArgs 
   }
 }
 
+// A lane that ran an element's chunks in turn left the chip to few elements of
+// many chunks: 1562 of 64 chunks of 16 levels took 2431 us, 58 this way.
 template <int kGroup>
 __global__ void __launch_bounds__(kDcfBitBlock) dcf_eval_bytes_kernel(DcfEvalArgs a) {
   SUFHIP_DCF_TABLE_SETUP();
   const KeySelPtr keys = kernarg_key_sel(offsetof(DcfEvalArgs, key_sel));
   const size_t stride = size_t(gridDim.x) * kDcfBitBlock;
   const size_t chunk_bytes = 32 + 33 * size_t(a.in_bits);
-  for (size_t pass = 0; pass < a.n; pass += stride) {
-    const size_t e = wave_base(pass, a.n) + (threadIdx.x & 63);
-    if (e >= a.n) continue;
+  const size_t walks = a.n * size_t(a.chunks);
+  for (size_t pass = 0; pass < walks; pass += stride) {
+    const size_t w = wave_base(pass, walks) + (threadIdx.x & 63);
+    if (w >= walks) continue;
+    const size_t e = w / size_t(a.chunks);
+    const int c = int(w - e * size_t(a.chunks));
     const uint8_t* key = a.broadcast ? a.keys : a.keys + e * a.key_bytes;
-    const uint32_t party = key[2] & 1u;
     uint64_t x = a.xs[e];
     if (a.in_bits < 64) x &= (uint64_t(1) << a.in_bits) - 1;
-    uint8_t* out = static_cast<uint8_t*>(a.out) + e * size_t(a.out_bytes);
-    for (int c = 0; c < a.chunks; ++c) {
-      const bool more = (c + 1) * chunk_bytes + 8 < a.key_bytes;
-      U128 r = walk_full<kGroup>(aes, keys, key + 8 + c * chunk_bytes, a.in_bits, x, party, more);
-      const int base = 16 * c;
-      const int take = a.out_bytes - base < 16 ? a.out_bytes - base : 16;
-      for (int b = 0; b < take; ++b) {
-        const uint64_t word = b < 8 ? r.lo : r.hi;
-        out[base + b] = uint8_t(word >> (8 * (b & 7)));
-      }
-    }
+    const bool more = size_t(c + 1) * chunk_bytes + 8 < a.key_bytes;
+    const U128 r = walk_full<kGroup>(aes, keys, key + 8 + size_t(c) * chunk_bytes, a.in_bits, x,
+                                     key[2] & 1u, more);
+    uint8_t* out = static_cast<uint8_t*>(a.out) + e * size_t(a.out_bytes) + 16 * c;
+    const int take = a.out_bytes - 16 * c < 16 ? a.out_bytes - 16 * c : 16;
+    for (int b = 0; b < take; ++b) out[b] = uint8_t((b < 8 ? r.lo : r.hi) >> (8 * (b & 7)));
   }
 }
 
@@ -351,17 +351,30 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
   const size_t walks = n * size_t(a.chunks);
   int cus = 0;
   if (int rc = cu_count(&cus)) return rc;
-  // Lanes per walk by walks per CU: 8 up to 160, 2 up to 320, then one.
-  // Bits of 64-level keys on 256 CUs, us with 8 / 2 / 1 lanes: 16384 walks 52 /
-  // 83 / 135, 32768 73 / 83 / 136, 40000 91 / 97 / 151, 50021 113 / 104 / 151,
-  // 65536 137 / 105 / 153, 80000 151 / 160 / 173, 131072 270 / 206 / 200,
-  // 262144 533 / 406 / 365.  Fewer lanes do less exchange per walk; more have
-  // a shorter serial chain.
+  // Lanes per walk by walks per CU: 8 up to 160, 2 up to 384, then one; bits
+  // take 8 lanes again from 256 to 320.  Fewer lanes do less exchange per
+  // walk, more have a shorter serial chain; a full pass is 128, 256 or 1024
+  // walks per CU, and just past one the next is as long.  Us on 256 CUs of
+  // 64-level keys with 8 / 2 / 1 lanes, bits and 8-byte additive shares:
+  //    40000 walks   88 /  93 / 151     93 / 100 / 168
+  //    50021        108 / 100 / 152    125 / 107 / 172
+  //    65536        132 / 101 / 154    152 / 108 / 184
+  //    65600        138 / 151 / 168    161 / 160 / 186
+  //    80000        150 / 156 / 174    174 / 168 / 191
+  //    98304        196 / 158 / 173    226 / 168 / 186
+  //   110000        215 / 192 / 185    249 / 205 / 206
+  //   131072        271 / 200 / 187    302 / 211 / 210
+  // 16-byte shares, payloads of 2 and 64 chunks (a walk is one chunk) and 16-
+  // and 32-level keys give the same choice; XOR byte shares lie between the
+  // columns (the choice costs them 4% at most).
   const size_t full = size_t(cus);
-  const bool quad = walks <= 160 * full, pair = !quad && walks <= 320 * full;
-  // Waves of 64 elements, or of 8 or 32 walks, one workgroup per CU at most.
+  const bool bytes = out_mode == SUFHIP_DCF_OUT_BYTES;
+  const bool quad =
+      walks <= 160 * full || (!bytes && walks > 256 * full && walks <= 320 * full);
+  const bool pair = !quad && walks <= 384 * full;
+  // Waves of 64, 8 or 32 walks, one workgroup per CU at most.
   const size_t per = quad ? 8 : (pair ? 32 : 64);
-  const size_t waves = ((quad || pair ? walks : n) + per - 1) / per;
+  const size_t waves = (walks + per - 1) / per;
   const dim3 grid(unsigned(waves < full ? waves : full));
   const dim3 block(unsigned(pair ? kPairBlock : kDcfBitBlock));
   const bool xor_group = group == SUFHIP_GROUP_XOR;

@@ -48,6 +48,38 @@ def mfma_ok(M, K, N):
     return M % 32 == 0 and N % 64 == 0 and K % 32 == 0 and K <= 8191
 
 
+def padded_form(M, K, N):
+    """The two-party matrix-core form, its extents padded to multiples of 32
+    with zero digits, for this product: whole extents always, others while the
+    padding costs less than the launches that the form saves (about 40 us).
+
+    Its time is the padded outputs' tiles, whatever of them is wanted: 20 us
+    and 19 ns for a tile of 32 x 32.  The launch-per-step form's is the
+    extents themselves, and under 24 of k it moves little for each output.
+    So thin products (few columns or rows of many, a short k) keep that form
+    past 5/2 million padding outputs, or 13/2 million from 12 of k on (from 16
+    on only if they are most of the outputs); their planes would also take up
+    to 32 times the shares' memory.  Us, padded / by steps:
+      65536 x 1 x 1      54 / 65     131072 x 12 x 1   103 / 126
+      131072 x 1 x 1     89 / 83     8 x 12 x 131072    89 / 102
+      1 x 1 x 131072     86 / 65     8 x 16 x 524288   366 / 307
+      2^20 x 1 x 1      707 / 346    524288 x 16 x 8   458 / 455
+      1500 x 1 x 2500    90 / 122    524288 x 24 x 8   540 / 640
+      31 x 1 x 524288   390 / 472    8 x 24 x 524288   400 / 416
+      524288 x 1 x 8    380 / 245    2^20 x 16 x 16    949 / 1097"""
+    if min(M, K, N) < 1:
+        return False
+    Mp, Kp, Np = (-(-v // 32) * 32 for v in (M, K, N))
+    if Kp > 4096:
+        return False
+    if (Mp, Kp, Np) == (M, K, N):
+        return True
+    if 8 * Kp * max(Mp, Np) >= 1 << 32 or Mp // 32 > 65535:  # plane offsets, tile rows
+        return False
+    return (K >= 24 or Mp * Np - M * N <= (5 if K < 12 else 13) << 19 or
+            (K >= 16 and 2 * M * N >= Mp * Np))
+
+
 class BeaverMatmulTrunc:
     """Dealer material (triples, truncation keys) for Y = trunc_f(X W), both
     parties.  Randomness: std::mt19937_64(seed) streams."""
@@ -81,11 +113,7 @@ class BeaverMatmulTrunc:
         # the truncation folded in, the triple shares' digit planes made here.
         # The launch-per-step form's buffers (u64 opens, products, masked open,
         # truncation workspaces) exist only when it is the form in use.
-        # Extents that are no multiple of 32 are padded with zero digits.
-        Mp, Kp, Np = (-(-v // 32) * 32 for v in (M, K, N))
-        whole = (Mp, Kp, Np) == (M, K, N)
-        self.fused = (use_mfma and Kp <= 4096 and frac_bits <= 13 and min(M, K, N) > 0 and
-                      (whole or 8 * Kp * max(Mp, Np) < 1 << 32))
+        self.fused = use_mfma and frac_bits <= 13 and padded_form(M, K, N)
         self.mm_work = None
         if not self.fused:
             self.work_bytes = lib.sufhip_trunc_work_bytes(frac_bits, M * N)
@@ -102,7 +130,7 @@ class BeaverMatmulTrunc:
         else:
             from . import layer, tasks
             self.tr = tasks.Trunc(None, frac_bits, M * N, self.prg_state, rnd=rnd)
-            self.padded = (Mp, Kp, Np)
+            self.padded = Mp, Kp, Np = tuple(-(-v // 32) * 32 for v in (M, K, N))
             self.Ap = tuple(layer.kb_planes(1, Mp, Kp) for _ in range(2))
             self.Bp = tuple(layer.kb_planes(1, Kp, Np) for _ in range(2))
             self.Dp, self.Ep = layer.kb_planes(1, Mp, Kp), layer.kb_planes(1, Kp, Np)

@@ -80,3 +80,30 @@ def test_bad_extents_are_refused():
         job[0].valid_rows, job[0].valid_cols, job[0].a_stride[2] = vr, vc, stride
         with pytest.raises(native.SufHipError):
             native.call("sufhip_kb_open_split_batch", job, 1, None)
+
+
+@pytest.mark.parametrize("M,K,N", [(1 << 18, 1, 1), (2, 11, 90000), (300000, 16, 3)])
+def test_thin_gate_keeps_the_step_form(M, K, N):
+    """Products that padding would blow up: the shares of the launch-per-step
+    form, and no more memory than it takes."""
+    say("matmul gate thin %dx%dx%d" % (M, K, N))
+    native.call("sufhip_init", 0)
+    rng = np.random.default_rng(M)
+    x, w = (rng.integers(-(1 << 14), 1 << 14, s) for s in (M * K, K * N))
+    x0, w0 = (rng.integers(0, 1 << 64, s, dtype=np.uint64) for s in (M * K, K * N))
+    X = (dev(x0), dev(x.view(np.uint64) - x0))
+    W = (dev(w0), dev(w.view(np.uint64) - w0))
+    held, outs = [], []
+    for use_mfma in (True, False):
+        before = torch.cuda.memory_allocated()
+        gate = matmul_gate.BeaverMatmulTrunc(M, K, N, STATE, 12, seed=7, use_mfma=use_mfma)
+        held.append(torch.cuda.memory_allocated() - before)
+        out = [torch.empty(M * N, dtype=torch.int64, device="cuda") for _ in range(2)]
+        gate.eval2(X, W, out)
+        outs.append([u64(o) for o in out])
+        del gate
+    assert held[0] <= held[1]
+    for p in (0, 1):
+        assert np.array_equal(outs[0][p], outs[1][p])
+    z = x.reshape(M, K) @ w.reshape(K, N)
+    assert np.array_equal((outs[0][0] + outs[0][1]).view(np.int64), z.ravel() >> 12)

@@ -156,7 +156,7 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
                     void* stream);
 
 /* One party's comparison bits of several broadcast keys (1-byte payload) at
- * the same N points, in one launch per 64 keys: what sufhip_dcf_eval gives in
+ * the same N points, in launches of up to 64 keys: what sufhip_dcf_eval gives in
  * mode SUFHIP_DCF_OUT_BIT for each key (composite_eval_batch_backend's
  * predicate and cut queries, composite_fss.hpp:2132-2250).  jobs is a host
  * array; job j writes d_out [N] bytes. */

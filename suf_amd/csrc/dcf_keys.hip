@@ -102,24 +102,39 @@ int sufhip_dcf_eval_keys(const uint8_t* prg_state, const sufhip_dcf_key_job* job
   fill_key_sel(prg, &a.key_sel);
   a.xs = d_xs;
   a.n = n;
-  for (int base = 0; base < count; base += kKeysPerLaunch) {
-    const int m = count - base < kKeysPerLaunch ? count - base : kKeysPerLaunch;
-    // As many tiles per key as give every CU a workgroup, of at least 8
-    // points (one wave of quad walks).
-    size_t tiles = size_t(cus / m > 0 ? cus / m : 1);
-    a.tile = (n + tiles - 1) / tiles;
-    if (a.tile < 8) a.tile = 8;
-    tiles = (n + a.tile - 1) / a.tile;
-    a.quad = a.tile <= 256;
-    a.depth = forest_depth(a.tile, 1);
-    for (int j = 0; j < m; ++j) {
-      a.key[j] = jobs[base + j].d_key;
-      a.out[j] = jobs[base + j].d_out;
-      a.bits[j] = uint8_t(jobs[base + j].in_bits);
+  // A launch gives every key the same number of equal tiles, as many as the
+  // CUs hold.  From kForestBlock points per CU on, where a key alone fills the
+  // chip, a launch's keys have one width and such a number that at most 1/16
+  // of the CUs stay without a tile: points with no common prefix walk 56 levels
+  // of a 64-bit key and 4 of a 12-bit one.  20 + 2 such keys at 2^18 points, us
+  // in one launch / by width: no common prefix 6290 / 5115 (5940 as a launch
+  // per key), points of 15 bits 1053 / 853.
+  const bool whole = n >= size_t(kForestBlock) * size_t(cus);
+  for (int bits = whole ? 64 : 1; bits >= 1; --bits) {
+    const auto taken = [&](int j) { return !whole || jobs[j].in_bits == bits; };
+    int left = 0;
+    for (int j = 0; j < count; ++j) left += taken(j) ? 1 : 0;
+    for (int j = 0, m = 0; left > 0; left -= m) {
+      m = left < kKeysPerLaunch ? left : kKeysPerLaunch;
+      if (whole)
+        while (m <= cus && 16 * (cus / m * m) < 15 * cus) --m;
+      // At least 8 points to a tile (one wave of quad walks).
+      size_t tiles = size_t(cus / m > 0 ? cus / m : 1);
+      a.tile = (n + tiles - 1) / tiles;
+      if (a.tile < 8) a.tile = 8;
+      tiles = (n + a.tile - 1) / a.tile;
+      a.quad = a.tile <= 256;
+      a.depth = forest_depth(a.tile, 1);
+      for (int q = 0; q < m; ++j) {
+        if (!taken(j)) continue;
+        a.key[q] = jobs[j].d_key;
+        a.out[q] = jobs[j].d_out;
+        a.bits[q++] = uint8_t(jobs[j].in_bits);
+      }
+      hipLaunchKernelGGL(dcf_eval_keys_kernel, dim3(unsigned(tiles), unsigned(m)),
+                         dim3(kForestBlock), 0, as_stream(stream), a);
+      if (int rc = check_launch("dcf_eval_keys_kernel")) return rc;
     }
-    hipLaunchKernelGGL(dcf_eval_keys_kernel, dim3(unsigned(tiles), unsigned(m)),
-                       dim3(kForestBlock), 0, as_stream(stream), a);
-    if (int rc = check_launch("dcf_eval_keys_kernel")) return rc;
   }
   return SUFHIP_OK;
 }

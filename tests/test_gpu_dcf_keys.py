@@ -30,7 +30,8 @@ def _points(shape, n, centre, rng):
 @pytest.mark.parametrize("shape", ["equal", "near", "wrap", "random"])
 @pytest.mark.parametrize("n,bits", [
     (1, [64]), (9, [1, 64, 12]), (300, [64] * 3 + [5]), (8 * 256 + 1, [64, 64]),
-    (257 * 256 + 3, [64, 9]), (4096, [64] * 20 + [12] * 2), (70000, [64] * 21), (65, [17] * 65)])
+    (257 * 256 + 3, [64, 9]), (4096, [64] * 20 + [12] * 2), (70000, [64] * 21), (65, [17] * 65),
+    (1024 * 256 - 1, [12, 64, 5]), (1024 * 256 + 77, [12, 64, 64, 9, 64, 12] + [64] * 4 + [3] * 45)])
 def test_bits_match_single_key_evaluation(n, bits, shape):
     say("dcf_eval_keys n=%d keys=%d shape=%s" % (n, len(bits), shape))
     native.call("sufhip_init", 0)

@@ -149,9 +149,11 @@ __device__ __forceinline__ uint32_t eval_program(const sufhip_composite_bool_arg
 // (a segment needs only the cut bits on its two sides and its own triples),
 // and the segments' terms are added through LDS.  One lane over all the
 // segments is a chain of a memory round trip per product: 27 us for 4096
-// elements, five segments and two outputs, 9 us this way.
-template <int kEll>
-__global__ void __launch_bounds__(512) composite_bool2_kernel(BoolArgs A) {
+// elements, five segments and two outputs, 9 us this way.  kOne is that form,
+// 256 elements to a workgroup, where each cut bit's triple is read once (the
+// launch's rule).
+template <int kEll, bool kOne>
+__global__ void __launch_bounds__(kOne ? 256 : 512) composite_bool2_kernel(BoolArgs A) {
   extern __shared__ uint64_t part[];  // [blockDim.y - 1][kEll][2][64]
   const sufhip_composite_bool_args& g = A.g;
   const Tri2 tri{{g.tri[0], g.tri[1]}, g.n};
@@ -159,17 +161,20 @@ __global__ void __launch_bounds__(512) composite_bool2_kernel(BoolArgs A) {
   const size_t t_bits = size_t(C > 0 ? 2 * C - 1 : 0);  // first triple of the bits' b2a
   const size_t t_sel = t_bits + size_t(S) * size_t(ell);  // first selector product
   const int lane = int(threadIdx.x);
-  const int wy = __builtin_amdgcn_readfirstlane(int(threadIdx.y)), ny = int(blockDim.y);
-  for (size_t base = size_t(blockIdx.x) * 64; base < g.n; base += size_t(gridDim.x) * 64) {
+  const int wy = kOne ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+  const int ny = kOne ? 1 : int(blockDim.y);
+  constexpr size_t kWide = kOne ? 256 : 64;
+  for (size_t base = size_t(blockIdx.x) * kWide; base < g.n; base += size_t(gridDim.x) * kWide) {
     const size_t i = base + size_t(lane);
     uint64_t acc[kEll][2];
 #pragma unroll
     for (int j = 0; j < kEll; ++j) acc[j][0] = acc[j][1] = 0;
     if (i < g.n) {
+      uint64_t prev[2] = {0, 0};  // additive cut_{s-1}
       for (int s = wy; s < S; s += ny) {
         // sel = (1 - cut_{s-1}) cut_s, without the missing one at the ends.
-        uint64_t prev[2] = {0, 0}, cur[2] = {0, 0}, sel[2];
-        if (s > 0)
+        uint64_t cur[2] = {0, 0}, sel[2];
+        if (!kOne && s > 0)
           tri.b2a(size_t(s - 1), i, g.cut[0][size_t(s - 1) * g.n + i] & 1u,
                   g.cut[1][size_t(s - 1) * g.n + i] & 1u, prev);
         if (s < C)
@@ -188,6 +193,8 @@ __global__ void __launch_bounds__(512) composite_bool2_kernel(BoolArgs A) {
           const uint64_t np[2] = {1 - prev[0], uint64_t(0) - prev[1]};
           tri.mul(size_t(C) + size_t(s - 1), i, np, cur, sel);
         }
+        prev[0] = cur[0];
+        prev[1] = cur[1];
         size_t and_idx = size_t(A.ands[s]);
 #pragma unroll
         for (int j = 0; j < kEll; ++j) {
@@ -207,7 +214,7 @@ __global__ void __launch_bounds__(512) composite_bool2_kernel(BoolArgs A) {
 #pragma unroll
         for (int p = 0; p < 2; ++p) part[(((wy - 1) * kEll + j) * 2 + p) * 64 + lane] = acc[j][p];
     }
-    __syncthreads();
+    if constexpr (!kOne) __syncthreads();
     if (wy == 0 && i < g.n) {
       for (int y = 1; y < ny; ++y)
 #pragma unroll
@@ -220,7 +227,7 @@ __global__ void __launch_bounds__(512) composite_bool2_kernel(BoolArgs A) {
         g.out[1][i * size_t(ell) + j] = acc[j][1];
       }
     }
-    __syncthreads();
+    if constexpr (!kOne) __syncthreads();
   }
 }
 
@@ -338,18 +345,33 @@ int sufhip_composite_bool2(const sufhip_composite_bool_args* args, void* stream)
   SUFHIP_REQUIRE(ands == 0 || (g.bit_tri[0] && g.bit_tri[1]),
                  "sufhip_composite_bool2: null bit triples");
   // Waves per 64 elements: one per segment, up to 8 (512 lanes leave the
-  // unrolled outputs their registers) and 30 KB of partial sums in LDS.
+  // unrolled outputs their registers) and 30 KB of partial sums in LDS.  The
+  // more waves, the more streams of triples at once (and neighbouring
+  // segments read a cut's triple twice), so two where the triples exceed half
+  // of the 256 MB last-level cache, and one past it, where memory bounds the
+  // launch.  Us for five segments and two outputs with a wave per segment /
+  // two waves / one: 65536 elements (85 MB) 24 / 29 / 37, 131072 (170 MB) 45 /
+  // 41 / 48, 170000 (220 MB) 55 / 48 / 53, 262144 (340 MB) 97 / 85 / 80,
+  // 524288 191 / 151 / 135.
   int waves = g.cuts + 1 < 8 ? g.cuts + 1 : 8;
+  const size_t triples = size_t(g.cuts > 0 ? 2 * g.cuts - 1 : 0) + 2 * size_t(progs);
+  const size_t bytes = g.n * triples * 2 * 3 * sizeof(uint64_t);
+  if (bytes > size_t(128) << 20 && waves > 2) waves = 2;
+  if (bytes > size_t(256) << 20) waves = 1;
   if ((waves - 1) * g.ell > 30) waves = 30 / g.ell + 1;
   const size_t lds = size_t(waves - 1) * size_t(g.ell) * 2 * 64 * sizeof(uint64_t);
-  const dim3 block(64, unsigned(waves));
-  size_t blocks = (g.n + 63) / 64;
+  const dim3 block(waves > 1 ? 64 : 256, unsigned(waves));
+  size_t blocks = (g.n + block.x - 1) / block.x;
   if (blocks > 32768) blocks = 32768;
+  const dim3 grid{unsigned(blocks)};
   const hipStream_t st = as_stream(stream);
   switch (g.ell) {
 #define SUFHIP_ELL_CASE(E)                                                                  \
   case E:                                                                                   \
-    hipLaunchKernelGGL(composite_bool2_kernel<E>, dim3(unsigned(blocks)), block, lds, st, a);   \
+    if (waves == 1)                                                                         \
+      hipLaunchKernelGGL((composite_bool2_kernel<E, true>), grid, block, lds, st, a);       \
+    else                                                                                    \
+      hipLaunchKernelGGL((composite_bool2_kernel<E, false>), grid, block, lds, st, a);      \
     break;
     SUFHIP_ELL_CASE(1)
     SUFHIP_ELL_CASE(2)

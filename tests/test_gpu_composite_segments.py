@@ -1,12 +1,15 @@
 """The boolean network's split over a gate's segments (one wave per segment of
-64 elements, up to 8 waves): both parties' shares equal the oracle's two-party
-composition for one segment, more segments than waves and up to 8 outputs, at
-whole and partial groups of 64 elements."""
+64 elements, up to 8 waves; two and one where the triples exceed 128 and 256
+MB): both parties' shares equal the oracle's two-party composition for one
+segment, more segments than waves and up to 8 outputs, at whole and partial
+groups of 64 elements, and the large batches' equal those of their own parts."""
 import numpy as np
 import pytest
+import torch
 
 import test_gpu_composite as base
-from suf_amd import native
+from gpu_util import say
+from suf_amd import composite, native
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +34,34 @@ def _spec(pieces, ell):
 def test_segments(pieces, ell, n):
     native.call("sufhip_init", 0)
     base._run(_spec(pieces, ell), n, 11 + n, share_check=True)
+
+
+@pytest.mark.parametrize("n", [104000 + 37, 208000 + 5])
+def test_batches_past_the_cache_equal_their_parts(n):
+    """A batch on two waves and on one, against the same triples and bits cut
+    into parts that take a wave per segment."""
+    say("composite network n=%d" % n)
+    native.call("sufhip_init", 0)
+    gate = composite.CompositeGate(_spec(5, 2), n, base.STATE, seed=3)
+    assert 128 << 20 < n * gate.T * 48 and (n * gate.T * 48 > 256 << 20) == (n > 200000)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    for t in gate.pred + gate.cutb:
+        t.copy_(torch.randint(0, 2, t.shape, dtype=torch.uint8, device="cuda", generator=g))
+    call = lambda a: native.call("sufhip_composite_bool2", native.ctypes.byref(a), None)  # noqa: E731
+    whole = [torch.empty(n * 2, dtype=torch.int64, device="cuda") for _ in range(2)]
+    call(gate.args(whole))
+    step = 60000
+    for lo in range(0, n, step):
+        m = min(step, n - lo)
+        cut = lambda t: t.reshape(-1, n)[:, lo:lo + m].contiguous()  # noqa: E731
+        out = [torch.empty(m * 2, dtype=torch.int64, device="cuda") for _ in range(2)]
+        a = gate.args(out)
+        a.n = m
+        held = []
+        for p in (0, 1):
+            parts = [cut(t) for t in (gate.pred[p], gate.cutb[p], gate.bit_tri[p], gate.tri[p])]
+            held.append(parts)
+            a.pred[p], a.cut[p], a.bit_tri[p], a.tri[p] = (t.data_ptr() for t in parts)
+        call(a)
+        for p in (0, 1):
+            assert torch.equal(out[p], whole[p][2 * lo:2 * (lo + m)]), (lo, p)

@@ -22,15 +22,13 @@ constexpr int kTruncHdrBytes = 64;
 // read per element at evaluation).
 constexpr int kTruncTableBits = 14;
 
-// The prepared carry share at point v.  Tables of up to kTruncTableBits bits
-// are 8-byte entries (32 KB at 12 bits, an L1's worth, where whole frontier
+// Entry v of a table of up to kTruncTableBits bits: the prepared carry share at
+// point v.  8 bytes each (32 KB at 12 bits, an L1's worth, where whole frontier
 // nodes take four times that: a gather's 64 lanes share fewer lines; spline
-// gate at 2^20 98.9 -> 96.9 us, the secure layer 289 -> 282); deeper full
-// domains keep the nodes of the frontier they are expanded from.
-__device__ __forceinline__ uint64_t trunc_table_at(const uint4* table, int f, uint64_t v) {
-  if (f <= kTruncTableBits) return reinterpret_cast<const uint64_t*>(table)[v];
-  const uint4 q = table[2 * v + 1];
-  return uint64_t(q.x) | uint64_t(q.y) << 32;
+// gate at 2^20 98.9 -> 96.9 us, the secure layer 289 -> 282).  Every launch
+// that folds a truncation in takes such tables only (make_epi).
+__device__ __forceinline__ uint64_t trunc_table_at(const uint4* table, uint64_t v) {
+  return reinterpret_cast<const uint64_t*>(table)[v];
 }
 
 struct TruncHdr {
@@ -101,15 +99,15 @@ __device__ __forceinline__ uint64_t trunc_carry_from(const TruncHdr& h, uint64_t
 }
 
 // One party's GapARS output at the public xhat from the key's header and its
-// prepared full-domain table (node v's value word holds the carry DCF's
-// share at v).  A key that is not a GapARS key for f bits yields 0; the table
-// read stays inside its 2^f nodes either way.
+// prepared full-domain table (f <= kTruncTableBits).  A key that is not a
+// GapARS key for f bits yields 0; the table read stays inside its 2^f entries
+// either way.
 __device__ __forceinline__ uint64_t trunc_table_eval_h(const TruncHdr& h, const uint4* table,
                                                        int f, uint64_t xhat) {
   if (h.tag != kTruncTag || h.kind != SUFHIP_TRUNC_GAPARS || int(h.f) != f) return 0;
   uint64_t carry = 0;
   if (h.flags & 1)
-    carry = trunc_carry_from(h, trunc_table_at(table, f, xhat & ((uint64_t(1) << f) - 1)));
+    carry = trunc_carry_from(h, trunc_table_at(table, xhat & ((uint64_t(1) << f) - 1)));
   return trunc_postproc<SUFHIP_TRUNC_GAPARS>(h, f, xhat, carry, 0, 0);
 }
 
@@ -137,7 +135,7 @@ __device__ __forceinline__ bool trunc_table_key_ok(const TruncHdr& h, int f) {
 __device__ __forceinline__ uint64_t trunc_table_word(const TruncHdr& h, const uint4* table, int f,
                                                      uint64_t xhat) {
   if (!trunc_table_key_ok(h, f) || !(h.flags & 1)) return 0;
-  return trunc_table_at(table, f, xhat & ((uint64_t(1) << f) - 1));
+  return trunc_table_at(table, xhat & ((uint64_t(1) << f) - 1));
 }
 __device__ __forceinline__ uint64_t trunc_table_out(const TruncHdr& h, int f, uint64_t xhat,
                                                     uint64_t word) {

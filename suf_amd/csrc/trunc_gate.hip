@@ -115,9 +115,9 @@ __global__ void __launch_bounds__(kDcfBlock) trunc_gen_kernel(TruncGenArgs a) {
                                 a.key0 + a.off[j], a.key1 + a.off[j]);
 }
 
-// Frontier node v: {s0, s1, s2, s3} and {v_lo, v_hi, t, 0}.  With d == f the
-// node's value word holds the final share at point v.
 // One launch evaluates one or both parties: grid.y selects the party slot.
+// tables: frontier nodes {s0, s1, s2, s3}, {v_lo, v_hi, t, 0}, or with d == f
+// the carry shares of the whole domain (full_domain_at).
 struct TruncEvalArgs {
   const uint8_t* keys[2];
   const uint64_t* xhat;
@@ -146,6 +146,14 @@ __device__ __forceinline__ uint64_t postproc(const Hdr& h, int f, uint64_t x, ui
 
 __device__ __forceinline__ uint64_t carry_from(const Hdr& h, uint64_t a) {
   return trunc_carry_from(h, a);
+}
+
+// The carry share at point v of a frontier of depth f: a table's entry, or past
+// kTruncTableBits the value word of the node that was expanded last.
+__device__ __forceinline__ uint64_t full_domain_at(const uint4* nodes, int f, uint64_t v) {
+  if (f <= kTruncTableBits) return trunc_table_at(nodes, v);
+  const uint4 q = nodes[2 * v + 1];
+  return uint64_t(q.x) | uint64_t(q.y) << 32;
 }
 
 // Gates with DCF walks per element: the 64-bit wrap key (TR, ARS) and sign
@@ -264,7 +272,7 @@ __global__ void __launch_bounds__(kForestBlock) trunc_eval_aes_kernel(TruncEvalA
         if (carry_walk) {
           c = share[kDcf * span + i];
         } else {
-          c = trunc_table_at(nodes, a.f, x & low);
+          c = full_domain_at(nodes, a.f, x & low);
         }
         carry = carry_from(h, c);
       }
@@ -288,7 +296,7 @@ __global__ void __launch_bounds__(256) trunc_eval_table_kernel(TruncEvalArgs a) 
   for (size_t e = size_t(blockIdx.x) * 256 + threadIdx.x; e < a.n; e += stride) {
     const uint64_t x = a.xhat[e];
     uint64_t carry = 0;
-    if (h.flags & 1) carry = carry_from(h, trunc_table_at(nodes, a.f, x & low));
+    if (h.flags & 1) carry = carry_from(h, full_domain_at(nodes, a.f, x & low));
     y[e] = postproc<SUFHIP_TRUNC_GAPARS>(h, a.f, x, carry, 0, 0);
   }
 }

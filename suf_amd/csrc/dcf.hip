@@ -34,7 +34,6 @@ namespace sufhip {
 namespace {
 
 struct DcfEvalArgs {
-  Prg4 prg;
   const uint8_t* keys;
   const uint64_t* xs;
   void* out;
@@ -44,7 +43,7 @@ struct DcfEvalArgs {
   int in_bits;
   int chunks;     // chunks to evaluate (1 for the bit modes)
   int out_bytes;  // bytes per element (OUT_BYTES)
-  DcfKeySel key_sel;  // the bit modes' round keys (scalar loads)
+  DcfKeySel key_sel;  // the round keys (scalar loads)
 };
 
 constexpr int kDcfBitBlock = 1024;
@@ -335,7 +334,9 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
   SUFHIP_REQUIRE(n < kMaxElems, "sufhip_dcf_eval: n too large");
   SUFHIP_REQUIRE(prg_state && d_keys && d_xs && d_out, "sufhip_dcf_eval: null pointer");
   DcfEvalArgs a{};
-  fill_prg4(prg_state, &a.prg);
+  Prg4 prg;
+  fill_prg4(prg_state, &prg);
+  fill_key_sel(prg, &a.key_sel);
   a.keys = d_keys;
   a.xs = d_xs;
   a.out = d_out;
@@ -346,7 +347,6 @@ int sufhip_dcf_eval(int group, int in_bits, int payload_len, const uint8_t* prg_
   a.chunks = 1;
   a.out_bytes = out_mode == SUFHIP_DCF_OUT_BYTES ? out_bytes : 1;
   hipStream_t s = as_stream(stream);
-  fill_key_sel(a.prg, &a.key_sel);
   if (out_mode == SUFHIP_DCF_OUT_BYTES) a.chunks = (out_bytes + 15) / 16;
   const size_t walks = n * size_t(a.chunks);
   int cus = 0;

@@ -5,6 +5,12 @@ import numpy as np
 import torch
 
 
+# Compute units of the GPU (256 where there is none: the tests that use it are
+# collected on the CPU too).
+CUS = (torch.cuda.get_device_properties(0).multi_processor_count if torch.cuda.is_available()
+       else 256)
+
+
 def dev(a):
     a = np.ascontiguousarray(a)
     if a.dtype == np.uint64:

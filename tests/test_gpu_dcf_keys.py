@@ -2,14 +2,14 @@
 points equal the one-key evaluation's and the oracle's, whatever the points
 share: all equal, a short interval (a long common prefix), an interval across
 0 (no common prefix), anything; for tiles of 8-lane walks and of one-lane
-walks with an expanded subtree, few-bit keys and more keys than one launch
-takes."""
+walks with an expanded subtree, few-bit keys, more keys than one launch takes
+and, from 1024 points per CU on, launches of one key width."""
 import numpy as np
 import pytest
 import torch
 
 import oracle_lib as ol
-from gpu_util import dev, host, say
+from gpu_util import CUS, dev, host, say
 from suf_amd import native, pfss
 
 pytestmark = pytest.mark.gpu
@@ -29,9 +29,9 @@ def _points(shape, n, centre, rng):
 
 @pytest.mark.parametrize("shape", ["equal", "near", "wrap", "random"])
 @pytest.mark.parametrize("n,bits", [
-    (1, [64]), (9, [1, 64, 12]), (300, [64] * 3 + [5]), (8 * 256 + 1, [64, 64]),
-    (257 * 256 + 3, [64, 9]), (4096, [64] * 20 + [12] * 2), (70000, [64] * 21), (65, [17] * 65),
-    (1024 * 256 - 1, [12, 64, 5]), (1024 * 256 + 77, [12, 64, 64, 9, 64, 12] + [64] * 4 + [3] * 45)])
+    (1, [64]), (9, [1, 64, 12]), (300, [64] * 3 + [5]), (8 * CUS + 1, [64, 64]),
+    (257 * CUS + 3, [64, 9]), (4096, [64] * 20 + [12] * 2), (70000, [64] * 21), (65, [17] * 65),
+    (1024 * CUS - 1, [12, 64, 5]), (1024 * CUS + 77, [12, 64, 64, 9, 64, 12] + [64] * 4 + [3] * 45)])
 def test_bits_match_single_key_evaluation(n, bits, shape):
     say("dcf_eval_keys n=%d keys=%d shape=%s" % (n, len(bits), shape))
     native.call("sufhip_init", 0)

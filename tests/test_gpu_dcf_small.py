@@ -7,13 +7,11 @@ import pytest
 import torch
 
 import oracle_lib as ol
-from gpu_util import best_us, dev, host, say, u64
+from gpu_util import CUS, best_us, dev, host, say, u64
 from suf_amd import native, pfss
 
 pytestmark = pytest.mark.gpu
 
-CUS = (torch.cuda.get_device_properties(0).multi_processor_count if torch.cuda.is_available()
-       else 256)
 # The largest batches of 8-lane walks, of 8-lane walks of bits past a full
 # pass of 2-lane ones, and of 2-lane walks.
 QUAD, AGAIN, PAIR = 160 * CUS, 320 * CUS, 384 * CUS

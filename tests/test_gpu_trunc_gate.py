@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle_lib as ol
-from gpu_util import best_us, dev, host, say, u64
+from gpu_util import CUS, best_us, dev, host, say, u64
 from suf_amd import native, pfss
 
 pytestmark = pytest.mark.gpu
@@ -132,8 +132,9 @@ def test_errors():
 
 def test_batched_prepare_matches_single_gate_path():
     # sufhip_trunc_prepare_batch (8 lanes per walk, local expansion of the
-    # table gates' last levels, up to 96 jobs per walk launch) against the
-    # one-gate prepare of sufhip_trunc_eval: equal shares for every gate.
+    # table gates' last levels, up to 96 jobs per walk launch) against
+    # sufhip_trunc_eval's prepare (the same walk, a launch per gate and party;
+    # that one is held against the oracle above): equal shares for every gate.
     # 52 gates = 104 jobs, so the batch takes two walk launches; the shapes
     # cover tables (f <= 14, including f below the local expansion depth),
     # walked prefixes with expansion launches (f = 24, n = 2^16) and
@@ -213,10 +214,10 @@ def test_batched_prepare_wide_launches(gates, f):
 
 def test_batched_prepare_past_one_round_of_768_lanes():
     """A batch of 960 lanes per CU (15 gates of 14 bits: 30 tables of 2^10
-    walks) costs about what one of 768 (12 gates) does, not two rounds of it
-    (1.75 times)."""
+    walks) costs about what one of 704 (11 gates) does (1.25 times), not two
+    rounds of 768 (1.8 times)."""
     from suf_amd import tasks
-    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+    if CUS != 256:
         pytest.skip("the gate counts are those of 256 CUs")
     dealer = tasks.Dealer(5)
     gs = [tasks.Trunc(dealer, 14, 64, STATE) for _ in range(15)]

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle_lib as ol
-from gpu_util import dev, say, u64
+from gpu_util import CUS, dev, say, u64
 from suf_amd import native, pfss
 
 pytestmark = pytest.mark.gpu
@@ -26,9 +26,9 @@ def _signed(v):
 @pytest.mark.parametrize("shape", ["equal", "near", "wrap", "random"])
 @pytest.mark.parametrize("kind,f,n", [
     (ol.TRUNC_TR, 12, 1), (ol.TRUNC_ARS, 12, 9), (ol.TRUNC_ARS, 24, 300),
-    (ol.TRUNC_TR, 16, 256 * 128 + 1), (ol.TRUNC_ARS, 12, 256 * 64 + 3),
-    (ol.TRUNC_ARS, 12, 256 * 128 + 129), (ol.TRUNC_ARS, 24, 98304 + 5),
-    (ol.TRUNC_GAPARS, 20, 256 * 256 + 7), (ol.TRUNC_GAPARS, 31, 50)])
+    (ol.TRUNC_TR, 16, CUS * 128 + 1), (ol.TRUNC_ARS, 12, CUS * 64 + 3),
+    (ol.TRUNC_ARS, 12, CUS * 128 + 129), (ol.TRUNC_ARS, 24, 98304 + 5),
+    (ol.TRUNC_GAPARS, 20, CUS * 256 + 7), (ol.TRUNC_GAPARS, 31, 50)])
 def test_tiles(kind, f, n, shape):
     say("trunc tiles kind=%d f=%d n=%d shape=%s" % (kind, f, n, shape))
     native.call("sufhip_init", 0)

@@ -214,17 +214,16 @@ def _timed(fn, threads):
 
 # Algorithmic HBM bytes of the two-party task kernels: the streams each
 # element (or row) brings in or sends out, both parties.  The truncation
-# gates' full-domain tables (2^f entries of which an evaluation reads the
-# 16-byte value half) and the LUT blobs are read by every workgroup but
-# stay in L2, so they count once per launch, at most 2^f x 16 bytes per gate
+# gates' full-domain tables (2^f entries of 8 bytes, f <= 14) and the LUT
+# blobs are read by every workgroup but stay in L2, so they count once per launch, at most 2^f x 8 bytes per gate
 # and party.  A CUBIC chain (spline gate, GeLU, nExp) streams x (16), three
 # products' triples (3 x 2 parties x 3 words x 8 = 144) and the output (16).
 CHAIN_CUBIC_BYTES = 16 + 144 + 16
 
 
 def trunc_table_bytes(gates, f=12):
-    """Bytes of the value halves of `gates` truncation tables, both parties."""
-    return gates * 2 * (1 << f) * 16
+    """Bytes of `gates` truncation tables, both parties."""
+    return gates * 2 * (1 << f) * 8
 
 
 def softmax_bytes(n_packed, rows, pre=0, indexed_input=False, out_written=True, n_dense=0,
@@ -306,7 +305,7 @@ def bench_spline(steps, warmup, n=1 << 20, frac_bits=12, cpu_seconds=0.0, shared
            "steps": steps,
            "roofline": roofline_hbm("gate_chain_kernel (CUBIC)", chain_ms, nbytes,
                                     "%d B per element (x 16, triples 144, out 16) x N + 3 "
-                                    "truncation tables once (2 x 2^%d x 16 B each)"
+                                    "truncation tables once (2 x 2^%d x 8 B each)"
                                     % (CHAIN_CUBIC_BYTES, frac_bits),
                                     note="per-party keystreams; the chain's AES-CTR keystream "
                                          "and dependent steps bind it, not HBM",
@@ -545,7 +544,7 @@ def bench_softmax_ln(steps, warmup, frac_bits=12, cpu=True, shared=True):
            "roofline": roofline_hbm(
                "softmax2_team_kernel", sm_ms, softmax_bytes(n_sm, len(offs) - 1),
                "per score 16 in + nExp triples 144 + normalisation shares 32 + 16 out; per row "
-               "164; 7 truncation tables once (2 x 2^12 x 16 B each)",
+               "164; 7 truncation tables once (2 x 2^12 x 8 B each)",
                note="per-party keystreams; bound by each row's chain of dependent steps (max "
                     "tree rounds, keystream AES, table reads), not HBM",
                traffic=SOFTMAX_TRAFFIC),
@@ -697,7 +696,7 @@ def bench_layer(steps, warmup, frac_bits=12, cpu=True, shared=True):
                                     out_written=False, n_dense=heads * seq * seq,
                                     dense_planes=True),
                "per packed score 20 in + nExp triples 144 + normalisation shares 32; per row "
-               "164; per dense entry 32; 9 truncation tables once (2 x 2^12 x 16 B each)",
+               "164; per dense entry 32; 9 truncation tables once (2 x 2^12 x 8 B each)",
                note="per-party keystreams; the layer's largest kernel, bound by each row's "
                     "dependent chain",
                traffic=LAYER_SOFTMAX_TRAFFIC),

@@ -867,8 +867,8 @@ int sufhip_layernorm2(const sufhip_layernorm2_args* args, void* stream) {
   const int grid = g.rows < cus * 8 ? g.rows : cus * 8;
   const int per = (g.cols + kLnBlock - 1) / kLnBlock;
   // More rows than CUs: 256 lanes per row leave the registers for two rows on
-  // a CU, where 512 hold one (300 x 1001: 38 -> 25 us, 256 rows then 44 before;
-  // a row alone takes about 1 us longer).
+  // a CU, where 512 hold one (300 x 1001: 38 -> 25 us).  A row alone takes
+  // about 1 us longer, so up to one row per CU keeps 512.
   const bool pair = g.rows > cus && per <= kLnMaxPer && !A.in_slices;
   const int block = (per <= kLnMaxPer || A.in_slices) && !pair ? kLnBlock : kLnWideBlock;
   A.row_groups = grid;

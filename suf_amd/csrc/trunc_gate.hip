@@ -65,7 +65,8 @@ int frontier_bits(int f, size_t n) {
 
 // Nodes of the walked level (k0) and of the final level (d) in the workspace:
 // level d always lands in the first 2^d slots, the level before it in the
-// 2^(d-1) slots after them.
+// 2^(d-1) slots after them.  (A table of up to kTruncTableBits bits takes 8
+// bytes per entry from the start of the same room.)
 int walk_bits(int d) { return d < kWalkFrontierBits ? d : kWalkFrontierBits; }
 
 // The batched prepare walks a table gate's whole domain (d = f <= 14) in one
@@ -646,8 +647,9 @@ using namespace sufhip;
 // stand-in, not device memory: the array's device address on each GPU comes
 // from hipGetSymbolAddress (noalloc_scratch below) and only that address is
 // passed to kernels.  1 MiB holds the carry frontier of any batch for
-// frac_bits <= 14 (the full-domain table, 786,432 bytes at f = 14) and of
-// batches below 2^16 points for larger frac_bits.
+// frac_bits <= 14 (sufhip_trunc_work_bytes asks for 786,432 bytes at f = 14,
+// of which the full-domain table takes the first 131,072) and of batches
+// below 2^16 points for larger frac_bits.
 static constexpr size_t kNoAllocScratchBytes = size_t(1) << 20;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 

@@ -26,9 +26,10 @@ Dealer (compile_suf_to_pfss_two_programs, src/compiler/suf_to_pfss.cpp:
   * one broadcast myl7 DCF key pair (payload 1, XOR group) per query and per
     cut; bit triples for AND / OR; Beaver triples for the network.
 Online: the DCF bits of every query and cut, both parties, at the public x^
-(one launch, sufhip_dcf_eval_keys), the whole selector / boolean network for both parties in one
-launch (sufhip_composite_bool2), and the arithmetic words through the
-interval LUT of the rotated pieces (sufhip_interval_lut_eval2).
+(sufhip_dcf_eval_keys: one launch, or one per key width for large batches),
+the whole selector / boolean network for both parties in one launch
+(sufhip_composite_bool2), and the arithmetic words through the interval LUT of
+the rotated pieces (sufhip_interval_lut_eval2).
 
 Offline key material travels as one composite tape per party
 (gates::write_composite_tape, composite_fss.hpp:2458-2641; suf_amd/tape.py):

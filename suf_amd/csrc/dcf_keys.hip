@@ -1,5 +1,5 @@
 // Comparison bits of several broadcast DCF keys at the same public points, in
-// one launch (sufhip_dcf_eval_keys): the predicate and cut queries of a
+// launches of up to 64 keys (sufhip_dcf_eval_keys): the predicate and cut queries of a
 // composite gate, which composite_eval_batch_backend evaluates one by one
 // (include/gates/composite_fss.hpp:2132-2250).
 //
